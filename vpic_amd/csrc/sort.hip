@@ -7,10 +7,12 @@
 // partition[v] = index of the first particle of voxel v, 0 below the first
 // interior voxel and np above the last (:335-340, :354-360).
 //
-// Main path (every axis of the grid within RS_MAXB - 2 cells): three stable
-// counting passes over (key, index) pairs, x then y then z digit of the
-// voxel (least significant first; the voxel index is monotone in (z, y, x)):
-//   k_rs_hist    per block of RS_BLK elements, the count of each digit
+// Main path (every axis of the grid within RS_MAXB - 2 cells): one to three
+// stable counting passes over (key, index) pairs, least significant digit
+// first.  A digit is the coordinate along one axis, or of two or all three
+// axes together while they have at most RS_MAXB values (the voxel index is
+// monotone in (z, y, x)):
+//   k_rs_hist    per block of elements, the count of each digit
 //                (LDS counters, runs of equal digits over consecutive lanes
 //                add once); the first pass reads the keys from the particles
 //   scan         exclusive scan of the (digit, block) counts
@@ -27,6 +29,7 @@
 #include "common.h"
 
 #include <atomic>
+#include <utility>
 
 namespace {
 
@@ -81,66 +84,87 @@ __global__ __launch_bounds__(256) void k_scatter(const int *__restrict__ keys,
   if (key >= 0) perm[base + (lane - s0)] = k;
 }
 
-// Block-wise exclusive scan: 256 threads x 8 items.
+// Exclusive scan of one value per thread of a workgroup of BS threads, and
+// the workgroup's total: shuffles within the wavefronts, the wavefronts'
+// totals through sh (BS / 64 ints).  Ends with a barrier, so sh may be
+// reused.
+template <int BS>
+__device__ __forceinline__ int block_exclusive_scan(int v, int *sh,
+                                                    int &total) {
+  const int lane = lane_id(), w = threadIdx.x >> 6;
+  int incl = v;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int o = __shfl_up(incl, d);
+    if (lane >= d) incl += o;
+  }
+  if (lane == 63) sh[w] = incl;
+  __syncthreads();
+  int base = 0, sum = 0;
+#pragma unroll
+  for (int k = 0; k < BS / 64; k++) {
+    const int c = sh[k];
+    base += k < w ? c : 0;
+    sum += c;
+  }
+  total = sum;
+  __syncthreads();
+  return base + incl - v;
+}
+
+// Scan of up to SCAN_ONE values by one workgroup (16 per thread): one launch
+// where three of them cost more than the values.
+constexpr int SCAN_ONE = 16384;
+// Values per workgroup of the three-launch scan (256 threads x 8).
 constexpr int SCAN_ITEMS = 2048;
 
-__device__ int block_exclusive_scan(int v, int *sh) {
-  // inclusive scan of 256 values in shared memory, returns exclusive
-  const int t = threadIdx.x;
-  sh[t] = v;
-  __syncthreads();
-  for (int d = 1; d < 256; d <<= 1) {
-    int x = t >= d ? sh[t - d] : 0;
-    __syncthreads();
-    sh[t] += x;
-    __syncthreads();
+template <int BS, int N>
+__device__ __forceinline__ int scan_items(const int *in, int *out, int64_t n,
+                                          int64_t base, int *sh) {
+  int v[N], s = 0, total;
+#pragma unroll
+  for (int i = 0; i < N; i++) {
+    v[i] = (base + i < n) ? in[base + i] : 0;
+    s += v[i];
   }
-  int incl = sh[t];
-  __syncthreads();
-  return incl - v;
+  int off = block_exclusive_scan<BS>(s, sh, total);
+#pragma unroll
+  for (int i = 0; i < N; i++) {
+    if (base + i < n) out[base + i] = off;
+    off += v[i];
+  }
+  return total;
+}
+
+__global__ __launch_bounds__(1024) void k_scan_one(const int *in, int *out,
+                                                   int n) {
+  __shared__ int sh[16];
+  scan_items<1024, 16>(in, out, n, threadIdx.x * 16, sh);
 }
 
 __global__ __launch_bounds__(256) void k_scan_local(const int *__restrict__ in,
                                                     int *__restrict__ out,
                                                     int64_t n,
                                                     int *__restrict__ sums) {
-  __shared__ int sh[256];
+  __shared__ int sh[4];
   const int64_t base = (int64_t)blockIdx.x * SCAN_ITEMS + threadIdx.x * 8;
-  int v[8], s = 0;
-#pragma unroll
-  for (int i = 0; i < 8; i++) {
-    v[i] = (base + i < n) ? in[base + i] : 0;
-    s += v[i];
-  }
-  int off = block_exclusive_scan(s, sh);
-#pragma unroll
-  for (int i = 0; i < 8; i++) {
-    if (base + i < n) out[base + i] = off;
-    off += v[i];
-  }
-  if (threadIdx.x == 255) sums[blockIdx.x] = off;
+  const int total = scan_items<256, 8>(in, out, n, base, sh);
+  if (threadIdx.x == 0) sums[blockIdx.x] = total;
 }
 
-__global__ __launch_bounds__(256) void k_scan_sums(int *sums, int nb) {
-  __shared__ int sh[256];
+// The workgroups' totals, 1024 at a time (13 chunks of 256 whose totals one
+// lane summed took 130 us for the 3225 totals of 4.2e8 particles on
+// 256x128x128 cells).
+__global__ __launch_bounds__(1024) void k_scan_sums(int *sums, int nb) {
+  __shared__ int sh[16];
   int carry = 0;
-  for (int c = 0; c < nb; c += 256) {
+  for (int c = 0; c < nb; c += 1024) {
     const int i = c + threadIdx.x;
     const int v = i < nb ? sums[i] : 0;
-    const int ex = block_exclusive_scan(v, sh);
+    int total;
+    const int ex = block_exclusive_scan<1024>(v, sh, total);
     if (i < nb) sums[i] = ex + carry;
-    __syncthreads();
-    // total of this chunk
-    sh[threadIdx.x] = v;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      int t = 0;
-      for (int j = 0; j < 256; j++) t += sh[j];
-      sh[0] = t;
-    }
-    __syncthreads();
-    carry += sh[0];
-    __syncthreads();
+    carry += total;
   }
 }
 
@@ -250,28 +274,32 @@ __global__ __launch_bounds__(256) void k_gather(
 }
 
 // --------------------------------------------------------------------------
-// Axis passes: the stable sort by voxel v = x + sx(y + sy z) as three stable
-// counting sorts of (key, index) pairs, by x, then y, then z (least
-// significant first).  Particles sorted at the last sort_p and moved a few
+// Digit passes: the stable sort by voxel v = x + sx(y + sy z) as stable
+// counting sorts of (key, index) pairs by the coordinates, x first (least
+// significant), neighbouring axes in one digit while their values fit the
+// LDS counters.  Particles sorted at the last sort_p and moved a few
 // cells since are still nearly in voxel order, so each pass sees long runs
 // of equal digits: one single-wavefront block counts and places them with
 // LDS counters, no global atomics, and lanes of a run write consecutive
 // slots.
 // --------------------------------------------------------------------------
-constexpr int RS_BLK = 16384;  // elements per block (one wavefront)
 constexpr int RS_MAXB = 2048;  // digit values per pass (LDS counters)
+// Elements per block (one wavefront).  A block is a serial chain of 64
+// elements at a time (0.55 us each), so a sort of few particles takes blocks
+// short enough for 16 wavefronts on every CU; many particles keep long ones,
+// which write fewer (digit, block) counts.
+constexpr int RS_BLK_MIN = 512, RS_BLK_MAX = 16384, RS_WAVES = 4096;
 
+// digit = (voxel / div) % mod: the coordinates along one or more axes
 struct SortDig {
-  unsigned sx1, sy1;  // nx + 2, ny + 2
+  unsigned div, mod;
   int nv;
 };
 
-__device__ __forceinline__ int axis_digit(int v, int axis, const SortDig &D) {
-  const unsigned t = (unsigned)v / D.sx1;
-  if (axis == 0) return v - (int)(t * D.sx1);
-  const unsigned z = t / D.sy1;
-  if (axis == 1) return (int)(t - z * D.sy1);
-  return (int)z;
+__device__ __forceinline__ int digit_of(int v, const SortDig &D) {
+  unsigned t = (unsigned)v;
+  if (D.div > 1) t /= D.div;
+  return (int)(t - (t / D.mod) * D.mod);
 }
 
 // Per block, the count of each digit: hist[d * nblocks + block].  SRC 0:
@@ -281,14 +309,14 @@ __device__ __forceinline__ int axis_digit(int v, int axis, const SortDig &D) {
 template <int SRC>
 __global__ __launch_bounds__(64) void k_rs_hist(
     const vpic_particle_t *__restrict__ p, const int *__restrict__ keys_in,
-    int *__restrict__ keys_out, int np, SortDig D, int axis, int nbins,
+    int *__restrict__ keys_out, int np, SortDig D, int blk, int nbins,
     int *__restrict__ hist, int nblocks, int *__restrict__ nbad) {
   __shared__ int h[RS_MAXB];
   const int lane = threadIdx.x;
   const int b = blockIdx.x;
   for (int d = lane; d < nbins; d += 64) h[d] = 0;
   __syncthreads();
-  const int base = b * RS_BLK, end = min(base + RS_BLK, np);
+  const int base = b * blk, end = min(base + blk, np);
   int bad = 0;
   // U rounds of 64 keys per batch; the next batch is loaded while this one
   // is counted
@@ -319,7 +347,7 @@ __global__ __launch_bounds__(64) void k_rs_hist(
       }
       if (SRC == 0) keys_out[i] = key;
     }
-    const int d = valid ? axis_digit(key, axis, D) : -1;
+    const int d = valid ? digit_of(key, D) : -1;
     // runs of equal digits over consecutive lanes: the last lane of a run
     // adds its length
     const int dn = __shfl_down(d, 1);
@@ -344,7 +372,7 @@ __global__ __launch_bounds__(64) void k_rs_hist(
 template <bool FIRST>
 __global__ __launch_bounds__(64) void k_rs_scatter(
     const int *__restrict__ keys_in, const int *__restrict__ idx_in, int np,
-    SortDig D, int axis, int nbins, int nbits, const int *__restrict__ offs,
+    SortDig D, int blk, int nbins, int nbits, const int *__restrict__ offs,
     int nblocks, int *__restrict__ keys_out, int *__restrict__ idx_out) {
   __shared__ int pos[RS_MAXB];
   const int lane = threadIdx.x;
@@ -352,7 +380,7 @@ __global__ __launch_bounds__(64) void k_rs_scatter(
   for (int d = lane; d < nbins; d += 64) pos[d] = offs[(int64_t)d * nblocks + b];
   __syncthreads();
   const uint64_t lt = (1ull << lane) - 1ull;
-  const int base = b * RS_BLK, end = min(base + RS_BLK, np);
+  const int base = b * blk, end = min(base + blk, np);
   // U rounds of 64 elements per batch; the next batch is loaded while this
   // one is placed
   constexpr int U = 4;
@@ -380,7 +408,7 @@ __global__ __launch_bounds__(64) void k_rs_scatter(
     const int key =
         FIRST ? ((unsigned)kk[u] < (unsigned)D.nv ? kk[u] : 0) : kk[u];
     const int idx = ii[u];
-    const int d = valid ? axis_digit(key, axis, D) : 0;
+    const int d = valid ? digit_of(key, D) : 0;
     // lanes holding the same digit
     uint64_t m = __ballot(valid);
     for (int bit = 0; bit < nbits; bit++) {
@@ -477,11 +505,16 @@ inline int blocks_for(int64_t n, int bs) { return (int)((n + bs - 1) / bs); }
 // Exclusive scan of n ints (in may equal out).  sums: ceil(n/2048) ints.
 int device_exclusive_scan(const int *in, int *out, int64_t n, int *sums,
                           hipStream_t s) {
+  if (n <= SCAN_ONE) {
+    hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(1024), 0, s, in, out, (int)n);
+    VPIC_LAUNCHED("k_scan_one");
+    return VPIC_OK;
+  }
   const int nb = blocks_for(n, SCAN_ITEMS);
   hipLaunchKernelGGL(k_scan_local, dim3(nb), dim3(256), 0, s, in, out, n,
                      sums);
   VPIC_LAUNCHED("k_scan_local");
-  hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(256), 0, s, sums, nb);
+  hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(1024), 0, s, sums, nb);
   VPIC_LAUNCHED("k_scan_sums");
   hipLaunchKernelGGL(k_scan_add, dim3(nb), dim3(256), 0, s, out, n,
                      (const int *)sums);
@@ -504,7 +537,42 @@ constexpr int SORT_KEYS_STALE = 1;
 std::atomic<long long> g_sort_keys_stale{0};
 void note_sort_keys_stale() { g_sort_keys_stale.fetch_add(1); }
 
-// The axis-pass sort (grids up to RS_MAXB - 2 cells per axis).  With
+// One pass of the digit sort: its digit, its values and its block length.
+struct SortPass {
+  SortDig D;
+  int nbins, blk, nblocks;
+};
+
+// The passes of grid g for np particles, x first: an axis joins the digit of
+// the one before it while together they have at most RS_MAXB values (two
+// passes fewer on a 12x10x9 box, one on a 32^3 box and on 2D grids), and the
+// blocks halve from RS_BLK_MAX until there are RS_WAVES of them, but keep
+// twice the digit's values (a shorter block would write more counts than it
+// has elements).
+int sort_passes(const vpic_grid_t *g, int np, SortPass out[3]) {
+  const unsigned ax[3] = {(unsigned)(g->nx + 2), (unsigned)(g->ny + 2),
+                          (unsigned)(g->nz + 2)};
+  int n = 0;
+  unsigned div = 1;
+  for (int k = 0; k < 3;) {
+    unsigned mod = ax[k++];
+    while (k < 3 && (uint64_t)mod * ax[k] <= (uint64_t)RS_MAXB) mod *= ax[k++];
+    SortPass &P = out[n++];
+    P.D.div = div;
+    P.D.mod = mod;
+    P.D.nv = g->nv;
+    P.nbins = (int)mod;
+    P.blk = RS_BLK_MAX;
+    while (P.blk > RS_BLK_MIN && np / P.blk < RS_WAVES &&
+           P.blk / 2 >= 2 * P.nbins)
+      P.blk /= 2;
+    P.nblocks = blocks_for(np, P.blk);
+    div *= mod;
+  }
+  return n;
+}
+
+// The digit sort (grids up to RS_MAXB - 2 cells per axis).  With
 // `hint` (the caller's copy of p[k].i, k < np) the first pass reads the
 // keys from it instead of from the particles, and the gather checks every
 // particle's voxel index against the key it was sorted by; a difference,
@@ -514,11 +582,13 @@ int sort_p_axes(vpic_particle_t *p, vpic_particle_t *aux, int np,
                 const int *hint, hipStream_t s) {
   SortScratch &S = sort_scratch();
   const int nv = g->nv;
-  const int nblocks = blocks_for(np, RS_BLK);
-  const int bins[3] = {g->nx + 2, g->ny + 2, g->nz + 2};
-  const int maxb = bins[0] > bins[1] ? (bins[0] > bins[2] ? bins[0] : bins[2])
-                                     : (bins[1] > bins[2] ? bins[1] : bins[2]);
-  const int64_t nh = (int64_t)maxb * nblocks;
+  SortPass pass[3];
+  const int npass = sort_passes(g, np, pass);
+  int64_t nh = 0;
+  for (int k = 0; k < npass; k++) {
+    const int64_t n = (int64_t)pass[k].nbins * pass[k].nblocks;
+    nh = n > nh ? n : nh;
+  }
   int rc;
   if ((rc = scratch_reserve(S.keys, sizeof(int) * (size_t)np)) ||
       (rc = scratch_reserve(S.perm, sizeof(int) * (size_t)np)) ||
@@ -533,24 +603,21 @@ int sort_p_axes(vpic_particle_t *p, vpic_particle_t *aux, int np,
   int *kb = (int *)S.keys2.ptr, *ib = (int *)S.idx2.ptr;
   int *hist = (int *)S.hist.ptr, *sums = (int *)S.sums.ptr;
   int *nbad = (int *)S.nbig.ptr;
-  SortDig D;
-  D.sx1 = (unsigned)(g->nx + 2);
-  D.sy1 = (unsigned)(g->ny + 2);
-  D.nv = nv;
   // nbad[0]: keys outside [0, nv); nbad[1]: particles whose voxel index is
   // not the caller's key
   hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, s, nbad, (int64_t)2, 0);
   VPIC_LAUNCHED("k_fill_int");
-  // pass x: keys from the particles into kb (or the caller's keys), then
+  // first pass: keys from the particles into kb (or the caller's keys), then
   // (keys, index) -> (ka, ia)
   if (hint) {
-    hipLaunchKernelGGL(k_rs_hist<2>, dim3(nblocks), dim3(64), 0, s,
+    hipLaunchKernelGGL(k_rs_hist<2>, dim3(pass[0].nblocks), dim3(64), 0, s,
                        (const vpic_particle_t *)nullptr, hint, (int *)nullptr,
-                       np, D, 0, bins[0], hist, nblocks, nbad);
+                       np, pass[0].D, pass[0].blk, pass[0].nbins, hist,
+                       pass[0].nblocks, nbad);
   } else {
-    hipLaunchKernelGGL(k_rs_hist<0>, dim3(nblocks), dim3(64), 0, s, p,
-                       (const int *)nullptr, kb, np, D, 0, bins[0], hist,
-                       nblocks, nbad);
+    hipLaunchKernelGGL(k_rs_hist<0>, dim3(pass[0].nblocks), dim3(64), 0, s, p,
+                       (const int *)nullptr, kb, np, pass[0].D, pass[0].blk,
+                       pass[0].nbins, hist, pass[0].nblocks, nbad);
     VPIC_LAUNCHED("k_rs_hist");
     int h_nbad = 0;
     VPIC_HIP(hipMemcpyAsync(&h_nbad, nbad, sizeof(int), hipMemcpyDeviceToHost,
@@ -562,29 +629,35 @@ int sort_p_axes(vpic_particle_t *p, vpic_particle_t *aux, int np,
                             "[0,nv); particles left unsorted", h_nbad);
   }
   VPIC_LAUNCHED("k_rs_hist");
-  if ((rc = device_exclusive_scan(hist, hist, (int64_t)bins[0] * nblocks,
+  if ((rc = device_exclusive_scan(hist, hist,
+                                  (int64_t)pass[0].nbins * pass[0].nblocks,
                                   sums, s)))
     return rc;
-  hipLaunchKernelGGL(k_rs_scatter<true>, dim3(nblocks), dim3(64), 0, s,
+  hipLaunchKernelGGL(k_rs_scatter<true>, dim3(pass[0].nblocks), dim3(64), 0, s,
                      hint ? hint : (const int *)kb, (const int *)nullptr, np,
-                     D, 0, bins[0], nbits_for(bins[0]), (const int *)hist,
-                     nblocks, ka, ia);
+                     pass[0].D, pass[0].blk, pass[0].nbins,
+                     nbits_for(pass[0].nbins), (const int *)hist,
+                     pass[0].nblocks, ka, ia);
   VPIC_LAUNCHED("k_rs_scatter");
-  // passes y and z: (ka, ia) -> (kb, ib) -> (ka, ia)
-  for (int axis = 1; axis < 3; axis++) {
-    const int *kin = axis == 1 ? ka : kb, *iin = axis == 1 ? ia : ib;
-    int *kout = axis == 1 ? kb : ka, *iout = axis == 1 ? ib : ia;
-    hipLaunchKernelGGL(k_rs_hist<1>, dim3(nblocks), dim3(64), 0, s,
-                       (const vpic_particle_t *)nullptr, kin, (int *)nullptr,
-                       np, D, axis, bins[axis], hist, nblocks, nbad);
+  // the other passes: (ka, ia) -> (kb, ib) -> (ka, ia); the sorted pairs end
+  // in (ka, ia)
+  for (int k = 1; k < npass; k++) {
+    const SortPass &P = pass[k];
+    hipLaunchKernelGGL(k_rs_hist<1>, dim3(P.nblocks), dim3(64), 0, s,
+                       (const vpic_particle_t *)nullptr, (const int *)ka,
+                       (int *)nullptr, np, P.D, P.blk, P.nbins, hist,
+                       P.nblocks, nbad);
     VPIC_LAUNCHED("k_rs_hist");
-    if ((rc = device_exclusive_scan(hist, hist,
-                                    (int64_t)bins[axis] * nblocks, sums, s)))
+    if ((rc = device_exclusive_scan(hist, hist, (int64_t)P.nbins * P.nblocks,
+                                    sums, s)))
       return rc;
-    hipLaunchKernelGGL(k_rs_scatter<false>, dim3(nblocks), dim3(64), 0, s,
-                       kin, iin, np, D, axis, bins[axis], nbits_for(bins[axis]),
-                       (const int *)hist, nblocks, kout, iout);
+    hipLaunchKernelGGL(k_rs_scatter<false>, dim3(P.nblocks), dim3(64), 0, s,
+                       (const int *)ka, (const int *)ia, np, P.D, P.blk,
+                       P.nbins, nbits_for(P.nbins), (const int *)hist,
+                       P.nblocks, kb, ib);
     VPIC_LAUNCHED("k_rs_scatter");
+    std::swap(ka, kb);
+    std::swap(ia, ib);
   }
   hipLaunchKernelGGL(k_gather_part<GATHER_GU>,
                      dim3(blocks_for((int64_t)np + 1, 128 * GATHER_GU)),
@@ -820,7 +893,7 @@ int launch_ens_sort(vpic_particle_t *P, vpic_particle_t *aux,
   return VPIC_OK;
 }
 
-// sort_p: the axis passes when every axis fits their LDS counters, else the
+// sort_p: the digit passes when every axis fits their LDS counters, else the
 // counting sort.
 int launch_sort_p(vpic_particle_t *p, vpic_particle_t *aux, int np,
                   int *partition, const vpic_grid_t *g, int in_place,
