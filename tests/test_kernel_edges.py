@@ -67,3 +67,70 @@ def test_sort_digit_groups(dev, n, np_):
                       keys.ptr, ctypes.byref(g), 0, None)
         assert H.same_bits(aux.download(), want)
         assert np.array_equal(dpart.download(), part)
+
+
+def _adjoint_inputs(g, np_, seed, fp64):
+    """Particles in random cells (so that no tile has the average), fields
+    with ghosts, as tensors of the run's precision."""
+    import torch
+    from vpic_amd import adjoint as A
+    rng = np.random.default_rng(seed)
+    p = np.zeros(np_, dtype=T.PARTICLE)
+    x, y, z = (rng.integers(1, k + 1, np_) for k in (g.nx, g.ny, g.nz))
+    p["i"] = g.voxel(x, y, z)
+    for c in ("dx", "dy", "dz"):
+        p[c] = rng.uniform(-1, 1, np_).astype(np.float32)
+    for c in ("ux", "uy", "uz"):
+        p[c] = (0.6 * rng.standard_normal(np_)).astype(np.float32)
+    p["w"] = np.float32(g.dV / max(np_ / (g.nx * g.ny * g.nz), 1))
+    f = H.random_fields(g, seed + 1, 0.02, 0.02)
+    if fp64:
+        P, F = A.host_particles64(p), A.fields64(f)
+    else:
+        P, F = p.view(np.float32).reshape(-1, 8), \
+            f.view(np.float32).reshape(-1, 20)
+    return torch.from_numpy(P).cuda(), torch.from_numpy(F).cuda()
+
+
+# tiles of 8x4x4 cells: one tile with a window that wraps onto itself, two
+# tiles an axis, a last tile of one cell, axes of one cell, an axis too long
+# to sort (chunks of particles, no windows); particle counts around a
+# wavefront and a workgroup, none; steps past a sort, checkpoints that do and
+# do not fall on one
+@pytest.mark.parametrize("n,np_,steps,ckpt", [
+    ((3, 2, 4), 1, 3, 2), ((8, 4, 4), 65, 10, 4), ((9, 5, 5), 257, 17, 3),
+    ((17, 8, 9), 3000, 9, 20), ((16, 1, 13), 1500, 12, 5),
+    ((1, 9, 1), 300, 9, 8), ((2100, 1, 1), 9000, 10, 4), ((6, 6, 6), 0, 4, 2)],
+    ids=lambda v: str(v).replace(" ", ""))
+def test_adjoint_tiles(dev, n, np_, steps, ckpt):
+    """The gradients do not depend on how particles share tiles: the same
+    particles in another order, each with its own gradient.  In FP64 the two
+    runs differ by the rounding of sums of at most np terms in another order
+    over the steps: 1e-10 of the largest is 1e5 times the rounding of one
+    value, for growth of a factor below that over these steps."""
+    import torch
+    from vpic_amd import adjoint as A
+    g = _box(*n, cell=0.1)
+    P, F = _adjoint_inputs(g, np_, 5, True)
+    order = torch.randperm(np_, generator=torch.Generator().manual_seed(3)
+                           ).cuda()
+    say("adjoint", n, np_, steps, ckpt)
+    w1, u1, d1, f1 = A.run(P, F, g, -1.0, 1.0, steps, ckpt, True, True, True)
+    w2, u2, d2, f2 = A.run(P[order].contiguous(), F, g, -1.0, 1.0, steps,
+                           ckpt, True, True, True)
+    w3 = A.run(P, F, g, -1.0, 1.0, steps, grads=False)[0]
+    assert abs(w1 - w2) <= 1e-12 * abs(w1) and abs(w1 - w3) <= 1e-12 * abs(w1)
+    for a, b in ((u1[order], u2), (d1[order], d2), (f1, f2)):
+        if a.numel():
+            assert float((a - b).abs().max()) <= \
+                1e-10 * float(a.abs().max()) + 1e-300
+    # FP32 against FP64: few particles and steps, so crossings fall on the
+    # same steps; 1e-2 in norm (the unstable 64^3 run over 200 steps, with
+    # moved crossings, parts by 1.6e-2)
+    if np_:
+        P4, F4 = _adjoint_inputs(g, np_, 5, False)
+        w4, u4, d4, f4 = A.run(P4, F4, g, -1.0, 1.0, steps, ckpt, True, True,
+                               True)
+        assert abs(w4 - w1) <= 1e-5 * abs(w1)
+        assert float((u4.double() - u1).norm()) <= 1e-2 * float(u1.norm())
+        assert float((f4.double() - f1).norm()) <= 1e-2 * float(f1.norm())

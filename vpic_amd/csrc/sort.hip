@@ -572,16 +572,14 @@ int sort_passes(const vpic_grid_t *g, int np, SortPass out[3]) {
   return n;
 }
 
-// The digit sort (grids up to RS_MAXB - 2 cells per axis).  With
-// `hint` (the caller's copy of p[k].i, k < np) the first pass reads the
-// keys from it instead of from the particles, and the gather checks every
-// particle's voxel index against the key it was sorted by; a difference,
-// or a key outside [0, nv), returns SORT_KEYS_STALE before p is touched.
-int sort_p_axes(vpic_particle_t *p, vpic_particle_t *aux, int np,
-                int *partition, const vpic_grid_t *g, int in_place,
-                const int *hint, hipStream_t s) {
+// The digit passes over np keys (np >= 1): `hint` (keys in any memory, one
+// outside [0, nv) sorted as 0 and counted in nbad[0]) or, without it, the
+// particles' voxel indices (an error when one is outside [0, nv)).  The sorted
+// keys and the order end in *sorted and *order (scratch).
+int sort_pairs(const vpic_particle_t *p, int np, const vpic_grid_t *g,
+               const int *hint, int **order, int **sorted, int **nbad_out,
+               hipStream_t s) {
   SortScratch &S = sort_scratch();
-  const int nv = g->nv;
   SortPass pass[3];
   const int npass = sort_passes(g, np, pass);
   int64_t nh = 0;
@@ -659,10 +657,26 @@ int sort_p_axes(vpic_particle_t *p, vpic_particle_t *aux, int np,
     std::swap(ka, kb);
     std::swap(ia, ib);
   }
+  *order = ia;
+  *sorted = ka;
+  *nbad_out = nbad;
+  return VPIC_OK;
+}
+
+// The digit sort (grids up to RS_MAXB - 2 cells per axis).  With
+// `hint` (the caller's copy of p[k].i, k < np) the first pass reads the
+// keys from it instead of from the particles, and the gather checks every
+// particle's voxel index against the key it was sorted by; a difference,
+// or a key outside [0, nv), returns SORT_KEYS_STALE before p is touched.
+int sort_p_axes(vpic_particle_t *p, vpic_particle_t *aux, int np,
+                int *partition, const vpic_grid_t *g, int in_place,
+                const int *hint, hipStream_t s) {
+  int rc, *ia, *ka, *nbad;
+  if ((rc = sort_pairs(p, np, g, hint, &ia, &ka, &nbad, s))) return rc;
   hipLaunchKernelGGL(k_gather_part<GATHER_GU>,
                      dim3(blocks_for((int64_t)np + 1, 128 * GATHER_GU)),
                      dim3(256), 0, s, p, (const int *)ia, (const int *)ka, np,
-                     nv, aux, partition, hint ? nbad + 1 : (int *)nullptr);
+                     g->nv, aux, partition, hint ? nbad + 1 : (int *)nullptr);
   VPIC_LAUNCHED("k_gather_part");
   if (hint) {
     int h[2] = {0, 0};
@@ -900,8 +914,7 @@ int launch_sort_p(vpic_particle_t *p, vpic_particle_t *aux, int np,
                   hipStream_t s) {
   push_invalidate_bins(p);
   push_invalidate_bins(aux);
-  if (np > 0 && g->nx + 2 <= RS_MAXB && g->ny + 2 <= RS_MAXB &&
-      g->nz + 2 <= RS_MAXB)
+  if (np > 0 && sort_keys_fit(g))
     return sort_p_axes(p, aux, np, partition, g, in_place, nullptr, s);
   return sort_p_counting(p, aux, np, partition, g, in_place, s);
 }
@@ -913,8 +926,7 @@ int launch_sort_p(vpic_particle_t *p, vpic_particle_t *aux, int np,
 int launch_sort_p_keys(vpic_particle_t *p, vpic_particle_t *aux, int np,
                        int *partition, const int *keys, const vpic_grid_t *g,
                        int in_place, hipStream_t s) {
-  if (!keys || !(np > 0 && g->nx + 2 <= RS_MAXB && g->ny + 2 <= RS_MAXB &&
-                 g->nz + 2 <= RS_MAXB))
+  if (!keys || !(np > 0 && sort_keys_fit(g)))
     return launch_sort_p(p, aux, np, partition, g, in_place, s);
   push_invalidate_bins(p);
   push_invalidate_bins(aux);
@@ -922,6 +934,22 @@ int launch_sort_p_keys(vpic_particle_t *p, vpic_particle_t *aux, int np,
   if (rc != SORT_KEYS_STALE) return rc;
   note_sort_keys_stale();
   return sort_p_axes(p, aux, np, partition, g, in_place, nullptr, s);
+}
+
+bool sort_keys_fit(const vpic_grid_t *g) {
+  return g->nx + 2 <= RS_MAXB && g->ny + 2 <= RS_MAXB && g->nz + 2 <= RS_MAXB;
+}
+
+int device_sort_keys(const int *keys, int np, const vpic_grid_t *g,
+                     int **order, int **sorted, int *bad, hipStream_t s) {
+  int rc, *nbad;
+  if ((rc = sort_pairs(nullptr, np, g, keys, order, sorted, &nbad, s)))
+    return rc;
+  if (bad) {
+    VPIC_HIP(hipMemcpyAsync(bad, nbad, sizeof(int), hipMemcpyDeviceToHost, s));
+    VPIC_HIP(hipStreamSynchronize(s));
+  }
+  return VPIC_OK;
 }
 
 long long sort_keys_stale_count() { return g_sort_keys_stale.load(); }
