@@ -842,13 +842,32 @@ int vpic_hip_ensemble_tune(vpic_ensemble_t *e, int32_t trial_steps,
  * dW/d(dx,dy,dz), f_bar[nv][6] = dW/d(ex,ey,ez,cbx,cby,cbz) of the initial
  * state.  *host_energy receives W.  All grid faces must be periodic.
  * Synchronous; allocates its checkpoints (about (n_step/ckpt_interval +
- * ckpt_interval) particle and field arrays). */
+ * ckpt_interval) particle and field arrays, and a permutation of the
+ * particles per eight steps) and releases them before it returns. */
 int vpic_hip_adjoint_bfield_energy(const void *p0, int32_t np, float q,
                                    float m, const void *f0,
                                    const vpic_grid_t *g, int32_t n_step,
                                    int32_t ckpt_interval, int32_t precision,
                                    double *host_energy, void *u_bar,
                                    void *d_bar, void *f_bar, void *stream);
+
+/* The same on device memory of the caller (256-byte aligned), who keeps it
+ * from call to call: `workspace` of at least the bytes that
+ * vpic_hip_adjoint_workspace gives for the same np, grid, steps, checkpoint
+ * interval, precision and grads (u_bar given or not).  The call owns it until
+ * it returns.  NULL: allocated and released by the call. */
+int vpic_hip_adjoint_workspace(int32_t np, const vpic_grid_t *g,
+                               int32_t n_step, int32_t ckpt_interval,
+                               int32_t precision, int32_t grads,
+                               int64_t *bytes);
+int vpic_hip_adjoint_bfield_energy_ws(const void *p0, int32_t np, float q,
+                                      float m, const void *f0,
+                                      const vpic_grid_t *g, int32_t n_step,
+                                      int32_t ckpt_interval,
+                                      int32_t precision, double *host_energy,
+                                      void *u_bar, void *d_bar, void *f_bar,
+                                      void *workspace, int64_t workspace_bytes,
+                                      void *stream);
 
 /* ------------------------------------------------------------------------ */
 /* Timing of the push kernel (hipEvents on the launch stream)               */

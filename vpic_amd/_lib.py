@@ -107,6 +107,10 @@ _SIGS = {
     "vpic_hip_adjoint_bfield_energy": [_vp, _i32, _f32, _f32, _vp, _pg, _i32,
                                        _i32, _i32, _pf64, _vp, _vp, _vp,
                                        _vp],
+    "vpic_hip_adjoint_workspace": [_i32, _pg, _i32, _i32, _i32, _i32, _pi64],
+    "vpic_hip_adjoint_bfield_energy_ws": [_vp, _i32, _f32, _f32, _vp, _pg,
+                                          _i32, _i32, _i32, _pf64, _vp, _vp,
+                                          _vp, _vp, _i64, _vp],
     "vpic_hip_ensemble_create": [_vp, _i32, _vp, _vp, _vp, _vp, _vp],
     "vpic_hip_ensemble_destroy": [_vp],
     "vpic_hip_ensemble_box": [_vp, _i32, _vp, _vp, _vp, _vp, _vp],

@@ -35,6 +35,23 @@ def set_momenta(part, u):
     return out
 
 
+def _workspace(np_, grid, n_step, ckpt, precision, grads, device):
+    """Device memory for one call from torch's caching allocator (a call's own
+    allocation of gigabytes costs up to three times its kernels): a tensor of
+    the default stream, which the library's work is ordered with, or None when
+    it does not fit (the library then allocates what it needs itself)."""
+    need = ctypes.c_int64()
+    _lib.call("vpic_hip_adjoint_workspace", np_, ctypes.byref(grid),
+              int(n_step), int(ckpt), precision, int(grads),
+              ctypes.byref(need))
+    try:
+        with torch.cuda.stream(torch.cuda.default_stream(device)):
+            # (the allocator aligns its blocks to 512 bytes)
+            return torch.empty(need.value, dtype=torch.uint8, device=device)
+    except torch.cuda.OutOfMemoryError:
+        return None
+
+
 def run(part, fields, grid, q, m, n_step, ckpt=20, grads=True,
         want_positions=False, want_fields=False):
     """The raw call: returns (energy, u_bar, d_bar, f_bar) with None for the
@@ -50,12 +67,15 @@ def run(part, fields, grid, q, m, n_step, ckpt=20, grads=True,
         if want_fields:
             fb = torch.empty((grid.nv, 6), dtype=part.dtype,
                              device=part.device)
-    _lib.call("vpic_hip_adjoint_bfield_energy", part.data_ptr(), np_,
+    ws = _workspace(np_, grid, n_step, ckpt, precision, grads, part.device)
+    _lib.call("vpic_hip_adjoint_bfield_energy_ws", part.data_ptr(), np_,
               float(q), float(m), fields.data_ptr(), ctypes.byref(grid),
               int(n_step), int(ckpt), precision, ctypes.byref(en),
               ub.data_ptr() if ub is not None else None,
               db.data_ptr() if db is not None else None,
-              fb.data_ptr() if fb is not None else None, None)
+              fb.data_ptr() if fb is not None else None,
+              ws.data_ptr() if ws is not None else None,
+              ws.numel() if ws is not None else 0, None)
     return en.value, ub, db, fb
 
 

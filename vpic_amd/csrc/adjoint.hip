@@ -1472,23 +1472,33 @@ __global__ void k_fields_out(R *dst, const Fld<R> *Fb, int nv) {
 // host driver
 // ---------------------------------------------------------------------------
 
-// One device allocation per call, cut into the run's arrays (an allocation
-// and a release of each of the dozens of arrays took longer than their
-// steps).
+// The device memory of a call, cut into the run's arrays: the caller's
+// workspace, or one allocation (each of the dozens of arrays allocated and
+// released on its own took longer than its steps; one allocation of 4.3 GB
+// still takes 1 to 95 ms against 31 ms of kernels, hence the workspace).
 struct Arena {
   char *p = nullptr;
-  size_t used = 0, size = 0;
+  bool own = false;
+  size_t used = 0;
   ~Arena() {
-    if (p) (void)hipFree(p);
+    if (own && p) (void)hipFree(p);
   }
-  int reserve(size_t bytes) {
+  int reserve(size_t bytes, void *ws, int64_t ws_bytes) {
+    if (ws) {
+      if (((uintptr_t)ws & 255u) != 0 || (int64_t)bytes > ws_bytes)
+        return vpic_set_error(VPIC_EINVAL, "adjoint run: the workspace of %lld "
+                              "bytes must be 256-byte aligned and hold %zu",
+                              (long long)ws_bytes, bytes);
+      p = (char *)ws;
+      return VPIC_OK;
+    }
     const hipError_t e = hipMalloc((void **)&p, bytes < 256 ? 256 : bytes);
     if (e != hipSuccess) {
       p = nullptr;
       return vpic_set_error(VPIC_ENOMEM, "adjoint: hipMalloc(%zu): %s", bytes,
                             hipGetErrorString(e));
     }
-    size = bytes;
+    own = true;
     return VPIC_OK;
   }
   static size_t room(size_t bytes) { return (bytes + 255) & ~(size_t)255; }
@@ -1708,16 +1718,18 @@ int check_periodic(const vpic_grid_t *g) {
   return VPIC_OK;
 }
 
-// The forward with checkpoints, then (when grads are wanted) the reverse.
+// The forward with checkpoints, then (when grads are wanted) the reverse; or
+// only the bytes that takes, when `want` is given.
 template <class R>
 int adjoint_run(const void *p0, int np, float q, float m, const void *f0,
-                const vpic_grid_t *g, int n_step, int ckpt, double *host_L,
-                void *u_bar, void *d_bar, void *f_bar, hipStream_t s) {
+                const vpic_grid_t *g, int n_step, int ckpt, bool grads,
+                double *host_L, void *u_bar, void *d_bar, void *f_bar,
+                void *ws, int64_t ws_bytes, int64_t *want, hipStream_t s) {
   int rc;
   if ((rc = check_periodic(g))) return rc;
-  if (np < 0 || n_step < 0 || (np > 0 && !p0) || !f0 || !host_L)
+  if (np < 0 || n_step < 0 ||
+      (!want && ((np > 0 && !p0) || !f0 || !host_L)))
     return vpic_set_error(VPIC_EINVAL, "adjoint run: bad arguments");
-  const bool grads = u_bar != nullptr;
   if (ckpt < 1) ckpt = n_step > 0 ? n_step : 1;
   Run<R> run;
   run.setup(g, np, q, m, s);
@@ -1771,7 +1783,11 @@ int adjoint_run(const void *p0, int np, float q, float m, const void *f0,
       fib = A.cut<R>(sizeof(R) * NI * (size_t)nv);
       accb = A.cut<R>(sizeof(R) * 12 * (size_t)nv);
     }
-    if (pass == 0 && (rc = A.reserve(A.used))) return rc;
+    if (want) {
+      *want = (int64_t)A.used;
+      return VPIC_OK;
+    }
+    if (pass == 0 && (rc = A.reserve(A.used, ws, ws_bytes))) return rc;
   }
   VPIC_HIP(hipMemsetAsync(run.err, 0, 64, s));
   if (np) VPIC_HIP(hipMemcpyAsync(run.p, p0, pbytes, hipMemcpyDeviceToDevice, s));
@@ -1865,18 +1881,50 @@ int adjoint_run(const void *p0, int np, float q, float m, const void *f0,
 
 }  // namespace
 
+extern "C" int vpic_hip_adjoint_workspace(int32_t np, const vpic_grid_t *g,
+                                          int32_t n_step,
+                                          int32_t ckpt_interval,
+                                          int32_t precision, int32_t grads,
+                                          int64_t *bytes) {
+  if (!bytes)
+    return vpic_set_error(VPIC_EINVAL, "adjoint workspace: bytes is NULL");
+  auto ask = [&](auto zero) {
+    return adjoint_run<decltype(zero)>(nullptr, np, 1.0f, 1.0f, nullptr, g,
+                                       n_step, ckpt_interval, grads != 0,
+                                       nullptr, nullptr, nullptr, nullptr,
+                                       nullptr, 0, bytes, nullptr);
+  };
+  if (precision == 4) return ask(0.0f);
+  if (precision == 8) return ask(0.0);
+  return vpic_set_error(VPIC_EINVAL, "adjoint run: precision %d (4 or 8)",
+                        precision);
+}
+
+extern "C" int vpic_hip_adjoint_bfield_energy_ws(
+    const void *p0, int32_t np, float q, float m, const void *f0,
+    const vpic_grid_t *g, int32_t n_step, int32_t ckpt_interval,
+    int32_t precision, double *host_energy, void *u_bar, void *d_bar,
+    void *f_bar, void *workspace, int64_t workspace_bytes, void *stream) {
+  const hipStream_t s = (hipStream_t)stream;
+  const bool grads = u_bar != nullptr;
+  if (precision == 4)
+    return adjoint_run<float>(p0, np, q, m, f0, g, n_step, ckpt_interval,
+                              grads, host_energy, u_bar, d_bar, f_bar,
+                              workspace, workspace_bytes, nullptr, s);
+  if (precision == 8)
+    return adjoint_run<double>(p0, np, q, m, f0, g, n_step, ckpt_interval,
+                               grads, host_energy, u_bar, d_bar, f_bar,
+                               workspace, workspace_bytes, nullptr, s);
+  return vpic_set_error(VPIC_EINVAL, "adjoint run: precision %d (4 or 8)",
+                        precision);
+}
+
 extern "C" int vpic_hip_adjoint_bfield_energy(
     const void *p0, int32_t np, float q, float m, const void *f0,
     const vpic_grid_t *g, int32_t n_step, int32_t ckpt_interval,
     int32_t precision, double *host_energy, void *u_bar, void *d_bar,
     void *f_bar, void *stream) {
-  const hipStream_t s = (hipStream_t)stream;
-  if (precision == 4)
-    return adjoint_run<float>(p0, np, q, m, f0, g, n_step, ckpt_interval,
-                              host_energy, u_bar, d_bar, f_bar, s);
-  if (precision == 8)
-    return adjoint_run<double>(p0, np, q, m, f0, g, n_step, ckpt_interval,
-                               host_energy, u_bar, d_bar, f_bar, s);
-  return vpic_set_error(VPIC_EINVAL, "adjoint run: precision %d (4 or 8)",
-                        precision);
+  return vpic_hip_adjoint_bfield_energy_ws(
+      p0, np, q, m, f0, g, n_step, ckpt_interval, precision, host_energy,
+      u_bar, d_bar, f_bar, nullptr, 0, stream);
 }
