@@ -162,3 +162,58 @@ def test_adjoint_workspace(dev):
         with pytest.raises(_lib.VpicError):
             call(ptr, n)
     assert A.run(P, F, g, -1.0, 1.0, 9, 4)[0] == pytest.approx(w, rel=1e-12)
+
+
+# one particle, around a workgroup's round, past one chunk per workgroup of
+# the least and of the most particles; in cell order (with drift), in no order
+# on a grid of more nodes than a chunk's table holds, axes of one cell
+@pytest.mark.parametrize("n,np_,order", [
+    ((4, 3, 5), 1, "sorted"), ((4, 3, 5), 511, "sorted"),
+    ((16, 9, 7), 513, "drifted"), ((64, 20, 10), 600001, "drifted"),
+    ((90, 60, 50), 40000, "random"), ((40, 1, 30), 70000, "drifted"),
+    ((1, 1, 6), 5000, "random")],
+    ids=lambda v: str(v).replace(" ", ""))
+def test_accumulate_rho_chunks(dev, n, np_, order):
+    """rhof against the same weights summed in FP64.  A node's sum of k terms
+    is off by at most k roundings of 2^-24 of the terms' magnitudes.  A term
+    w (1 +- dx)(1 +- dy)(1 +- dz) is formed as w -+ dx w and so on: six
+    roundings of values up to 8 w, whatever cancels."""
+    g = _box(*n)
+    rng = np.random.default_rng(np_ + 1)
+    c = [rng.integers(1, k + 1, np_) for k in n]
+    i = g.voxel(*c)
+    if order != "random":
+        i = np.sort(i)
+    p = np.zeros(np_, dtype=T.PARTICLE)
+    if order == "drifted":
+        moved = rng.random(np_) < 0.4
+        x = i % (g.nx + 2)
+        i = np.where(moved, i - x + 1 + (x + np_ % 2) % g.nx, i)
+    p["i"] = i
+    for k in ("dx", "dy", "dz"):
+        p[k] = rng.uniform(-1, 1, np_).astype(np.float32)
+    p["w"] = rng.uniform(0.5, 2, np_).astype(np.float32)
+    f = H.random_full_fields(g, 3)
+    want = f["rhof"].astype(np.float64)
+    mag, terms, full = np.abs(want), np.zeros(g.nv), np.zeros(g.nv)
+    d = [p[k].astype(np.float64) for k in ("dx", "dy", "dz")]
+    for k in range(8):
+        s = [(k >> a & 1) for a in range(3)]
+        w = p["w"] * (-0.7 * np.float64(g.r8V))
+        for a in range(3):
+            w = w * (1 + (2 * s[a] - 1) * d[a])
+        at = p["i"] + s[0] + s[1] * g.sy + s[2] * g.sz
+        np.add.at(want, at, w)
+        np.add.at(mag, at, np.abs(w))
+        np.add.at(terms, at, 1)
+        np.add.at(full, at, 8 * p["w"] * 0.7 * np.float64(g.r8V))
+    df, dp = dev.DeviceArray.from_host(f), dev.DeviceArray.from_host(p)
+    say("accumulate_rho_p", n, np_, order)
+    _lib.call("vpic_hip_accumulate_rho_p", df.ptr, dp.ptr, np_, -0.7,
+              ctypes.byref(g), None)
+    out = df.download()
+    err = np.abs(out["rhof"] - want)
+    assert np.all(err <= 2.0 ** -24 * ((terms + 2) * mag + 6 * full))
+    for k in T.FIELD_FLOATS:
+        if k != "rhof":
+            assert np.array_equal(out[k], f[k])

@@ -112,6 +112,68 @@ __device__ __forceinline__ int lanes_below(uint64_t m) {
       (unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
 }
 
+// A value of another lane by DPP (lanes without a valid source read 0).
+template <int CTRL, int ROW_MASK>
+__device__ __forceinline__ float dpp_get(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(
+      0, __float_as_int(v), CTRL, ROW_MASK, 0xf, true));
+}
+template <int CTRL, int ROW_MASK>
+__device__ __forceinline__ double dpp_get(double v) {
+  const long long b = __double_as_longlong(v);
+  const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(
+      0, (int)b, CTRL, ROW_MASK, 0xf, true);
+  const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp(
+      0, (int)(b >> 32), CTRL, ROW_MASK, 0xf, true);
+  return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+
+// Sums `v` over every run of lanes with the same key: the last lane of a run
+// ends with its sum (and gets true).  Whole wavefronts only.  Steps of 1, 2,
+// 4 and 8 lanes inside the 16-lane rows (row_shr), then the rows' carries
+// (row_bcast:15, row_bcast:31), each adding only within the run.
+template <class R, int N>
+__device__ __forceinline__ bool run_sums(int key, R (&v)[N]) {
+  const int lane = lane_id();
+  const int prev = __shfl_up(key, 1);
+  const uint64_t heads = __ballot(lane == 0 || prev != key);
+  const uint64_t upto = lane == 63 ? ~0ull : ((2ull << lane) - 1ull);
+  const int first = 63 - __clzll(heads & upto);
+  const int r = lane & 15;
+#define VPIC_RUN_STEP(CTRL, MASK, TAKE)                 \
+  {                                                \
+    const bool take_ = (TAKE);                     \
+    _Pragma("unroll") for (int k = 0; k < N; k++) { \
+      const R t_ = dpp_get<CTRL, MASK>(v[k]);      \
+      v[k] += take_ ? t_ : R(0);                   \
+    }                                              \
+  }
+  VPIC_RUN_STEP(0x111, 0xf, r >= 1 && lane - 1 >= first)
+  VPIC_RUN_STEP(0x112, 0xf, r >= 2 && lane - 2 >= first)
+  VPIC_RUN_STEP(0x114, 0xf, r >= 4 && lane - 4 >= first)
+  VPIC_RUN_STEP(0x118, 0xf, r >= 8 && lane - 8 >= first)
+  VPIC_RUN_STEP(0x142, 0xa, ((lane >> 4) & 1) && first <= (lane & ~15) - 1)
+  VPIC_RUN_STEP(0x143, 0xc, lane >= 32 && first <= 31)
+#undef VPIC_RUN_STEP
+  return lane == 63 || (((heads >> lane) >> 1) & 1ull);
+}
+
+// Sum over a workgroup of BS threads (all of them call): wavefronts by
+// shuffles, their sums through sh (BS / 64 doubles).  Valid in thread 0.
+template <int BS>
+__device__ __forceinline__ double block_sum(double v, double *sh) {
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) v += __shfl_down(v, d);
+  __syncthreads();
+  if (lane_id() == 0) sh[threadIdx.x >> 6] = v;
+  __syncthreads();
+  double s = 0.0;
+  if (threadIdx.x == 0)
+#pragma unroll
+    for (int k = 0; k < BS / 64; k++) s += sh[k];
+  return s;
+}
+
 // ---------------------------------------------------------------------------
 // Host-side helpers shared by the launchers (defined in api.hip)
 // ---------------------------------------------------------------------------

@@ -482,14 +482,18 @@ __global__ void k_adjust_tang_e(vpic_field_t *f, FaceGeom G, int4 m0,
 // energy_f: per-voxel FP32 terms, FP64 sums (per-block partials, then one
 // block folds them in a fixed order).
 // ---------------------------------------------------------------------------
+// (few partials, as in diag.hip: their sum is one workgroup's work)
+constexpr int MAX_PARTIALS = 1024;
+
 __global__ __launch_bounds__(256) void k_energy_f(const vpic_field_t *__restrict__ f,
                                                   Box b, int nx, int ny,
                                                   float4 q, float4 h,
                                                   double *__restrict__ part) {
-  __shared__ double red[6][256];
-  int x, y, z;
+  __shared__ double sh[4];
   double en[6] = {0, 0, 0, 0, 0, 0};
-  if (box_coords(b, blockIdx.x * (int64_t)blockDim.x + threadIdx.x, x, y, z)) {
+  int x, y, z;
+  for (int64_t l = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+       box_coords(b, l, x, y, z); l += (int64_t)gridDim.x * blockDim.x) {
     const int v = vox(x, y, z, nx, ny);
     const int sy = nx + 2, sz = (ny + 2) * sy;
     const float4 e0 = F4(f, v)[0], b0 = F4(f, v)[1];
@@ -499,44 +503,33 @@ __global__ __launch_bounds__(256) void k_energy_f(const vpic_field_t *__restrict
     const float eyz = F4(f, v + sy + sz)[0].x;
     const float ezx = F4(f, v + sz + 1)[0].y;
     const float exy = F4(f, v + 1 + sy)[0].z;
-    en[0] = (double)(q.x * (e0.x * e0.x + ey_.x * ey_.x + ez_.x * ez_.x +
-                            eyz * eyz));
-    en[1] = (double)(q.y * (e0.y * e0.y + ez_.y * ez_.y + ex_.y * ex_.y +
-                            ezx * ezx));
-    en[2] = (double)(q.z * (e0.z * e0.z + ex_.z * ex_.z + ey_.z * ey_.z +
-                            exy * exy));
-    en[3] = (double)(h.x * (b0.x * b0.x + bx_.x * bx_.x));
-    en[4] = (double)(h.y * (b0.y * b0.y + by_.y * by_.y));
-    en[5] = (double)(h.z * (b0.z * b0.z + bz_.z * bz_.z));
+    en[0] += (double)(q.x * (e0.x * e0.x + ey_.x * ey_.x + ez_.x * ez_.x +
+                             eyz * eyz));
+    en[1] += (double)(q.y * (e0.y * e0.y + ez_.y * ez_.y + ex_.y * ex_.y +
+                             ezx * ezx));
+    en[2] += (double)(q.z * (e0.z * e0.z + ex_.z * ex_.z + ey_.z * ey_.z +
+                             exy * exy));
+    en[3] += (double)(h.x * (b0.x * b0.x + bx_.x * bx_.x));
+    en[4] += (double)(h.y * (b0.y * b0.y + by_.y * by_.y));
+    en[5] += (double)(h.z * (b0.z * b0.z + bz_.z * bz_.z));
   }
-  for (int k = 0; k < 6; k++) red[k][threadIdx.x] = en[k];
-  __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if (threadIdx.x < s)
-      for (int k = 0; k < 6; k++)
-        red[k][threadIdx.x] += red[k][threadIdx.x + s];
-    __syncthreads();
+#pragma unroll
+  for (int k = 0; k < 6; k++) {
+    const double s = block_sum<256>(en[k], sh);
+    if (threadIdx.x == 0) part[6 * (int64_t)blockIdx.x + k] = s;
   }
-  if (threadIdx.x < 6) part[6 * (int64_t)blockIdx.x + threadIdx.x] =
-      red[threadIdx.x][0];
 }
 
 __global__ __launch_bounds__(256) void k_fold_partials(const double *part,
                                                        int nblk, int width,
                                                        double *out) {
-  __shared__ double red[256];
+  __shared__ double sh[4];
   for (int k = 0; k < width; k++) {
     double s = 0;
     for (int i = threadIdx.x; i < nblk; i += blockDim.x)
       s += part[(int64_t)width * i + k];
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int st = 128; st > 0; st >>= 1) {
-      if (threadIdx.x < st) red[threadIdx.x] += red[threadIdx.x + st];
-      __syncthreads();
-    }
-    if (threadIdx.x == 0) out[k] = red[0];
-    __syncthreads();
+    s = block_sum<256>(s, sh);
+    if (threadIdx.x == 0) out[k] = s;
   }
 }
 
@@ -737,32 +730,28 @@ __global__ __launch_bounds__(256) void k_sq_partials(const vpic_field_t *__restr
                                                      Box b, int nx, int ny,
                                                      int nz,
                                                      double *__restrict__ part) {
-  __shared__ double red[256];
+  __shared__ double sh[4];
   int x, y, z;
   double e = 0;
-  if (box_coords(b, blockIdx.x * (int64_t)blockDim.x + threadIdx.x, x, y, z)) {
+  for (int64_t l = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+       box_coords(b, l, x, y, z); l += (int64_t)gridDim.x * blockDim.x) {
     const float d = reinterpret_cast<const float *>(
         f + vox(x, y, z, nx, ny))[DIVB ? 7 : 3];
     if (DIVB) {
-      e = d * d;
+      e += d * d;
     } else {
       const int nb = (x == 1 || x == nx + 1) + (y == 1 || y == ny + 1) +
                      (z == 1 || z == nz + 1);
       if (nb == 0) {
-        e = d * d;
+        e += d * d;
       } else {
         const double w = nb == 1 ? 0.5 : nb == 2 ? 0.25 : 0.125;
-        e = w * (double)d * (double)d;
+        e += w * (double)d * (double)d;
       }
     }
   }
-  red[threadIdx.x] = e;
-  __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if (threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) part[blockIdx.x] = red[0];
+  const double s = block_sum<256>(e, sh);
+  if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 
 // synchronize_tang_e_norm_b on the periodic face pair of axis X
@@ -1158,6 +1147,7 @@ int launch_energy_f(double en[6], const vpic_field_t *f, const vpic_grid_t *g,
   Box b = {1, 1, 1, g->nx, g->ny, g->nz};
   int64_t n = (int64_t)g->nx * g->ny * g->nz;
   int nblk = blocks_for(n, 256);
+  if (nblk > MAX_PARTIALS) nblk = MAX_PARTIALS;
   int rc;
   if ((rc = scratch_reserve(S.part, sizeof(double) * 6 * (size_t)nblk)) ||
       (rc = scratch_reserve(S.out, sizeof(double) * 8)))
@@ -1282,7 +1272,8 @@ int launch_compute_rms_div_err(double *out, const vpic_field_t *f,
   EnergyScratch &S = energy_scratch();
   const Box b = divb ? Box{1, 1, 1, g->nx, g->ny, g->nz} : node_box(g);
   const int64_t n = divb ? (int64_t)g->nx * g->ny * g->nz : node_count(g);
-  const int nblk = blocks_for(n, 256);
+  int nblk = blocks_for(n, 256);
+  if (nblk > MAX_PARTIALS) nblk = MAX_PARTIALS;
   int rc;
   if ((rc = scratch_reserve(S.part, sizeof(double) * (size_t)nblk))) return rc;
   if (divb)
