@@ -217,3 +217,45 @@ def test_accumulate_rho_chunks(dev, n, np_, order):
     for k in T.FIELD_FLOATS:
         if k != "rhof":
             assert np.array_equal(out[k], f[k])
+
+
+# one particle; 16 lanes of one voxel and one more; few particles over a grid
+# of two slabs of voxels; axes of one cell; an axis too long to sort by
+@pytest.mark.parametrize("n,np_", [
+    ((4, 3, 5), 1), ((2, 1, 2), 16 * 4 + 1), ((9, 8, 7), 12000),
+    ((70, 70, 63), 30000), ((33, 1, 20), 5000), ((2100, 1, 1), 4000)],
+    ids=lambda v: str(v).replace(" ", ""))
+def test_hydro_voxel_sums(dev, orc, n, np_):
+    """The moments of particles in no order against the oracle's, within the
+    1e-5 of each moment's largest value that its other order of summing
+    allows; added to what the array holds."""
+    g = _box(*n)
+    rng = np.random.default_rng(np_)
+    f = H.random_fields(g, 4, 0.1, 0.2)
+    fi = H.interp_array(g)
+    orc.load_interpolator(fi, f, g)
+    p = np.zeros(np_, dtype=T.PARTICLE)
+    p["i"] = g.voxel(*(rng.integers(1, k + 1, np_) for k in n))
+    for k in ("dx", "dy", "dz"):
+        p[k] = rng.uniform(-1, 1, np_).astype(np.float32)
+    for k in ("ux", "uy", "uz"):
+        p[k] = (0.3 * rng.standard_normal(np_)).astype(np.float32)
+    p["w"] = rng.uniform(0.5, 2, np_).astype(np.float32)
+    want = np.zeros(g.nv, dtype=T.HYDRO)
+    want["rho"] = 0.25
+    dh = dev.DeviceArray.from_host(want)
+    orc.accumulate_hydro_p(want, p, -1.0, 1.0, fi, g)
+    dp, dfi = dev.DeviceArray.from_host(p), dev.DeviceArray.from_host(fi)
+    say("accumulate_hydro_p", n, np_)
+    _lib.call("vpic_hip_accumulate_hydro_p", dh.ptr, dp.ptr, np_, -1.0, 1.0,
+              dfi.ptr, ctypes.byref(g), None, None)
+    got = dh.download()
+    for k in T.HYDRO_FIELDS:
+        assert np.max(np.abs(got[k] - want[k])) <= \
+            1e-5 * np.max(np.abs(want[k])), k
+    # a particle whose nodes leave the grid is skipped and reported
+    p["i"][np_ // 2] = g.nv - 3
+    dp = dev.DeviceArray.from_host(p)
+    with pytest.raises(_lib.VpicError, match="1 particles"):
+        _lib.call("vpic_hip_accumulate_hydro_p", dh.ptr, dp.ptr, np_, -1.0,
+                  1.0, dfi.ptr, ctypes.byref(g), None, None)

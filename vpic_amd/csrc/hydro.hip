@@ -7,11 +7,18 @@
 //
 // Each particle's half E kick, half Boris rotation, velocity and trilinear
 // node weights are the reference's expressions in the same order; the 14
-// node sums differ only in summation order.  With the sort-time partition
-// the particles of a tile of cells are pushed by one workgroup: a lane
-// sums its consecutive particles of one voxel in registers (8 nodes x 14
-// moments), adds the sums to an LDS window of the tile's nodes when the
-// voxel changes, and the window is added to the array at the end.
+// node sums differ only in summation order.
+//
+// A particle adds 112 numbers (8 nodes x 14 moments), so what costs is
+// adding them up: a sort of the particle indices by their voxels as they are
+// now (not as a partition of the last sort_p has them) lets 16 lanes sum the
+// particles of one voxel in registers and add the lanes up with DPP; the
+// voxels' 112 sums go to a buffer, slab by slab, and every node gathers the
+// eight it takes.  No atomics.  1.5e7 particles on 72x64x50 cells that drifted
+// by half a cell since the sort: 0.77 ms, of which the sort is 0.33 (6.5
+// ms with LDS windows per tile, whose float atomics a drifted particle needs
+// one by one).  Grids with an axis too long for that sort go particle by
+// particle with global atomics.
 #include "common.h"
 
 namespace {
@@ -20,12 +27,11 @@ struct HydroCoef {
   float qsp, qdt_2mc, qdt_4mc2, mspc, c, r8V;
 };
 
-struct HydroTile {
-  int tx, ty, tz, ntx, nty, ntz;
-};
-
-constexpr int HY_BS = 512;
-constexpr int HY_MAXROWS = 256;
+constexpr int HY_LANES = 16;  // lanes per voxel (one DPP row)
+constexpr int HY_SUMS = 8 * 14;
+// Slabs of voxels whose sums (448 B each) stay in the 256-MB cache between
+// the kernel that writes them and the one that reads them.
+constexpr int64_t HY_SLAB_BYTES = (int64_t)128 << 20;
 
 // The per-particle part of accumulate_hydro_p_pipeline_scalar
 // (hydro_p_pipeline.cc:65-172): node weights wn[8] and the 14 moments per
@@ -118,14 +124,13 @@ __device__ __forceinline__ int node_off(int k, int sy, int sz) {
   return (k & 1) + ((k >> 1) & 1) * sy + (k >> 2) * sz;
 }
 
-// Flat: one lane per particle, global float atomics (no partition).
+// Flat: one lane per particle, global float atomics (no sort).
 __global__ __launch_bounds__(256) void k_hydro_flat(
-    const vpic_particle_t *__restrict__ p, const int *__restrict__ start,
-    int np, const vpic_interpolator_t *__restrict__ f0, float *__restrict__ hy,
+    const vpic_particle_t *__restrict__ p, int np,
+    const vpic_interpolator_t *__restrict__ f0, float *__restrict__ hy,
     HydroCoef C, int nv, int sy, int sz, int *__restrict__ nbad) {
-  const int n0 = start ? min(max(*start, 0), np) : 0;
-  for (int n = n0 + blockIdx.x * blockDim.x + threadIdx.x; n < np;
-       n += gridDim.x * blockDim.x) {
+  for (int64_t n = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; n < np;
+       n += (int64_t)gridDim.x * blockDim.x) {
     const float4 *pp = reinterpret_cast<const float4 *>(p + n);
     const float4 A = pp[0], B = pp[1];
     const int ii = __float_as_int(A.w);
@@ -148,112 +153,109 @@ __global__ __launch_bounds__(256) void k_hydro_flat(
   }
 }
 
-// Tiled: one workgroup per tile of cells over the partition rows; the
-// window holds the tile's nodes (x0..x1+1, ...), component-major.
-__global__ __launch_bounds__(HY_BS) void k_hydro_tiled(
-    const vpic_particle_t *__restrict__ p, int np, const int *__restrict__ part,
-    const vpic_interpolator_t *__restrict__ f0, float *__restrict__ hy,
-    HydroCoef C, GridDev G, HydroTile T, int *__restrict__ nbad) {
-  extern __shared__ float hwin[];  // 14 * nnode
-  __shared__ int row_start[HY_MAXROWS];
-  __shared__ int row_pref[HY_MAXROWS + 1];
-  const int t = threadIdx.x;
-  int b = blockIdx.x;
-  const int btx = b % T.ntx;
-  b /= T.ntx;
-  const int bty = b % T.nty;
-  const int btz = b / T.nty;
-  const int x0 = 1 + btx * T.tx, y0 = 1 + bty * T.ty, z0 = 1 + btz * T.tz;
-  const int x1 = min(x0 + T.tx - 1, G.nx), y1 = min(y0 + T.ty - 1, G.ny),
-            z1 = min(z0 + T.tz - 1, G.nz);
-  const int rows_y = y1 - y0 + 1;
-  const int nrow = rows_y * (z1 - z0 + 1);
-  const int wnx = x1 - x0 + 2, wny = y1 - y0 + 2, wnz = z1 - z0 + 2;
-  const int nnode = wnx * wny * wnz;
-  const int sx1 = G.nx + 2, sy1 = G.ny + 2;
-  const int sy = sx1, sz = sx1 * sy1;
-  for (int r = t; r < nrow; r += HY_BS) {
-    const int y = y0 + r % rows_y, z = z0 + r / rows_y;
-    int s = part[vox(x0, y, z, G.nx, G.ny)];
-    int e = part[vox(x1 + 1, y, z, G.nx, G.ny)];
-    s = min(max(s, 0), np);
-    e = min(max(e, s), np);
-    row_start[r] = s;
-    row_pref[r + 1] = e - s;
+// The particles' voxels as sort keys; one whose nodes are not all on the grid
+// is counted and takes the last voxel, which no valid particle has.
+__global__ __launch_bounds__(256) void k_hydro_keys(
+    const vpic_particle_t *__restrict__ p, int np, int vmax, int nv,
+    int *__restrict__ keys, int *__restrict__ nbad) {
+  for (int64_t n = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; n < np;
+       n += (int64_t)gridDim.x * blockDim.x) {
+    int v = p[n].i;
+    if ((unsigned)v >= (unsigned)vmax) {
+      atomicAdd(nbad, 1);
+      v = nv - 1;
+    }
+    keys[n] = v;
   }
-  for (int k = t; k < 14 * nnode; k += HY_BS) hwin[k] = 0.0f;
-  __syncthreads();
-  if (t == 0) {
-    row_pref[0] = 0;
-    for (int r = 0; r < nrow; r++) row_pref[r + 1] += row_pref[r];
-  }
-  __syncthreads();
-  const int total = row_pref[nrow];
+}
 
+// start[v] = the first place whose key is not below v (v = 0..nv).
+__global__ __launch_bounds__(256) void k_hydro_starts(
+    const int *__restrict__ keys, int np, int nv, int *__restrict__ start) {
+  const int v = blockIdx.x * blockDim.x + threadIdx.x;
+  if (v > nv) return;
+  int lo = 0, hi = np;
+  while (lo < hi) {
+    const int mid = lo + ((hi - lo) >> 1);
+    if (keys[mid] < v)
+      lo = mid + 1;
+    else
+      hi = mid;
+  }
+  start[v] = lo;
+}
+
+// Level of the reduce-scatter of N values over a 16-lane row: the upper lanes
+// of each pair keep the upper half of the values, the lower the lower, plus
+// the partner's.
+template <int CTRL, int N>
+__device__ __forceinline__ void row_halve(bool upper, const float (&v)[2 * N],
+                                          float (&o)[N]) {
+#pragma unroll
+  for (int k = 0; k < N; k++)
+    o[k] = (upper ? v[k + N] : v[k]) +
+           dpp_get<CTRL, 0xf>(upper ? v[k] : v[k + N]);
+}
+
+// Sums of the particles of voxels [v0, v1), 16 lanes each, to
+// sums[(v - v0) * 112 + 14 node + moment]; nothing is written for a voxel
+// without particles.
+__global__ __launch_bounds__(256) void k_hydro_cells(
+    const vpic_particle_t *__restrict__ p, const int *__restrict__ order,
+    const int *__restrict__ start, const vpic_interpolator_t *__restrict__ f0,
+    float *__restrict__ sums, HydroCoef C, int v0, int v1) {
+  const int j = threadIdx.x & (HY_LANES - 1);
+  const int v = v0 + (int)((blockIdx.x * (int64_t)blockDim.x + threadIdx.x) /
+                           HY_LANES);
+  int s = 0, e = 0;
+  if (v < v1) {
+    s = start[v];
+    e = start[v + 1];
+  }
   float acc[8][14];
 #pragma unroll
   for (int k = 0; k < 8; k++)
 #pragma unroll
     for (int c = 0; c < 14; c++) acc[k][c] = 0.0f;
-  int key = -1;
-  int bad = 0;
-
-  auto flush = [&]() {
-    const int v = key;
-    const int zz = v / sz, rem = v - zz * sz, yy = rem / sy, xx = rem - yy * sy;
-    const int lx = xx - x0, ly = yy - y0, lz = zz - z0;
-#pragma unroll
-    for (int k = 0; k < 8; k++) {
-      const int ax = lx + (k & 1), ay = ly + ((k >> 1) & 1), az = lz + (k >> 2);
-      if ((unsigned)ax < (unsigned)wnx && (unsigned)ay < (unsigned)wny &&
-          (unsigned)az < (unsigned)wnz) {
-        const int s = ax + wnx * (ay + wny * az);
-#pragma unroll
-        for (int c = 0; c < 14; c++) atomicAdd(&hwin[c * nnode + s], acc[k][c]);
-      } else {
-        float *h = hy + 16 * (int64_t)(v + node_off(k, sy, sz));
-#pragma unroll
-        for (int c = 0; c < 14; c++) atomic_add_f32(h + c, acc[k][c]);
-      }
-#pragma unroll
-      for (int c = 0; c < 14; c++) acc[k][c] = 0.0f;
-    }
-  };
-
-  // lane t takes one contiguous run of the tile's slots (the rows of the
-  // partition back to back), so its particles mostly share a voxel and
-  // the register sums reach the LDS window about once per voxel
-  const int per = (total + HY_BS - 1) / HY_BS;
-  const int k0 = min(t * per, total), k1 = min(k0 + per, total);
-  int r = 0;
-  while (r + 1 < nrow && row_pref[r + 1] <= k0) r++;
-  for (int k = k0; k < k1; k++) {
-    while (k >= row_pref[r + 1]) r++;
-    const int n = row_start[r] + (k - row_pref[r]);
-    const float4 *pp = reinterpret_cast<const float4 *>(p + n);
+  for (int k = s + j; k < e; k += HY_LANES) {
+    const float4 *pp = reinterpret_cast<const float4 *>(p + order[k]);
     const float4 A = pp[0], B = pp[1];
-    const int ii = __float_as_int(A.w);
-    if ((unsigned)ii >= (unsigned)G.nv || ii + sz + sy + 1 >= G.nv) {
-      bad++;
-      continue;
-    }
-    if (ii != key) {
-      if (key >= 0) flush();
-      key = ii;
-    }
-    hydro_particle(A, B, f0 + ii, C, acc);
+    hydro_particle(A, B, f0 + v, C, acc);
   }
-  if (key >= 0) flush();
-  if (bad) atomicAdd(nbad, bad);
-  __syncthreads();
-  for (int k = t; k < 14 * nnode; k += HY_BS) {
-    const float v = hwin[k];
-    if (v == 0.0f) continue;
-    const int c = k / nnode, s = k - c * nnode;
-    const int ax = s % wnx, ay = (s / wnx) % wny, az = s / (wnx * wny);
-    atomic_add_f32(hy + 16 * (int64_t)vox(x0 + ax, y0 + ay, z0 + az, G.nx, G.ny) + c,
-                   v);
+  // (whole rows run from here: the lanes of a row share a voxel)
+  float a112[HY_SUMS], a56[56], a28[28], a14[14], a7[7];
+#pragma unroll
+  for (int k = 0; k < HY_SUMS; k++) a112[k] = acc[k / 14][k % 14];
+  row_halve<0x140, 56>(j & 8, a112, a56);  // row_mirror
+  row_halve<0x141, 28>(j & 4, a56, a28);   // row_half_mirror
+  row_halve<0x1b, 14>(j & 2, a28, a14);    // quad_perm 3,2,1,0
+  row_halve<0xb1, 7>(j & 1, a14, a7);      // quad_perm 1,0,3,2
+  if (s < e) {
+    float *o = sums + (int64_t)(v - v0) * HY_SUMS + 7 * j;
+#pragma unroll
+    for (int k = 0; k < 7; k++) o[k] = a7[k];
   }
+}
+
+// Nodes [n0, n1): 16 lanes each, one per moment, gather the eight voxels
+// (from v0 on in sums) a node belongs to.
+__global__ __launch_bounds__(256) void k_hydro_nodes(
+    const float *__restrict__ sums, const int *__restrict__ start,
+    float *__restrict__ hy, int v0, int vmax, int n0, int n1, int sy, int sz) {
+  const int c = threadIdx.x & 15;
+  const int n = n0 + (int)((blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >>
+                           4);
+  if (n >= n1 || c >= 14) return;
+  float s = 0.0f;
+  bool any = false;
+#pragma unroll
+  for (int k = 0; k < 8; k++) {
+    const int v = n - node_off(k, sy, sz);
+    if (v < 0 || v >= vmax || start[v] == start[v + 1]) continue;
+    any = true;
+    s += sums[(int64_t)(v - v0) * HY_SUMS + 14 * k + c];
+  }
+  if (any) hy[16 * (int64_t)n + c] += s;
 }
 
 // synchronize_hydro_array (hydro_array.cc:131-311) for one domain: local
@@ -304,7 +306,7 @@ __global__ __launch_bounds__(256) void k_hydro_zero(float4 *h, int64_t n4) {
 }
 
 struct HydroScratch {
-  DeviceScratch nbad;
+  DeviceScratch nbad, keys, start, sums;
 };
 HydroScratch &hydro_scratch() {
   static thread_local HydroScratch s[16];
@@ -345,27 +347,57 @@ int launch_accumulate_hydro_p(vpic_hydro_t *h, const vpic_particle_t *p,
   C.mspc = g->cvac * m;
   C.c = g->cvac;
   C.r8V = g->r8V;
-  if (np > 0) {
-    if (partition) {
-      HydroTile T = {8, 8, 4, 0, 0, 0};
-      T.ntx = (g->nx + T.tx - 1) / T.tx;
-      T.nty = (g->ny + T.ty - 1) / T.ty;
-      T.ntz = (g->nz + T.tz - 1) / T.tz;
-      const size_t lds = sizeof(float) * 14 * (T.tx + 1) * (T.ty + 1) * (T.tz + 1);
-      const GridDev G = make_grid_dev(g);
-      hipLaunchKernelGGL(k_hydro_tiled, dim3(T.ntx * T.nty * T.ntz),
-                         dim3(HY_BS), lds, s, p, np, partition, f,
-                         (float *)h, C, G, T, nbad);
-      VPIC_LAUNCHED("k_hydro_tiled");
-    }
-    // without a partition every particle, with one the particles past it
-    // (added since the sort), one lane each
+  // (the voxels are the particles' own: the partition of their last sort is
+  // not needed)
+  (void)partition;
+  // voxels whose eight nodes lie on the grid
+  const int vmax = g->nv - g->sz - g->sy - 1;
+  if (np > 0 && !sort_keys_fit(g)) {
     int nb = blocks_for(np, 256);
     if (nb > 16384) nb = 16384;
-    hipLaunchKernelGGL(k_hydro_flat, dim3(nb), dim3(256), 0, s, p,
-                       partition ? partition + g->nv : (const int *)nullptr,
-                       np, f, (float *)h, C, g->nv, g->sy, g->sz, nbad);
+    hipLaunchKernelGGL(k_hydro_flat, dim3(nb), dim3(256), 0, s, p, np, f,
+                       (float *)h, C, g->nv, g->sy, g->sz, nbad);
     VPIC_LAUNCHED("k_hydro_flat");
+  } else if (np > 0) {
+    // nodes per slab; their voxels reach back by one plane, row and cell
+    const int back = g->sz + g->sy + 1;
+    int64_t slab = HY_SLAB_BYTES / (4 * HY_SUMS) - back;
+    if (slab < back) slab = back;
+    if (slab > g->nv) slab = g->nv;
+    if ((rc = scratch_reserve(S.keys, sizeof(int) * (size_t)np)) ||
+        (rc = scratch_reserve(S.start, sizeof(int) * ((size_t)g->nv + 1))) ||
+        (rc = scratch_reserve(S.sums, sizeof(float) * HY_SUMS *
+                                          (size_t)(slab + back))))
+      return rc;
+    int *keys = (int *)S.keys.ptr, *start = (int *)S.start.ptr;
+    float *sums = (float *)S.sums.ptr;
+    int nb = blocks_for(np, 256);
+    if (nb > 8192) nb = 8192;
+    hipLaunchKernelGGL(k_hydro_keys, dim3(nb), dim3(256), 0, s, p, np, vmax,
+                       g->nv, keys, nbad);
+    VPIC_LAUNCHED("k_hydro_keys");
+    int *order, *sorted;
+    if ((rc = device_sort_keys(keys, np, g, &order, &sorted, nullptr, s)))
+      return rc;
+    hipLaunchKernelGGL(k_hydro_starts, dim3(blocks_for((int64_t)g->nv + 1, 256)),
+                       dim3(256), 0, s, (const int *)sorted, np, g->nv, start);
+    VPIC_LAUNCHED("k_hydro_starts");
+    for (int64_t n0 = 0; n0 < g->nv; n0 += slab) {
+      const int64_t n1 = n0 + slab < g->nv ? n0 + slab : g->nv;
+      const int64_t v0 = n0 > back ? n0 - back : 0;
+      const int64_t v1 = n1 < vmax ? n1 : vmax;
+      if (v1 <= v0) continue;
+      hipLaunchKernelGGL(k_hydro_cells,
+                         dim3(blocks_for((v1 - v0) * HY_LANES, 256)),
+                         dim3(256), 0, s, p, (const int *)order,
+                         (const int *)start, f, sums, C, (int)v0, (int)v1);
+      VPIC_LAUNCHED("k_hydro_cells");
+      hipLaunchKernelGGL(k_hydro_nodes, dim3(blocks_for((n1 - n0) * 16, 256)),
+                         dim3(256), 0, s, (const float *)sums,
+                         (const int *)start, (float *)h, (int)v0, vmax,
+                         (int)n0, (int)n1, g->sy, g->sz);
+      VPIC_LAUNCHED("k_hydro_nodes");
+    }
   }
   int h_bad = 0;
   VPIC_HIP(hipMemcpyAsync(&h_bad, nbad, sizeof(int), hipMemcpyDeviceToHost, s));
