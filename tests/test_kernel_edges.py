@@ -259,3 +259,33 @@ def test_hydro_voxel_sums(dev, orc, n, np_):
     with pytest.raises(_lib.VpicError, match="1 particles"):
         _lib.call("vpic_hip_accumulate_hydro_p", dh.ptr, dp.ptr, np_, -1.0,
                   1.0, dfi.ptr, ctypes.byref(g), None, None)
+
+
+# the one-launch jf fold and tangential-B ghosts where an axis has one or two
+# cells (its two faces are neighbours), periodic or with walls on one axis
+@pytest.mark.parametrize("wall", [None, 0, 1, 2])
+@pytest.mark.parametrize("n", [(1, 1, 1), (1, 5, 3), (2, 2, 2), (4, 1, 1),
+                               (3, 2, 70)],
+                         ids=lambda v: "x".join(map(str, v)))
+def test_faces_in_one_launch(dev, orc, n, wall):
+    """Bit for bit the oracle's axis after axis."""
+    g = T.grid_periodic(0, 0, 0, *n, *n, 0.4)
+    if wall is not None:
+        g.fbc[wall] = g.fbc[wall + 3] = T.BC_PEC_FIELDS
+    f = H.random_full_fields(g, 9)
+    mp = T.vacuum_params()
+    df = dev.DeviceArray.from_host(f)
+    say("faces", n, wall)
+    G = ctypes.byref(g)
+    _lib.call("vpic_hip_synchronize_jf", df.ptr, G, None)
+    _lib.call("vpic_hip_vacuum_advance_e", df.ptr, G, ctypes.byref(mp), 1.0,
+              None)
+    _lib.call("vpic_hip_compute_div_e_err", df.ptr, G, ctypes.byref(mp), None)
+    _lib.call("vpic_hip_clean_div_b", df.ptr, G, None)
+    orc.synchronize_jf(f, g)
+    orc.vacuum_advance_e(f, g, mp)
+    orc.compute_div_e_err(f, g, mp)
+    orc.clean_div_b(f, g)
+    got = df.download()
+    for c in T.FIELD_FLOATS:
+        assert H.same_bits(got[c], f[c]), c

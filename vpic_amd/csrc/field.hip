@@ -28,12 +28,13 @@ struct Box {
 
 __device__ __forceinline__ bool box_coords(const Box &b, int64_t l, int &x,
                                            int &y, int &z) {
+  // (a grid has fewer than 2^31 voxels: 32-bit divisions)
   if (l >= (int64_t)b.nxr * b.nyr * b.nzr) return false;
-  int t = (int)(l / b.nxr);
-  x = b.x0 + (int)(l - (int64_t)t * b.nxr);
-  z = t / b.nyr;
-  y = b.y0 + (t - z * b.nyr);
-  z += b.z0;
+  const unsigned v = (unsigned)l, nx = (unsigned)b.nxr, ny = (unsigned)b.nyr;
+  const unsigned t = v / nx, w = t / ny;
+  x = b.x0 + (int)(v - t * nx);
+  y = b.y0 + (int)(t - w * ny);
+  z = b.z0 + (int)w;
   return true;
 }
 
@@ -264,12 +265,54 @@ __device__ __forceinline__ void fold_jf_at(vpic_field_t *f, const FaceGeom &G,
   }
 }
 
-__global__ void k_fold_jf(vpic_field_t *f, FaceGeom G, int X) {
-  const int Y = (X + 1) % 3, Z = (X + 2) % 3;
-  const int wy = G.n[Y] + 1, wz = G.n[Z] + 1;
-  for (int l = blockIdx.x * blockDim.x + threadIdx.x; l < wy * wz;
-       l += gridDim.x * blockDim.x)
-    fold_jf_at(f, G, X, l);
+// The periodic jf folds of all axes in one launch (three took 15 us of a step
+// of a 32^3 box, this one 5).  Component C (blockIdx.y) is folded along the
+// two other axes, P before Q in the reference's order x, y, z: on a face its
+// two copies become their sum, on an edge where both axes fold its four
+// copies the sum along P of each pair and then the sum of the two.  One
+// thread reads and writes all copies of an element, so no other thread sees
+// half a fold.  Sums of two are the same in either order, so the result is
+// the three launches' bit for bit.  fold: bit k, axis k is periodic.
+__global__ __launch_bounds__(256) void k_fold_jf(vpic_field_t *f, FaceGeom G,
+                                                 int fold) {
+  const int C = blockIdx.y;
+  const int P = C == 0 ? 1 : 0, Q = C == 2 ? 1 : 2;
+  const bool fp = (fold >> P) & 1, fq = (fold >> Q) & 1;
+  const int nP = G.n[P], nQ = G.n[Q], nC = G.n[C];
+  const int hp = nP * G.s[P], hq = nQ * G.s[Q];  // to the other copy
+  // elements along C (1..nC): the P faces (q = 1..nQ+1, of which q = nQ+1
+  // belongs to q = 1 where Q folds too), then the Q faces off the P faces
+  const int mp = fp ? (fq ? nQ : nQ + 1) : 0;
+  const int mq = fq ? (fp ? nP - 1 : nP + 1) : 0;
+  const int64_t total = (int64_t)nC * (mp + mq);
+  for (int64_t l = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; l < total;
+       l += (int64_t)gridDim.x * blockDim.x) {
+    const int m = (int)(l / nC), c = 1 + (int)(l - (int64_t)m * nC);
+    int v = c * G.s[C];
+    if (m < mp) {
+      v += G.s[P] + (1 + m) * G.s[Q];
+      float &a = fcomp(f, v, 3, C), &b = fcomp(f, v + hp, 3, C);
+      const float s = a + b;
+      if (fq && m == 0) {
+        float &d = fcomp(f, v + hq, 3, C), &e = fcomp(f, v + hp + hq, 3, C);
+        const float t = s + (d + e);
+        a = t;
+        b = t;
+        d = t;
+        e = t;
+      } else {
+        a = s;
+        b = s;
+      }
+    } else {
+      // p = 2..nP where P folds, 1..nP+1 otherwise
+      v += (m - mp + (fp ? 2 : 1)) * G.s[P] + G.s[Q];
+      float &a = fcomp(f, v, 3, C), &b = fcomp(f, v + hq, 3, C);
+      const float s = a + b;
+      a = s;
+      b = s;
+    }
+  }
 }
 
 // local_adjust_rhof + local_adjust_rhob (local.cc:376-440) on one local face:
@@ -405,8 +448,17 @@ __device__ __forceinline__ void ghost_tang_b_at(vpic_field_t *f,
   }
 }
 
-__global__ void k_ghost_tang_b(vpic_field_t *f, FaceGeom G, int X, int mlo,
-                               int mhi) {
+// Boundary codes of the six faces, by value.
+struct FaceModes {
+  int m[6];
+};
+
+// All three axes in one launch (blockIdx.y): an axis reads and writes the two
+// components along its faces on its own planes 0, 1, n and n + 1, up to plane
+// n of the other component's axis, so no axis reads what another writes.
+__global__ void k_ghost_tang_b(vpic_field_t *f, FaceGeom G, FaceModes M) {
+  const int X = blockIdx.y;
+  const int mlo = M.m[X], mhi = M.m[X + 3];
   const int Y = (X + 1) % 3, Z = (X + 2) % 3;
   const int wy = G.n[Y] + 1, wz = G.n[Z] + 1;
   for (int l = blockIdx.x * blockDim.x + threadIdx.x; l < wy * wz;
@@ -544,8 +596,10 @@ __global__ __launch_bounds__(256) void k_fold_partials(const double *part,
 // plane with rw = 1, lw = 0 (remote.cc:137-207); local faces copy
 // (anti-symmetric) or negate (symmetric, pmc) e and tca of the adjacent
 // plane (local.cc:129-179).
-__global__ void k_ghost_norm_e(vpic_field_t *f, FaceGeom G, int X, int mlo,
-                               int mhi) {
+// All axes in one launch (blockIdx.y): axis X touches only component X.
+__global__ void k_ghost_norm_e(vpic_field_t *f, FaceGeom G, FaceModes M) {
+  const int X = blockIdx.y;
+  const int mlo = M.m[X], mhi = M.m[X + 3];
   const int Y = (X + 1) % 3, Z = (X + 2) % 3;
   const int nX = G.n[X];
   const int wy = G.n[Y] + 1, wz = G.n[Z] + 1;
@@ -583,8 +637,11 @@ __global__ void k_ghost_norm_e(vpic_field_t *f, FaceGeom G, int X, int mlo,
 // div_b_err ghosts of axis X (cell planes 0 and nX+1, Y in 1..nY, Z in
 // 1..nZ): periodic as above (remote.cc:209-281); local faces copy (anti-
 // symmetric) or negate (symmetric, pmc) (local.cc:182-221).
-__global__ void k_ghost_div_b(vpic_field_t *f, FaceGeom G, int X, int mlo,
-                              int mhi) {
+// All axes in one launch (blockIdx.y): the ghosts of one axis lie off the
+// cells that another reads.
+__global__ void k_ghost_div_b(vpic_field_t *f, FaceGeom G, FaceModes M) {
+  const int X = blockIdx.y;
+  const int mlo = M.m[X], mhi = M.m[X + 3];
   const int Y = (X + 1) % 3, Z = (X + 2) % 3;
   const int nX = G.n[X];
   const int wy = G.n[Y], wz = G.n[Z];
@@ -805,6 +862,12 @@ FaceGeom face_geom(const vpic_grid_t *g) {
   G.s[1] = g->sy;
   G.s[2] = g->sz;
   return G;
+}
+
+FaceModes face_codes(const vpic_grid_t *g) {
+  FaceModes M;
+  for (int k = 0; k < 6; k++) M.m[k] = g->fbc[k];
+  return M;
 }
 
 int face_blocks(const vpic_grid_t *g) {
@@ -1062,9 +1125,11 @@ int launch_synchronize_jf(vpic_field_t *f, const vpic_grid_t *g,
     hipLaunchKernelGGL(k_adjust_jf, dim3(fb), dim3(256), 0, s, f, G, k, mode);
     VPIC_LAUNCHED("k_adjust_jf");
   }
-  for (int X = 0; X < 3; X++) {
-    if (g->fbc[X] != VPIC_BC_PERIODIC) continue;
-    hipLaunchKernelGGL(k_fold_jf, dim3(fb), dim3(256), 0, s, f, G, X);
+  int fold = 0;
+  for (int X = 0; X < 3; X++)
+    if (g->fbc[X] == VPIC_BC_PERIODIC) fold |= 1 << X;
+  if (fold) {
+    hipLaunchKernelGGL(k_fold_jf, dim3(fb, 3), dim3(256), 0, s, f, G, fold);
     VPIC_LAUNCHED("k_fold_jf");
   }
   return VPIC_OK;
@@ -1116,11 +1181,9 @@ int launch_vacuum_advance_e(vpic_field_t *f, const vpic_grid_t *g,
                             const vpic_field_params_t *m, hipStream_t s) {
   FaceGeom G = face_geom(g);
   const int fb = face_blocks(g);
-  for (int X = 0; X < 3; X++) {
-    hipLaunchKernelGGL(k_ghost_tang_b, dim3(fb), dim3(256), 0, s, f, G, X,
-                       g->fbc[X], g->fbc[X + 3]);
-    VPIC_LAUNCHED("k_ghost_tang_b");
-  }
+  hipLaunchKernelGGL(k_ghost_tang_b, dim3(fb, 3), dim3(256), 0, s, f, G,
+                     face_codes(g));
+  VPIC_LAUNCHED("k_ghost_tang_b");
   // vacuum_advance_e_pipeline.h:23-33, in float.
   const ECoef c = make_ecoef(g, m);
   Box b = {1, 1, 1, g->nx + 1, g->ny + 1, g->nz + 1};
@@ -1233,11 +1296,9 @@ int launch_compute_div_e_err(vpic_field_t *f, const vpic_grid_t *g,
                              hipStream_t s) {
   const FaceGeom G = face_geom(g);
   const int fb = face_blocks(g);
-  for (int X = 0; X < 3; X++) {
-    hipLaunchKernelGGL(k_ghost_norm_e, dim3(fb), dim3(256), 0, s, f, G, X,
-                       g->fbc[X], g->fbc[X + 3]);
-    VPIC_LAUNCHED("k_ghost_norm_e");
-  }
+  hipLaunchKernelGGL(k_ghost_norm_e, dim3(fb, 3), dim3(256), 0, s, f, G,
+                     face_codes(g));
+  VPIC_LAUNCHED("k_ghost_norm_e");
   const int nx = g->nx, ny = g->ny, nz = g->nz;
   const Box b = node_box(g);
   const int nblk = blocks_for(node_count(g), 256);
@@ -1334,11 +1395,9 @@ int launch_clean_div_b(vpic_field_t *f, const vpic_grid_t *g, hipStream_t s) {
   pz *= alphadt;
   const FaceGeom G = face_geom(g);
   const int fb = face_blocks(g);
-  for (int X = 0; X < 3; X++) {
-    hipLaunchKernelGGL(k_ghost_div_b, dim3(fb), dim3(256), 0, s, f, G, X,
-                       g->fbc[X], g->fbc[X + 3]);
-    VPIC_LAUNCHED("k_ghost_div_b");
-  }
+  hipLaunchKernelGGL(k_ghost_div_b, dim3(fb, 3), dim3(256), 0, s, f, G,
+                     face_codes(g));
+  VPIC_LAUNCHED("k_ghost_div_b");
   hipLaunchKernelGGL(k_clean_div_b, dim3(blocks_for(node_count(g), 256)),
                      dim3(256), 0, s, f, node_box(g), g->nx, g->ny, g->nz, px,
                      py, pz);
@@ -1350,11 +1409,9 @@ int launch_compute_curl_b(vpic_field_t *f, const vpic_grid_t *g,
                           const vpic_field_params_t *m, hipStream_t s) {
   const FaceGeom G = face_geom(g);
   const int fb = face_blocks(g);
-  for (int X = 0; X < 3; X++) {
-    hipLaunchKernelGGL(k_ghost_tang_b, dim3(fb), dim3(256), 0, s, f, G, X,
-                       g->fbc[X], g->fbc[X + 3]);
-    VPIC_LAUNCHED("k_ghost_tang_b");
-  }
+  hipLaunchKernelGGL(k_ghost_tang_b, dim3(fb, 3), dim3(256), 0, s, f, G,
+                     face_codes(g));
+  VPIC_LAUNCHED("k_ghost_tang_b");
   // vacuum_compute_curl_b_pipeline.h:22-27
   ECoef c = {};
   c.px_muz = ((g->nx > 1) ? g->cvac * g->dt * g->rdx : 0) * m->rmuz;
