@@ -268,7 +268,9 @@ int vpic_hip_advance_p_noalloc(vpic_particle_t *p, int32_t np, float q,
                                const vpic_grid_t *g, void *stream);
 
 /* Tile shape (cells) of the partition-driven push; its LDS window holds
- * (tx+2)(ty+2)(tz+2) accumulators (a halo of one cell).  Default 7x8x7.
+ * (tx+2)(ty+2)(tz+2) accumulators (a halo of one cell).  Until this or
+ * vpic_hip_push_tile_window is called, 7x8x7 on large grids and a shape
+ * chosen from the grid's size and particles on others.
  * No reference counterpart (the reference's pipelines split particles,
  * not cells). */
 int vpic_hip_push_tile(int32_t tx, int32_t ty, int32_t tz);
@@ -284,7 +286,7 @@ int vpic_hip_push_tile(int32_t tx, int32_t ty, int32_t tz);
 int vpic_hip_push_tile_window(int32_t tx, int32_t ty, int32_t tz,
                               int32_t halo);
 
-/* The tile shape and halo in use: out[0..3] = tx, ty, tz, halo.  No
+/* The tile shape and halo set, or 7, 8, 7, 1: out[0..3] = tx, ty, tz, halo.  No
  * reference counterpart. */
 int vpic_hip_push_get_tile(int32_t *out);
 

@@ -35,6 +35,8 @@
 // Both end with k_order_movers: movers the grid cannot handle, sorted by
 // particle index, truncated at max_nm (excess rolled back to the voxel
 // index, advance_p_pipeline.cc:228-236).
+#include <string.h>
+
 #include <mutex>
 #include <vector>
 
@@ -887,21 +889,25 @@ __global__ __launch_bounds__(256) void k_ens_push(
 }
 
 // --------------------------------------------------------------------------
-// Flat kernel: particles [n0, np), any order, grid-stride over whole
+// Flat push: particles [n0, np), any order, grid-stride over whole
 // wavefronts.  n0 = *start clamped to [0,np] (the end of the sort-time
 // partition when the tiled kernel ran first), or 0 when start is NULL.
+// Crossers go to xlist for k_move_p_list; the rare excess over xcap (every
+// crosser when xcap is 0) is moved right here.
 // --------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_advance_p(
+__device__ __forceinline__ void flat_push(
     vpic_particle_t *__restrict__ p, const int *__restrict__ start, int np,
     const vpic_interpolator_t *__restrict__ f0, float *__restrict__ acc,
     vpic_particle_mover_t *__restrict__ xlist, int xcap,
-    vpic_particle_mover_t *__restrict__ rlist, int *__restrict__ cnt,
-    PushCoef C, GridDev G, int *__restrict__ vkeys) {
+    vpic_particle_mover_t *__restrict__ rlist, int rcap,
+    int *__restrict__ cnt, const PushCoef &C, const GridDev &G,
+    int *__restrict__ vkeys) {
   const int n0 = start ? min(max(*start, 0), np) : 0;
   const int lane = lane_id();
   const GlobalSink sink{acc};
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   int64_t nn = n0 + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (nn - lane >= np) return;
   float4 A, B;
   load_particle(p, (int)nn, nn < np, A, B);
   for (; nn - lane < np; nn += stride) {
@@ -916,13 +922,15 @@ __global__ __launch_bounds__(256) void k_advance_p(
     if (vkeys && valid && !R.cross) vkeys[n] = __float_as_int(A.w);
 
     // Cell crossers: compact into the crosser list (ballot + one atomic per
-    // wavefront); the rare overflow of the list is moved right here.
+    // wavefront)
     const uint64_t cm = __ballot(R.cross);
     if (cm) {
       const int leader = __ffsll((unsigned long long)cm) - 1;
       int base = 0;
-      if (lane == leader) base = atomicAdd(cnt, __popcll(cm));
-      base = __shfl(base, leader);
+      if (xcap > 0) {
+        if (lane == leader) base = atomicAdd(cnt, __popcll(cm));
+        base = __shfl(base, leader);
+      }
       if (R.cross) {
         const int slot = base + __popcll(cm & ((1ull << lane) - 1ull));
         vpic_particle_mover_t mv;
@@ -934,13 +942,23 @@ __global__ __launch_bounds__(256) void k_advance_p(
           xlist[slot] = mv;
         } else if (dev_move_p(p, mv, sink, G, C.qsp,
                               vkeys ? vkeys + n : nullptr)) {
-          push_returned_mover(p, mv, rlist, xcap, cnt);
+          push_returned_mover(p, mv, rlist, rcap, cnt);
         }
       }
     }
     A = An;
     B = Bn;
   }
+}
+
+__global__ __launch_bounds__(256) void k_advance_p(
+    vpic_particle_t *__restrict__ p, int np,
+    const vpic_interpolator_t *__restrict__ f0, float *__restrict__ acc,
+    vpic_particle_mover_t *__restrict__ xlist, int xcap,
+    vpic_particle_mover_t *__restrict__ rlist, int *__restrict__ cnt,
+    PushCoef C, GridDev G, int *__restrict__ vkeys) {
+  flat_push(p, nullptr, np, f0, acc, xlist, xcap, rlist, xcap, cnt, C, G,
+            vkeys);
 }
 
 __global__ __launch_bounds__(256) void k_move_p_list(
@@ -1018,6 +1036,17 @@ constexpr int TILE_MAXSP = 2;
 struct TileSpeciesSet {
   TileSpecies s[TILE_MAXSP];
 };
+
+// The particles past each species' partition (added since its sort), after
+// the tiled push: one launch for all species (blockIdx.y), crossers moved in
+// place, since there are few or none.
+__global__ __launch_bounds__(256) void k_advance_tail(
+    TileSpeciesSet SS, const vpic_interpolator_t *__restrict__ f0,
+    float *__restrict__ acc, GridDev G) {
+  const TileSpecies &S = SS.s[blockIdx.y];
+  flat_push(S.p, S.part + G.nv, S.np, f0, acc, nullptr, 0, S.rlist, S.rcap,
+            S.cnt, S.C, G, S.vkeys);
+}
 
 constexpr int TILE_BS = VPIC_TILE_BS;     // threads per workgroup
 constexpr int TILE_WAVES = TILE_BS / 64;
@@ -1146,6 +1175,94 @@ __device__ __forceinline__ void drain_wave_queue(
       BS.key[n] = (unsigned char)o;
       atomicAdd(BS.cnt + o, 1);
     }
+  }
+}
+
+// Start of a tiled push: clears the species' counters and, when there are more
+// tiles than CUs, orders the tiles by their particles, the fullest first (in
+// 16 classes of half a power of two each, in the grid's order within a class),
+// so that a dense region neither starts last nor falls on the few XCDs that
+// its columns of tiles are dealt to.  A tile's particles are estimated from
+// three of its rows.
+constexpr int ORDER_CLASSES = 16;
+constexpr int ORDER_MAX = 32768;  // tiles; more keep the grid's order
+
+__global__ __launch_bounds__(1024) void k_push_begin(
+    TileSpeciesSet SS, int nsp, GridDev G, TileGeom T, int *__restrict__ est,
+    int *__restrict__ order) {
+  __shared__ int top, count[ORDER_CLASSES], cursor[ORDER_CLASSES];
+  const int t = threadIdx.x, lane = lane_id();
+  for (int k = 0; k < nsp; k++)
+    if (t < 4) SS.s[k].cnt[t] = 0;
+  if (!order) return;
+  const int ntiles = T.ntx * T.nty * T.ntz;
+  if (t == 0) top = 1;
+  if (t < ORDER_CLASSES) count[t] = 0;
+  __syncthreads();
+  int mine = 0;
+  for (int b = t; b < ntiles; b += 1024) {
+    const int bx = b % T.ntx, by = (b / T.ntx) % T.nty, bz = b / (T.ntx * T.nty);
+    const int x0 = 1 + bx * T.tx, y0 = 1 + by * T.ty, z0 = 1 + bz * T.tz;
+    const int x1 = min(x0 + T.tx - 1, G.nx), y1 = min(y0 + T.ty - 1, G.ny),
+              z1 = min(z0 + T.tz - 1, G.nz);
+    const int ym = (y0 + y1) >> 1, zm = (z0 + z1) >> 1;
+    int64_t n = 0;
+    for (int k = 0; k < nsp; k++) {
+      const int *part = SS.s[k].part;
+      n += part[vox(x1 + 1, y0, z0, G.nx, G.ny)] -
+           part[vox(x0, y0, z0, G.nx, G.ny)];
+      n += part[vox(x1 + 1, ym, zm, G.nx, G.ny)] -
+           part[vox(x0, ym, zm, G.nx, G.ny)];
+      n += part[vox(x1 + 1, y1, z1, G.nx, G.ny)] -
+           part[vox(x0, y1, z1, G.nx, G.ny)];
+    }
+    n = n * ((y1 - y0 + 1) * (z1 - z0 + 1)) / 3;
+    const int e = (int)(n < 1 ? 1 : n > 0x3fffffff ? 0x3fffffff : n);
+    est[b] = e;
+    mine = max(mine, e);
+  }
+  atomicMax(&top, mine);
+  __syncthreads();
+  const float l0 = log2f((float)top);
+  auto cls = [&](int b) {
+    const int c = (int)(2.0f * (l0 - log2f((float)est[b])));
+    return min(max(c, 0), ORDER_CLASSES - 1);
+  };
+  // slots of a class for the lanes of a wavefront that hold one of its tiles
+  auto take = [&](int *where, int c, bool on) {
+    int at = 0;
+    uint64_t todo = __ballot(on);
+    while (todo) {
+      const int leader = __ffsll((unsigned long long)todo) - 1;
+      const int cl = __shfl(c, leader);
+      const uint64_t same = __ballot(on && c == cl) & todo;
+      int base = 0;
+      if (lane == leader) base = atomicAdd(where + cl, __popcll(same));
+      base = __shfl(base, leader);
+      if (on && c == cl) at = base + lanes_below(same);
+      todo &= ~same;
+    }
+    return at;
+  };
+  const int rounds = (ntiles + 1023) / 1024;
+  for (int r = 0; r < rounds; r++) {
+    const int b = r * 1024 + t;
+    take(count, b < ntiles ? cls(b) : 0, b < ntiles);
+  }
+  __syncthreads();
+  if (t == 0) {
+    int at = 0;
+    for (int c = 0; c < ORDER_CLASSES; c++) {
+      cursor[c] = at;
+      at += count[c];
+    }
+  }
+  __syncthreads();
+  for (int r = 0; r < rounds; r++) {
+    const int b = r * 1024 + t;
+    const int at = take(cursor, b < ntiles ? cls(b) : 0, b < ntiles);
+    if (b < ntiles) order[at] = b;
+    __syncthreads();  // classes keep the grid's order round by round
   }
 }
 
@@ -1663,9 +1780,10 @@ __global__ __launch_bounds__(TILE_BS, TILE_MIN_WAVES) void k_advance_p_tiled(
     TileSpeciesSet SS, const vpic_interpolator_t *__restrict__ f0,
     float *__restrict__ acc, float *__restrict__ wbuf, int wstride,
     vpic_particle_t *__restrict__ trash, GridDev G, TileGeom T, BinArgs Bn,
-    OowBuckets OB) {
-  tiled_push<GS, MODE, NSP>(blockIdx.x, SS.s, f0, acc, wbuf, wstride, trash,
-                            G, T, Bn, OB);
+    OowBuckets OB, const int *__restrict__ order) {
+  const int tile = order ? order[blockIdx.x] : (int)blockIdx.x;
+  tiled_push<GS, MODE, NSP>(__builtin_amdgcn_readfirstlane(tile), SS.s, f0,
+                            acc, wbuf, wstride, trash, G, T, Bn, OB);
 }
 
 // Add the tiles' windows into the accumulator: voxel v receives the
@@ -1698,51 +1816,55 @@ __device__ __forceinline__ void merge_tile(int tile, float *__restrict__ acc,
   const int t = threadIdx.x;
   // the sub-buckets addressed to this tile: code d of source tile
   // (this tile - offset(d)), periodic in the tile indices
-  __shared__ int sb_n[27];
+  __shared__ int sb_n[27];       // records, then their running total
   __shared__ int64_t sb_at[27];
-  __shared__ float sb_max[27];
+  __shared__ unsigned sb_max;    // largest magnitude (bits)
   __shared__ int sb_total;
-  if (t < 27) {
+  if (t == 0) sb_max = 0u;
+  __syncthreads();
+  if (t < 64) {
     int n = 0;
-    int64_t at = 0;
-    float mx = 0.0f;
-    if (OB.cap > 0) {
+    if (t < 27 && OB.cap > 0) {
       const int ox = t % 3 - 1, oy = (t / 3) % 3 - 1, oz = t / 9 - 1;
       const int sx = (bx - ox + T.ntx) % T.ntx, sy = (by - oy + T.nty) % T.nty,
                 sz = (bz - oz + T.ntz) % T.ntz;
       const int src = sx + T.ntx * (sy + T.nty * sz);
-      at = (int64_t)(27 * src + t) * OB.cap;
       n = min(OB.cnt[2 * (27 * src + t)], OB.cap);
-      mx = __uint_as_float((unsigned)OB.cnt[2 * (27 * src + t) + 1]);
+      sb_at[t] = (int64_t)(27 * src + t) * OB.cap;
+      // (magnitudes are not negative, so their bits order as they do)
+      if (n > 0) atomicMax(&sb_max, (unsigned)OB.cnt[2 * (27 * src + t) + 1]);
     }
-    sb_n[t] = n;
-    sb_at[t] = at;
-    sb_max[t] = n > 0 ? mx : 0.0f;
-  }
-  __syncthreads();
-  if (t == 0) {
-    int tot = 0;
-    for (int d = 0; d < 27; d++) tot += sb_n[d];
-    sb_total = tot;
+    int incl = n;
+#pragma unroll
+    for (int d = 1; d < 32; d <<= 1) {
+      const int o = __shfl_up(incl, d);
+      if (t >= d) incl += o;
+    }
+    if (t < 27) sb_n[t] = incl;
+    if (t == 26) sb_total = incl;
   }
   __syncthreads();
   const int nrec = sb_total;
-  (void)tile;
   double bscale = 0.0;
   if (nrec > 0) {
     // every component of every record is at most the largest magnitude
     // the pushing tiles recorded
-    float m = 0.0f;
-    for (int d = 0; d < 27; d++) m = fmaxf(m, sb_max[d]);
+    const float m = __uint_as_float(sb_max);
     for (int k = t; k < 12 * ncell; k += blockDim.x) bsum[k] = 0ull;
     __syncthreads();
     int ex = 0;
     const double bound = (double)m * (double)nrec;
     if (bound > 0.0) frexp(bound, &ex);  // every sum is below 2^ex
     bscale = ldexp(1.0, 50 - ex);
-    for (int d = 0; d < 27; d++) {
-      const float4 *rec = OB.rec + 4 * sb_at[d];
-      for (int r = t; r < sb_n[d]; r += blockDim.x) {
+    // the records of all sub-buckets back to back, so that every lane has
+    // one (a loop over the sub-buckets waits for memory 27 times, 13 us
+    // with a record or two in each)
+    int d = 0;
+    for (int k = t; k < nrec; k += blockDim.x) {
+      while (d < 26 && k >= sb_n[d]) d++;
+      {
+        const int r = k - (d > 0 ? sb_n[d - 1] : 0);
+        const float4 *rec = OB.rec + 4 * sb_at[d];
         const float4 a = rec[4 * r], c = rec[4 * r + 1], e = rec[4 * r + 2],
                      f = rec[4 * r + 3];
         const int v = __float_as_int(a.x);
@@ -1756,9 +1878,9 @@ __device__ __forceinline__ void merge_tile(int tile, float *__restrict__ acc,
         const float jv[12] = {a.y, a.z, a.w, c.x, c.y, c.z,
                               c.w, e.x, e.y, e.z, e.w, f.x};
 #pragma unroll
-        for (int k = 0; k < 12; k++)
-          atomicAdd(&bsum[k * ncell + cell],
-                    (unsigned long long)to_fixed((double)jv[k] * bscale));
+        for (int k2 = 0; k2 < 12; k2++)
+          atomicAdd(&bsum[k2 * ncell + cell],
+                    (unsigned long long)to_fixed((double)jv[k2] * bscale));
       }
     }
     __syncthreads();
@@ -2042,10 +2164,29 @@ __global__ __launch_bounds__(256) void k_bin_scatter(
 // (index, slot) pairs in global memory by one workgroup), keep the first
 // max_nm and roll the rest back.  dev_nm[0] = nm, dev_nm[1] = n_ignored,
 // dev_nm[2] = particles skipped for an out-of-range voxel index.
-__global__ __launch_bounds__(1024) void k_order_movers(
-    vpic_particle_t *__restrict__ p, const vpic_particle_mover_t *rlist,
-    int rcap, int2 *__restrict__ buf, vpic_particle_mover_t *__restrict__ pm,
-    int max_nm, const int *__restrict__ cnt, int *__restrict__ dev_nm) {
+// One workgroup per species.
+struct MoverOut {
+  vpic_particle_t *p;
+  const vpic_particle_mover_t *rlist;
+  int rcap, max_nm;
+  int2 *buf;
+  vpic_particle_mover_t *pm;
+  const int *cnt;
+  int *dev_nm;
+};
+struct MoverOutSet {
+  MoverOut s[TILE_MAXSP];
+};
+
+__global__ __launch_bounds__(1024) void k_order_movers(MoverOutSet MS) {
+  const MoverOut &M = MS.s[blockIdx.x];
+  vpic_particle_t *__restrict__ p = M.p;
+  const vpic_particle_mover_t *rlist = M.rlist;
+  int2 *__restrict__ buf = M.buf;
+  vpic_particle_mover_t *__restrict__ pm = M.pm;
+  const int rcap = M.rcap, max_nm = M.max_nm;
+  const int *__restrict__ cnt = M.cnt;
+  int *__restrict__ dev_nm = M.dev_nm;
   const int n = min(cnt[1], rcap);
   const int lost = cnt[2];
   const int t = threadIdx.x, T = blockDim.x;
@@ -2167,7 +2308,7 @@ struct PushScratch {
   // their ordering buffer
   DeviceScratch counters[TILE_MAXSP], xlist[TILE_MAXSP], rlist[TILE_MAXSP],
       sortbuf[TILE_MAXSP];
-  DeviceScratch wbuf, trash, inject;
+  DeviceScratch wbuf, trash, inject, order;
   DeviceScratch ocnt, orec;  // out-of-window buckets (OowBuckets)
   BinState bins[8];
   int64_t bin_clock = 0;
@@ -2191,6 +2332,7 @@ int pow2_at_least(int64_t n) {
 // sort intervals (8x8x8, whose coefficients fit for the tile only, took 6%
 // longer per push)
 TileGeom g_tile = {7, 8, 7, 0, 0, 0, 0, 0, 0, 1, 1, 1, 1};
+bool g_tile_set = false;  // the caller chose g_tile
 int g_group = 16;  // lanes sharing one run of particles in the tiled push
 int g_bin_mode = 0;  // tile lists: 0 off, 1 when drift warrants, 2 always
 
@@ -2211,7 +2353,7 @@ BinState &bin_state(PushScratch &S, const void *p) {
 
 typedef void (*TiledKernel)(TileSpeciesSet, const vpic_interpolator_t *,
                             float *, float *, int, vpic_particle_t *, GridDev,
-                            TileGeom, BinArgs, OowBuckets);
+                            TileGeom, BinArgs, OowBuckets, const int *);
 
 int tiled_kernel_id(int gs) {
   int id = 0;
@@ -2282,12 +2424,102 @@ bool tile_fits(int tx, int ty, int tz, int h) {
   return 96 * w + 72 * (size_t)tx * ty * tz <= (size_t)TILE_DYN_BYTES;
 }
 
+constexpr int PUSH_CUS = 256;  // compute units of the chip
+
+// Estimated microseconds of a tiled push of grid g with ppc particles per
+// cell (all species) in tiles of tx x ty x tz: a tile costs 27 us (its
+// staging, barriers and drains), 5 ns per window cell (written, then read by
+// the merge) and per particle 4.2 ns, more by 0.55 of the surface cells' share
+// (deposits outside the tile; measured 5.0 ns for 7x8x7, 5.6 for 8x8x4, 6.0
+// for 8x4x4, 6.6 for 32x2x2 at 32^3 cells, 128 per cell), one tile at a time
+// on each CU, whole tiles in whole rounds.  Between particle walls a plasma
+// is not uniform: there a tile of four times the mean density has to fit into
+// the push as well (a current sheet of 512x257 cells, 2 x 48 per cell: 709 us
+// in tiles of 32x16, 540 in tiles of 10x10).
+double tile_cost(const vpic_grid_t *g, double ppc, int tx, int ty, int tz) {
+  const int n[3] = {g->nx, g->ny, g->nz}, t[3] = {tx, ty, tz};
+  double full = 1, all = 1, cells = 1, wcells = 1, surface = 0;
+  for (int k = 0; k < 3; k++) {
+    full *= n[k] / t[k];
+    all *= (n[k] + t[k] - 1) / t[k];
+    cells *= t[k];
+    wcells *= t[k] + (n[k] > 1 ? 2 : 0);
+    surface += n[k] > 1 ? 1.0 / t[k] : 0.0;
+  }
+  const double per = 4.2e-3 * (1 + 0.55 * surface);
+  const double one = 27 + 5e-3 * wcells + cells * ppc * per;
+  const double total = all * (27 + 5e-3 * wcells) +
+                       (double)g->nx * g->ny * g->nz * ppc * per;
+  double rounds = full / PUSH_CUS;
+  rounds = rounds > (int)rounds ? (int)rounds + 1 : rounds;
+  if (rounds < 1) rounds = 1;
+  bool walls = false;
+  for (int k = 0; k < 6; k++) walls |= g->pbc[k] != VPIC_BC_PERIODIC;
+  double bound = rounds * one;
+  const double mean = total / PUSH_CUS, dense = 27 + 4 * (one - 27);
+  if (walls && dense > bound) bound = dense;
+  return bound > mean ? bound : mean;
+}
+
+// The tile of a push: the caller's, else 7x8x7 (the best of the shapes timed
+// on large grids) unless the cost above finds one 5% cheaper: on grids of
+// few tiles, where 7x8x7 leaves CUs without one (32^3 cells: 100 tiles, 277
+// us a push of 2 x 64 per cell; 8x4x4 gives every CU one, 126 us; 12x10x9
+// cells, 2 x 8 per cell: 68 to 26 us), and on 2D grids, where 7x1x7 is too
+// small to amortise a tile's fixed cost.
+TileGeom push_tile_for(const vpic_grid_t *g, int64_t np) {
+  if (g_tile_set) return g_tile;
+  const double ppc = (double)np / ((double)g->nx * g->ny * g->nz);
+  struct Choice {
+    int nx = 0, ny = 0, nz = 0, pbc[6] = {0};
+    int64_t np = 0;
+    TileGeom T;
+  };
+  // (the last answer: a run asks for the same sizes at every step)
+  static thread_local Choice last;
+  if (last.nx == g->nx && last.ny == g->ny && last.nz == g->nz &&
+      last.np == np && memcmp(last.pbc, g->pbc, sizeof last.pbc) == 0)
+    return last.T;
+  TileGeom T = g_tile;
+  const int mx = g->nx < 32 ? g->nx : 32, my = g->ny < 16 ? g->ny : 16,
+            mz = g->nz < 16 ? g->nz : 16;
+  double best = 0.95 * tile_cost(g, ppc, T.tx < g->nx ? T.tx : g->nx,
+                                 T.ty < g->ny ? T.ty : g->ny,
+                                 T.tz < g->nz ? T.tz : g->nz);
+  // (at least two cells along an axis that has them)
+  for (int tz = mz < 2 ? mz : 2; tz <= mz; tz++)
+    for (int ty = my < 2 ? my : 2; ty <= my; ty++)
+      for (int tx = mx < 2 ? mx : 2; tx <= mx; tx++) {
+        if (tx * ty * tz > TILE_MAXCELLS || ty * tz > TILE_MAXROWS) continue;
+        // the coefficients of the whole window staged beside it
+        const size_t w = (size_t)(tx + (g->nx > 1 ? 2 : 0)) *
+                         (ty + (g->ny > 1 ? 2 : 0)) *
+                         (tz + (g->nz > 1 ? 2 : 0));
+        if ((96 + 72) * w > (size_t)TILE_DYN_BYTES) continue;
+        const double c = tile_cost(g, ppc, tx, ty, tz);
+        if (c < best) {
+          best = c;
+          T.tx = tx;
+          T.ty = ty;
+          T.tz = tz;
+        }
+      }
+  last.nx = g->nx;
+  last.ny = g->ny;
+  last.nz = g->nz;
+  last.np = np;
+  memcpy(last.pbc, g->pbc, sizeof last.pbc);
+  last.T = T;
+  return T;
+}
+
 }  // namespace
 
 // Tile shape and window halo of the tiled push (the window of a tile is
 // (tx+2h)(ty+2h)(tz+2h) cells of 96 B in LDS).
 int push_set_tile(int tx, int ty, int tz, int halo) {
   if (!tile_fits(tx, ty, tz, halo)) return VPIC_EINVAL;
+  g_tile_set = true;
   g_tile.tx = tx;
   g_tile.ty = ty;
   g_tile.tz = tz;
@@ -2363,25 +2595,26 @@ int launch_flat_push(vpic_particle_t *p, int np, float q, const PushCoef &C,
                      const vpic_interpolator_t *f, int *cnt,
                      vpic_particle_mover_t *xlist,
                      vpic_particle_mover_t *rlist, int2 *sortbuf, int xcap,
-                     hipStream_t s) {
+                     int *keys, bool timed, hipStream_t s) {
   hipLaunchKernelGGL(k_clear_counters, dim3(1), dim3(64), 0, s, cnt);
   VPIC_LAUNCHED("k_clear_counters");
   if (np > 0) {
     int64_t want = ((int64_t)np + 255) / 256;
     const int blocks = (int)(want < 16384 ? want : 16384);
-    hipLaunchKernelGGL(k_advance_p, dim3(blocks), dim3(256), 0, s, p,
-                       (const int *)nullptr, np, f, (float *)a, xlist, xcap,
-                       rlist, cnt, C, G, (int *)nullptr);
+    if (timed) push_timing_record(s, np, true);
+    hipLaunchKernelGGL(k_advance_p, dim3(blocks), dim3(256), 0, s, p, np, f,
+                       (float *)a, xlist, xcap, rlist, cnt, C, G, keys);
     VPIC_LAUNCHED("k_advance_p");
+    if (timed) push_timing_record(s, np, false);
     int mblocks = (xcap + 255) / 256;
     if (mblocks > 8192) mblocks = 8192;
     hipLaunchKernelGGL(k_move_p_list, dim3(mblocks), dim3(256), 0, s, p,
-                       xlist, xcap, rlist, (float *)a, cnt, q, G,
-                       (int *)nullptr);
+                       xlist, xcap, rlist, (float *)a, cnt, q, G, keys);
     VPIC_LAUNCHED("k_move_p_list");
   }
-  hipLaunchKernelGGL(k_order_movers, dim3(1), dim3(1024), 0, s, p, rlist,
-                     xcap, sortbuf, pm, max_nm, cnt, dev_nm);
+  MoverOutSet MS = {};
+  MS.s[0] = {p, rlist, xcap, max_nm, sortbuf, pm, cnt, dev_nm};
+  hipLaunchKernelGGL(k_order_movers, dim3(1), dim3(1024), 0, s, MS);
   VPIC_LAUNCHED("k_order_movers");
   return VPIC_OK;
 }
@@ -2452,7 +2685,7 @@ int launch_advance_p_noalloc(vpic_particle_t *p, int np, float q, float m,
   push_invalidate_bins(p);
   return launch_flat_push(p, np, q, push_coef(q, m, g), make_grid_dev(g), pm,
                           max_nm, dev_nm, a, f, cnt, xlist, rlist, sortbuf,
-                          xcap, s);
+                          xcap, nullptr, false, s);
 }
 
 int launch_advance_p(vpic_particle_t *p, int np, float q, float m,
@@ -2509,8 +2742,6 @@ int launch_advance_p_set(int nsp, const vpic_push_species_t *sp,
     rlist[k] = (vpic_particle_mover_t *)S.rlist[k].ptr;
     C[k] = push_coef(sp[k].q, sp[k].m, g);
     np_total += sp[k].np;
-    hipLaunchKernelGGL(k_clear_counters, dim3(1), dim3(64), 0, s, cnt[k]);
-    VPIC_LAUNCHED("k_clear_counters");
     // a flat push moves particles without recording their tiles
     if (!sp[k].partition) push_invalidate_bins(sp[k].p);
   }
@@ -2518,13 +2749,17 @@ int launch_advance_p_set(int nsp, const vpic_push_species_t *sp,
   // the timing brackets the main push kernel only: k_advance_p_tiled when
   // a partition is given, else k_advance_p
   const bool timed = push_timing_on();
-  const int *flat_start[TILE_MAXSP] = {};
-  if (sp[0].partition && np_total > 0) {
-    // (one species here, or several that all have partitions)
+  if (!sp[0].partition || np_total == 0)
+    // (one species: several in one launch all have partitions)
+    return launch_flat_push(sp[0].p, sp[0].np, sp[0].q, C[0], G, sp[0].pm,
+                            sp[0].max_nm, sp[0].dev_nm, a, f, cnt[0],
+                            xlist[0], rlist[0], (int2 *)S.sortbuf[0].ptr,
+                            xcap[0], sp[0].keys, timed, s);
+  {
     vpic_particle_t *p = sp[0].p;
     const int np = sp[0].np;
     const int *partition = sp[0].partition;
-    TileGeom T = g_tile;
+    TileGeom T = push_tile_for(g, np_total);
     // a tile no larger than the grid (a 2D grid's tiles are one cell
     // thick; the window then has no halo along that axis either)
     T.tx = T.tx < g->nx ? T.tx : g->nx;
@@ -2652,18 +2887,30 @@ int launch_advance_p_set(int nsp, const vpic_push_species_t *sp,
       BA.oow = ctl + 4;
       BSt = &B;
     }
-    if (timed) push_timing_record(s, np_total, true);
-    // without binning only the mode-0 instance; with it all three, of
-    // which the one matching the device's binning state runs
     TileSpeciesSet SS = {};
     for (int k = 0; k < nsp; k++)
       SS.s[k] = {sp[k].p, sp[k].partition, rlist[k], cnt[k], sp[k].keys,
                  C[k], sp[k].np, xcap[k]};
+    // fullest tiles first, where some CU gets more than one
+    int *order = nullptr, *est = nullptr;
+    if (nblk > PUSH_CUS && nblk <= ORDER_MAX) {
+      if ((rc = scratch_reserve(S.order, sizeof(int) * 2 * (size_t)nblk)))
+        return rc;
+      est = (int *)S.order.ptr;
+      order = est + nblk;
+    }
+    hipLaunchKernelGGL(k_push_begin, dim3(1), dim3(1024), 0, s, SS, nsp, G, T,
+                       est, order);
+    VPIC_LAUNCHED("k_push_begin");
+    if (timed) push_timing_record(s, np_total, true);
+    // without binning only the mode-0 instance; with it all three, of
+    // which the one matching the device's binning state runs
     for (int mode = 0; mode < (BSt ? 3 : 1); mode++) {
       hipLaunchKernelGGL(tiled_kernel(g_group, mode, nsp), dim3(nblk),
                          dim3(TILE_BS), lds, s, SS, f, (float *)a,
                          (float *)S.wbuf.ptr, wstride,
-                         (vpic_particle_t *)S.trash.ptr, G, T, BA, OB);
+                         (vpic_particle_t *)S.trash.ptr, G, T, BA, OB,
+                         (const int *)order);
       VPIC_LAUNCHED("k_advance_p_tiled");
     }
     if (timed) push_timing_record(s, np_total, false);
@@ -2678,32 +2925,19 @@ int launch_advance_p_set(int nsp, const vpic_push_species_t *sp,
                        OB);
     VPIC_LAUNCHED("k_merge_windows");
     // particles past the partition (added since the sort) go flat
-    for (int k = 0; k < nsp; k++) flat_start[k] = sp[k].partition + g->nv;
+    int most = 0;
+    for (int k = 0; k < nsp; k++) most = most < sp[k].np ? sp[k].np : most;
+    int64_t want = ((int64_t)most + 255) / 256;
+    hipLaunchKernelGGL(k_advance_tail, dim3(want < 1024 ? want : 1024, nsp),
+                       dim3(256), 0, s, SS, f, (float *)a, G);
+    VPIC_LAUNCHED("k_advance_tail");
   }
-  for (int k = 0; k < nsp; k++) {
-    const int np = sp[k].np;
-    if (np > 0) {
-      int64_t want = ((int64_t)np + 255) / 256;
-      const int blocks = (int)(want < 16384 ? want : 16384);
-      const bool flat_timed = timed && !sp[k].partition;
-      if (flat_timed) push_timing_record(s, np, true);
-      hipLaunchKernelGGL(k_advance_p, dim3(blocks), dim3(256), 0, s, sp[k].p,
-                         flat_start[k], np, f, (float *)a, xlist[k], xcap[k],
-                         rlist[k], cnt[k], C[k], G, sp[k].keys);
-      VPIC_LAUNCHED("k_advance_p");
-      if (flat_timed) push_timing_record(s, np, false);
-      int mblocks = (xcap[k] + 255) / 256;
-      if (mblocks > 8192) mblocks = 8192;
-      hipLaunchKernelGGL(k_move_p_list, dim3(mblocks), dim3(256), 0, s,
-                         sp[k].p, xlist[k], xcap[k], rlist[k], (float *)a,
-                         cnt[k], sp[k].q, G, sp[k].keys);
-      VPIC_LAUNCHED("k_move_p_list");
-    }
-    hipLaunchKernelGGL(k_order_movers, dim3(1), dim3(1024), 0, s, sp[k].p,
-                       rlist[k], xcap[k], (int2 *)S.sortbuf[k].ptr, sp[k].pm,
-                       sp[k].max_nm, cnt[k], sp[k].dev_nm);
-    VPIC_LAUNCHED("k_order_movers");
-  }
+  MoverOutSet MS = {};
+  for (int k = 0; k < nsp; k++)
+    MS.s[k] = {sp[k].p, rlist[k], xcap[k], sp[k].max_nm,
+               (int2 *)S.sortbuf[k].ptr, sp[k].pm, cnt[k], sp[k].dev_nm};
+  hipLaunchKernelGGL(k_order_movers, dim3(nsp), dim3(1024), 0, s, MS);
+  VPIC_LAUNCHED("k_order_movers");
   return VPIC_OK;
 }
 
