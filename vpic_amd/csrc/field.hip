@@ -287,9 +287,21 @@ __global__ __launch_bounds__(256) void k_fold_jf(vpic_field_t *f, FaceGeom G,
   const int64_t total = (int64_t)nC * (mp + mq);
   for (int64_t l = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; l < total;
        l += (int64_t)gridDim.x * blockDim.x) {
-    const int m = (int)(l / nC), c = 1 + (int)(l - (int64_t)m * nC);
+    // the lower axis of a face fastest, so that lanes go along x (or y)
+    const bool on_p = l < (int64_t)nC * mp;
+    const int64_t r = on_p ? l : l - (int64_t)nC * mp;
+    const int other = on_p ? Q : P, mo = on_p ? mp : mq;
+    int m, c;
+    if (C < other) {
+      m = (int)(r / nC);
+      c = 1 + (int)(r - (int64_t)m * nC);
+    } else {
+      c = (int)(r / mo);
+      m = (int)(r - (int64_t)c * mo);
+      c++;
+    }
     int v = c * G.s[C];
-    if (m < mp) {
+    if (on_p) {
       v += G.s[P] + (1 + m) * G.s[Q];
       float &a = fcomp(f, v, 3, C), &b = fcomp(f, v + hp, 3, C);
       const float s = a + b;
@@ -306,7 +318,7 @@ __global__ __launch_bounds__(256) void k_fold_jf(vpic_field_t *f, FaceGeom G,
       }
     } else {
       // p = 2..nP where P folds, 1..nP+1 otherwise
-      v += (m - mp + (fp ? 2 : 1)) * G.s[P] + G.s[Q];
+      v += (m + (fp ? 2 : 1)) * G.s[P] + G.s[Q];
       float &a = fcomp(f, v, 3, C), &b = fcomp(f, v + hq, 3, C);
       const float s = a + b;
       a = s;
@@ -416,10 +428,12 @@ __device__ __forceinline__ void ghost_tang_b_at(vpic_field_t *f,
                                                 int mlo, int mhi, int l) {
   const int Y = (X + 1) % 3, Z = (X + 2) % 3;
   const int nX = G.n[X];
-  const int wy = G.n[Y] + 1;
+  const int wy = G.n[Y] + 1, wz = G.n[Z] + 1;
   const float rw = 1.0f, lw = 0.0f;
   {
-    const int yy = 1 + l % wy, zz = 1 + l / wy;
+    // lanes along x where the face has it (Z is x on the y faces)
+    const int yy = 1 + (X == 1 ? l / wz : l % wy),
+              zz = 1 + (X == 1 ? l % wz : l / wy);
     const int g0 = face_vox(G, X, 0, yy, zz);
     const int g1 = face_vox(G, X, nX + 1, yy, zz);
     const int i1 = face_vox(G, X, 1, yy, zz);

@@ -1185,13 +1185,14 @@ __device__ __forceinline__ void drain_wave_queue(
 // its columns of tiles are dealt to.  A tile's particles are estimated from
 // three of its rows.
 constexpr int ORDER_CLASSES = 16;
-constexpr int ORDER_MAX = 32768;  // tiles; more keep the grid's order
+constexpr int ORDER_MAX = 8192;  // tiles; more keep the grid's order
 
 __global__ __launch_bounds__(1024) void k_push_begin(
-    TileSpeciesSet SS, int nsp, GridDev G, TileGeom T, int *__restrict__ est,
+    TileSpeciesSet SS, int nsp, GridDev G, TileGeom T,
     int *__restrict__ order) {
+  __shared__ int est[ORDER_MAX];
   __shared__ int top, count[ORDER_CLASSES], cursor[ORDER_CLASSES];
-  const int t = threadIdx.x, lane = lane_id();
+  const int t = threadIdx.x;
   for (int k = 0; k < nsp; k++)
     if (t < 4) SS.s[k].cnt[t] = 0;
   if (!order) return;
@@ -1228,27 +1229,7 @@ __global__ __launch_bounds__(1024) void k_push_begin(
     const int c = (int)(2.0f * (l0 - log2f((float)est[b])));
     return min(max(c, 0), ORDER_CLASSES - 1);
   };
-  // slots of a class for the lanes of a wavefront that hold one of its tiles
-  auto take = [&](int *where, int c, bool on) {
-    int at = 0;
-    uint64_t todo = __ballot(on);
-    while (todo) {
-      const int leader = __ffsll((unsigned long long)todo) - 1;
-      const int cl = __shfl(c, leader);
-      const uint64_t same = __ballot(on && c == cl) & todo;
-      int base = 0;
-      if (lane == leader) base = atomicAdd(where + cl, __popcll(same));
-      base = __shfl(base, leader);
-      if (on && c == cl) at = base + lanes_below(same);
-      todo &= ~same;
-    }
-    return at;
-  };
-  const int rounds = (ntiles + 1023) / 1024;
-  for (int r = 0; r < rounds; r++) {
-    const int b = r * 1024 + t;
-    take(count, b < ntiles ? cls(b) : 0, b < ntiles);
-  }
+  for (int b = t; b < ntiles; b += 1024) atomicAdd(&count[cls(b)], 1);
   __syncthreads();
   if (t == 0) {
     int at = 0;
@@ -1258,11 +1239,11 @@ __global__ __launch_bounds__(1024) void k_push_begin(
     }
   }
   __syncthreads();
-  for (int r = 0; r < rounds; r++) {
+  // (1024 tiles at a time, so that a class roughly keeps the grid's order)
+  for (int r = 0; r * 1024 < ntiles; r++) {
     const int b = r * 1024 + t;
-    const int at = take(cursor, b < ntiles ? cls(b) : 0, b < ntiles);
-    if (b < ntiles) order[at] = b;
-    __syncthreads();  // classes keep the grid's order round by round
+    if (b < ntiles) order[atomicAdd(&cursor[cls(b)], 1)] = b;
+    __syncthreads();
   }
 }
 
@@ -2892,15 +2873,14 @@ int launch_advance_p_set(int nsp, const vpic_push_species_t *sp,
       SS.s[k] = {sp[k].p, sp[k].partition, rlist[k], cnt[k], sp[k].keys,
                  C[k], sp[k].np, xcap[k]};
     // fullest tiles first, where some CU gets more than one
-    int *order = nullptr, *est = nullptr;
+    int *order = nullptr;
     if (nblk > PUSH_CUS && nblk <= ORDER_MAX) {
-      if ((rc = scratch_reserve(S.order, sizeof(int) * 2 * (size_t)nblk)))
+      if ((rc = scratch_reserve(S.order, sizeof(int) * (size_t)nblk)))
         return rc;
-      est = (int *)S.order.ptr;
-      order = est + nblk;
+      order = (int *)S.order.ptr;
     }
     hipLaunchKernelGGL(k_push_begin, dim3(1), dim3(1024), 0, s, SS, nsp, G, T,
-                       est, order);
+                       order);
     VPIC_LAUNCHED("k_push_begin");
     if (timed) push_timing_record(s, np_total, true);
     // without binning only the mode-0 instance; with it all three, of

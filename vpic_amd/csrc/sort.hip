@@ -286,9 +286,13 @@ __global__ __launch_bounds__(256) void k_gather(
 constexpr int RS_MAXB = 2048;  // digit values per pass (LDS counters)
 // Elements per block (one wavefront).  A block is a serial chain of 64
 // elements at a time (0.55 us each), so a sort of few particles takes blocks
-// short enough for 16 wavefronts on every CU; many particles keep long ones,
-// which write fewer (digit, block) counts.
+// short enough for 16 wavefronts on every CU, as long as the (digit, block)
+// counts they write stay below RS_COUNTS; many particles keep long ones, which
+// write fewer counts.  (Blocks kept to twice the digit's values took 49 us a
+// scatter for 8640 particles of 12x10x9 cells, 16 us now, and 52 us for
+// 2.1e6 of 32^3, 36 us now.)
 constexpr int RS_BLK_MIN = 512, RS_BLK_MAX = 16384, RS_WAVES = 4096;
+constexpr int64_t RS_COUNTS = 4 << 20;
 
 // digit = (voxel / div) % mod: the coordinates along one or more axes
 struct SortDig {
@@ -546,9 +550,8 @@ struct SortPass {
 // The passes of grid g for np particles, x first: an axis joins the digit of
 // the one before it while together they have at most RS_MAXB values (two
 // passes fewer on a 12x10x9 box, one on a 32^3 box and on 2D grids), and the
-// blocks halve from RS_BLK_MAX until there are RS_WAVES of them, but keep
-// twice the digit's values (a shorter block would write more counts than it
-// has elements).
+// blocks halve from RS_BLK_MAX until there are RS_WAVES of them or RS_COUNTS
+// counts.
 int sort_passes(const vpic_grid_t *g, int np, SortPass out[3]) {
   const unsigned ax[3] = {(unsigned)(g->nx + 2), (unsigned)(g->ny + 2),
                           (unsigned)(g->nz + 2)};
@@ -564,7 +567,7 @@ int sort_passes(const vpic_grid_t *g, int np, SortPass out[3]) {
     P.nbins = (int)mod;
     P.blk = RS_BLK_MAX;
     while (P.blk > RS_BLK_MIN && np / P.blk < RS_WAVES &&
-           P.blk / 2 >= 2 * P.nbins)
+           (int64_t)P.nbins * blocks_for(np, P.blk / 2) <= RS_COUNTS)
       P.blk /= 2;
     P.nblocks = blocks_for(np, P.blk);
     div *= mod;
