@@ -289,3 +289,59 @@ def test_faces_in_one_launch(dev, orc, n, wall):
     got = df.download()
     for c in T.FIELD_FLOATS:
         assert H.same_bits(got[c], f[c]), c
+
+
+# batches of voxels in the collision operator: 64 voxels at most (sparse, most
+# voxels with 0 or 1 particle), batches that end inside a neighbourhood, and
+# voxels that just fill a batch of 1792 particles or exceed it; partners many,
+# few and none
+@pytest.mark.parametrize("n,lo,hi,crowd", [
+    ((70, 2, 2), 0, 2, ()), ((13, 5, 4), 20, 90, ()),
+    ((4, 3, 3), 0, 9, (1791, 1792, 1793, 4100)), ((2, 1, 1), 1792, 1792, ()),
+    ((3, 2, 1), 700, 1500, ())],
+    ids=["sparse", "ordinary", "crowded", "full", "large"])
+def test_collision_batches(dev, orc, n, lo, hi, crowd):
+    """Bit for bit the oracle's voxel after voxel, within a species and
+    between two in both orders of their sizes."""
+    g = T.grid_periodic(0, 0, 0, *n, *n, 0.2)
+    rng = np.random.default_rng(17)
+    v = np.arange(g.nv)
+    x, y, z = v % (g.nx + 2), v // (g.nx + 2) % (g.ny + 2), v // (
+        (g.nx + 2) * (g.ny + 2))
+    inner = np.nonzero((x >= 1) & (x <= g.nx) & (y >= 1) & (y <= g.ny) &
+                       (z >= 1) & (z <= g.nz))[0]
+
+    def species(lo, hi, crowd, w):
+        c = np.zeros(g.nv, np.int64)
+        c[inner] = rng.integers(lo, hi + 1, len(inner))
+        c[inner[1:1 + len(crowd)]] = crowd
+        p = np.zeros(int(c.sum()), T.PARTICLE)
+        p["i"] = np.repeat(np.arange(g.nv, dtype=np.int32), c)
+        for k in ("dx", "dy", "dz"):
+            p[k] = rng.uniform(-1, 1, len(p)).astype(np.float32)
+        for k in ("ux", "uy", "uz"):
+            p[k] = (0.1 * rng.standard_normal(len(p))).astype(np.float32)
+        p["w"] = rng.choice(np.array(w, np.float32), len(p))
+        part = np.zeros(g.nv + 1, np.int32)
+        part[1:] = np.cumsum(c)
+        return p, part
+
+    pe, parte = species(lo, hi, crowd, [1.0])
+    pi, parti = species(0, 7, crowd[:2], [1.0, 2.5])
+    de, dpe = dev.DeviceArray.from_host(pe), dev.DeviceArray.from_host(parte)
+    di, dpi = dev.DeviceArray.from_host(pi), dev.DeviceArray.from_host(parti)
+    E = (pe, parte, de, dpe, -1.0, 1.0)
+    I = (pi, parti, di, dpi, 1.0, 25.0)
+    # a draw that the shuffle rejects, so that the words behind it move up:
+    # the 693rd of voxel 18 (1792 particles where each voxel has as many)
+    word = int(orc.philox4x32((693 // 4, 18, 5469, 0), (1234, 0))[693 % 4])
+    assert word // ((2**32 - 1) // (1792 - 693)) >= 1792 - 693
+    for call, a, b in [(0, E, E), (1, E, I), (2, I, E), (5469, E, E)]:
+        say("collide", n, call)
+        orc.takizuka_abe(a[0], a[1], a[4], a[5], b[0], b[1], b[4], b[5], 0.5,
+                         2, 1234, call, g)
+        _lib.call("vpic_hip_takizuka_abe", a[2].ptr, a[3].ptr, len(a[0]),
+                  a[4], a[5], b[2].ptr, b[3].ptr, len(b[0]), b[4], b[5], 0.5,
+                  2, 1234, call, ctypes.byref(g), None)
+        assert H.same_bits(de.download(), pe), call
+        assert H.same_bits(di.download(), pi), call
