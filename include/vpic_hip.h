@@ -513,6 +513,19 @@ int vpic_hip_vacuum_advance_e(vpic_field_t *f, const vpic_grid_t *g,
                               const vpic_field_params_t *mp, float frac,
                               void *stream);
 
+/* The field part of a step (advance.cc:107-141): clear_jf,
+ * unload_accumulator_array, synchronize_jf, advance_b(1/2), vacuum_advance_e,
+ * advance_b(1/2) and load_interpolator_array, with the separate calls' results
+ * bit for bit.  `work`: 16 bytes of device memory per voxel of the grid
+ * (g->nv), 16-byte aligned, which the caller keeps until the work queued on
+ * `stream` is done; its contents do not matter before or after.  With it a grid
+ * whose six faces are periodic takes four launches.  NULL, or any other grid:
+ * the separate calls. */
+int vpic_hip_field_step(vpic_field_t *f, const vpic_accumulator_t *a,
+                        vpic_interpolator_t *fi, void *work,
+                        const vpic_grid_t *g, const vpic_field_params_t *mp,
+                        void *stream);
+
 /* energy_f: six FP64 field energies {ex,ey,ez,bx,by,bz}
  * (vacuum_energy_f_pipeline.h:17-75; vacuum_energy_f_pipeline.cc:13-97).
  * Synchronous. */

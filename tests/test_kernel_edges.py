@@ -345,3 +345,44 @@ def test_collision_batches(dev, orc, n, lo, hi, crowd):
                   2, 1234, call, ctypes.byref(g), None)
         assert H.same_bits(de.download(), pe), call
         assert H.same_bits(di.download(), pi), call
+
+
+# the field part of a step in four launches, where axes have one or two cells
+# (ghosts and faces are neighbours), rows past a workgroup, and with walls
+# (the separate calls) or without a work array
+@pytest.mark.parametrize("wall,work", [(None, True), (None, False),
+                                       (1, True)])
+@pytest.mark.parametrize("n", [(1, 1, 1), (1, 5, 3), (2, 2, 2), (4, 1, 1),
+                               (3, 2, 70), (300, 2, 3), (17, 16, 15)],
+                         ids=lambda v: "x".join(map(str, v)))
+def test_field_step(dev, n, wall, work):
+    """Bit for bit the separate calls, ghosts and interpolators included, from
+    any content of the work array, twice in a row."""
+    g = T.grid_periodic(0, 0, 0, *n, *n, 0.4)
+    if wall is not None:
+        g.fbc[wall] = g.fbc[wall + 3] = T.BC_PEC_FIELDS
+    f = H.random_full_fields(g, 9)
+    rng = np.random.default_rng(2)
+    acc = rng.standard_normal((g.nv, 12)).astype(np.float32)
+    mp = T.vacuum_params(damp=0.02)
+    G, M = ctypes.byref(g), ctypes.byref(mp)
+    da = dev.DeviceArray.from_host(acc)
+    a, b = (dev.DeviceArray.from_host(f) for _ in range(2))
+    ia, ib = dev.interpolators(g), dev.interpolators(g)
+    ia.zero()
+    ib.zero()
+    w = dev.DeviceArray.from_host(
+        np.full((g.nv, 4), np.nan, np.float32)) if work else None
+    say("field step", n, wall, work)
+    for _ in range(2):
+        _lib.call("vpic_hip_clear_jf_unload_accumulator_array", a.ptr, da.ptr,
+                  G, None)
+        _lib.call("vpic_hip_synchronize_jf", a.ptr, G, None)
+        _lib.call("vpic_hip_advance_b", a.ptr, G, 0.5, None)
+        _lib.call("vpic_hip_vacuum_advance_e", a.ptr, G, M, 1.0, None)
+        _lib.call("vpic_hip_advance_b", a.ptr, G, 0.5, None)
+        _lib.call("vpic_hip_load_interpolator_array", ia.ptr, a.ptr, G, None)
+        _lib.call("vpic_hip_field_step", b.ptr, da.ptr, ib.ptr,
+                  w.ptr if work else None, G, M, None)
+        assert H.same_bits(b.download(), a.download())
+        assert H.same_bits(ib.download(), ia.download())

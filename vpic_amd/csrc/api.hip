@@ -599,6 +599,19 @@ extern "C" int vpic_hip_vacuum_advance_e(vpic_field_t *f, const vpic_grid_t *g,
   return launch_vacuum_advance_e(f, g, mp, S(stream));
 }
 
+extern "C" int vpic_hip_field_step(vpic_field_t *f,
+                                   const vpic_accumulator_t *a,
+                                   vpic_interpolator_t *fi, void *work,
+                                   const vpic_grid_t *g,
+                                   const vpic_field_params_t *mp,
+                                   void *stream) {
+  int rc = check_grid(g);
+  if (rc || (rc = check_fields_supported(g))) return rc;
+  CHECK(f && a && fi && mp && aligned16(f) && aligned16(work),
+        "bad argument");
+  return launch_field_step(f, a, fi, work, g, mp, S(stream));
+}
+
 extern "C" int vpic_hip_energy_f(double host_en[6], const vpic_field_t *f,
                                  const vpic_grid_t *g,
                                  const vpic_field_params_t *mp, void *stream) {

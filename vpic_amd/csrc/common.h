@@ -384,6 +384,10 @@ int launch_synchronize_rho(vpic_field_t *f, const vpic_grid_t *g,
                            hipStream_t s);
 int launch_advance_b(vpic_field_t *f, const vpic_grid_t *g, float frac,
                      hipStream_t s);
+int launch_field_step(vpic_field_t *f, const vpic_accumulator_t *a,
+                      vpic_interpolator_t *fi, void *work,
+                      const vpic_grid_t *g, const vpic_field_params_t *m,
+                      hipStream_t s);
 int launch_vacuum_advance_e(vpic_field_t *f, const vpic_grid_t *g,
                             const vpic_field_params_t *mp, hipStream_t s);
 int launch_energy_f(double en[6], const vpic_field_t *f, const vpic_grid_t *g,

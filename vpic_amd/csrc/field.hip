@@ -69,19 +69,15 @@ __device__ __forceinline__ const float4 *F4(const vpic_field_t *f, int v) {
 // ---------------------------------------------------------------------------
 // load_interpolator_array
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ void load_interpolator_at(
-    vpic_interpolator_t *__restrict__ fi, const vpic_field_t *__restrict__ f,
-    int x, int y, int z, int nx, int ny) {
+// The coefficients of cell v from E and B of its lower corner (e0, b0), E of
+// the neighbours along x, y, z, ex, ey, ez of those across an edge (yz, zx,
+// xy) and the normal B of the upper faces.
+__device__ __forceinline__ void store_interpolator(
+    vpic_interpolator_t *__restrict__ fi, int v, const float4 &e0,
+    const float4 &ex_, const float4 &ey_, const float4 &ez_, float e_yz,
+    float e_zx, float e_xy, const float4 &b0, float bx1, float by1,
+    float bz1) {
   const float fourth = 0.25f, half = 0.50f;
-  const int v = vox(x, y, z, nx, ny);
-  const int sy = nx + 2, sz = (ny + 2) * sy;
-  const float4 e0 = F4(f, v)[0], b0 = F4(f, v)[1];
-  const float4 ex_ = F4(f, v + 1)[0], bx_ = F4(f, v + 1)[1];
-  const float4 ey_ = F4(f, v + sy)[0], by_ = F4(f, v + sy)[1];
-  const float4 ez_ = F4(f, v + sz)[0], bz_ = F4(f, v + sz)[1];
-  const float e_yz = F4(f, v + sy + sz)[0].x;  // pfyz->ex
-  const float e_zx = F4(f, v + sz + 1)[0].y;   // pfzx->ey
-  const float e_xy = F4(f, v + 1 + sy)[0].z;   // pfxy->ez
   float w0, w1, w2, w3;
   float4 o0, o1, o2, o3;
   w0 = e0.x; w1 = ey_.x; w2 = ez_.x; w3 = e_yz;
@@ -99,13 +95,13 @@ __device__ __forceinline__ void load_interpolator_at(
   o2.y = fourth * ((w3 - w0) + (w1 - w2));
   o2.z = fourth * ((w3 - w0) - (w1 - w2));
   o2.w = fourth * ((w3 + w0) - (w1 + w2));
-  w0 = b0.x; w1 = bx_.x;
+  w0 = b0.x; w1 = bx1;
   o3.x = half * (w1 + w0);
   o3.y = half * (w1 - w0);
-  w0 = b0.y; w1 = by_.y;
+  w0 = b0.y; w1 = by1;
   o3.z = half * (w1 + w0);
   o3.w = half * (w1 - w0);
-  w0 = b0.z; w1 = bz_.z;
+  w0 = b0.z; w1 = bz1;
   float4 *out = reinterpret_cast<float4 *>(fi + v);
   out[0] = o0;
   out[1] = o1;
@@ -113,6 +109,20 @@ __device__ __forceinline__ void load_interpolator_at(
   out[3] = o3;
   reinterpret_cast<float2 *>(out + 4)[0] =
       make_float2(half * (w1 + w0), half * (w1 - w0));
+}
+
+__device__ __forceinline__ void load_interpolator_at(
+    vpic_interpolator_t *__restrict__ fi, const vpic_field_t *__restrict__ f,
+    int x, int y, int z, int nx, int ny) {
+  const int v = vox(x, y, z, nx, ny);
+  const int sy = nx + 2, sz = (ny + 2) * sy;
+  store_interpolator(fi, v, F4(f, v)[0], F4(f, v + 1)[0], F4(f, v + sy)[0],
+                     F4(f, v + sz)[0],
+                     F4(f, v + sy + sz)[0].x,  // pfyz->ex
+                     F4(f, v + sz + 1)[0].y,   // pfzx->ey
+                     F4(f, v + 1 + sy)[0].z,   // pfxy->ez
+                     F4(f, v)[1], F4(f, v + 1)[1].x, F4(f, v + sy)[1].y,
+                     F4(f, v + sz)[1].z);
 }
 
 __global__ __launch_bounds__(256) void k_load_interpolator(
@@ -266,16 +276,15 @@ __device__ __forceinline__ void fold_jf_at(vpic_field_t *f, const FaceGeom &G,
 }
 
 // The periodic jf folds of all axes in one launch (three took 15 us of a step
-// of a 32^3 box, this one 5).  Component C (blockIdx.y) is folded along the
+// of a 32^3 box, this one 5).  Component C is folded along the
 // two other axes, P before Q in the reference's order x, y, z: on a face its
 // two copies become their sum, on an edge where both axes fold its four
 // copies the sum along P of each pair and then the sum of the two.  One
 // thread reads and writes all copies of an element, so no other thread sees
 // half a fold.  Sums of two are the same in either order, so the result is
 // the three launches' bit for bit.  fold: bit k, axis k is periodic.
-__global__ __launch_bounds__(256) void k_fold_jf(vpic_field_t *f, FaceGeom G,
-                                                 int fold) {
-  const int C = blockIdx.y;
+__device__ __forceinline__ void fold_jf(vpic_field_t *f, const FaceGeom &G,
+                                        int fold, int C) {
   const int P = C == 0 ? 1 : 0, Q = C == 2 ? 1 : 2;
   const bool fp = (fold >> P) & 1, fq = (fold >> Q) & 1;
   const int nP = G.n[P], nQ = G.n[Q], nC = G.n[C];
@@ -327,6 +336,11 @@ __global__ __launch_bounds__(256) void k_fold_jf(vpic_field_t *f, FaceGeom G,
   }
 }
 
+__global__ __launch_bounds__(256) void k_fold_jf(vpic_field_t *f, FaceGeom G,
+                                                 int fold) {
+  fold_jf(f, G, fold, blockIdx.y);
+}
+
 // local_adjust_rhof + local_adjust_rhob (local.cc:376-440) on one local face:
 // mode 1 (anti-symmetric) zeroes rhof and rhob, mode 2 doubles rhof.
 __global__ void k_adjust_rho(vpic_field_t *f, FaceGeom G, int k, int mode) {
@@ -369,25 +383,40 @@ __global__ void k_fold_rho(vpic_field_t *f, FaceGeom G, int X) {
 // ---------------------------------------------------------------------------
 // advance_b
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ void advance_b_at(vpic_field_t *__restrict__ f,
-                                             int x, int y, int z, int nx,
-                                             int ny, int nz, float px,
-                                             float py, float pz) {
-  const int v = vox(x, y, z, nx, ny);
+// b0 advanced at voxel (x, y, z) of 1..n+1, whose E is e0: cbx on x in 1..nx+1
+// (y<=ny, z<=nz), cby on y in 1..ny+1, cbz on z in 1..nz+1; each neighbour is
+// read only where its component is updated.  False: nothing to update.
+__device__ __forceinline__ bool advance_b_val(const vpic_field_t *f, int v,
+                                              int x, int y, int z, int nx,
+                                              int ny, int nz, float px,
+                                              float py, float pz,
+                                              const float4 &e0, float4 &ex1,
+                                              float4 &ey1, float4 &ez1,
+                                              float4 &b0) {
   const int sy = nx + 2, sz = (ny + 2) * sy;
-  const float4 e0 = F4(f, v)[0];
-  float4 b0 = F4(f, v)[1];
   const bool ux = x <= nx, uy = y <= ny, uz = z <= nz;
-  // cbx on x in 1..nx+1 (y<=ny, z<=nz), cby on y in 1..ny+1, cbz on z in
-  // 1..nz+1; each neighbour is read only where its component is updated.
-  float4 ex1 = e0, ey1 = e0, ez1 = e0;
+  ex1 = e0;
+  ey1 = e0;
+  ez1 = e0;
   if (ux && (uy || uz)) ex1 = F4(f, v + 1)[0];
   if (uy && (ux || uz)) ey1 = F4(f, v + sy)[0];
   if (uz && (ux || uy)) ez1 = F4(f, v + sz)[0];
   if (uy && uz) b0.x -= (py * (ey1.z - e0.z) - pz * (ez1.y - e0.y));
   if (ux && uz) b0.y -= (pz * (ez1.x - e0.x) - px * (ex1.z - e0.z));
   if (ux && uy) b0.z -= (px * (ex1.y - e0.y) - py * (ey1.x - e0.x));
-  if ((uy && uz) || (ux && uz) || (ux && uy)) F4(f, v)[1] = b0;
+  return (uy && uz) || (ux && uz) || (ux && uy);
+}
+
+__device__ __forceinline__ void advance_b_at(vpic_field_t *__restrict__ f,
+                                             int x, int y, int z, int nx,
+                                             int ny, int nz, float px,
+                                             float py, float pz) {
+  const int v = vox(x, y, z, nx, ny);
+  const float4 e0 = F4(f, v)[0];
+  float4 b0 = F4(f, v)[1], ex1, ey1, ez1;
+  if (advance_b_val(f, v, x, y, z, nx, ny, nz, px, py, pz, e0, ex1, ey1, ez1,
+                    b0))
+    F4(f, v)[1] = b0;
 }
 
 __global__ __launch_bounds__(256) void k_advance_b(vpic_field_t *__restrict__ f,
@@ -423,7 +452,9 @@ __global__ void k_adjust_norm_b(vpic_field_t *f, FaceGeom G, int4 m0,
 // take the opposite interior face with rw = 1, lw = 0 (remote.cc:105-116 for
 // equal cell sizes); local faces copy (anti-symmetric) or negate
 // (symmetric/pmc) the first interior plane (local.cc:67-81).
-__device__ __forceinline__ void ghost_tang_b_at(vpic_field_t *f,
+// b(v, axis): the component of B; low(v, axis, value): stores a low ghost.
+template <class B, class Low>
+__device__ __forceinline__ void ghost_tang_b_of(B b, Low low,
                                                 const FaceGeom &G, int X,
                                                 int mlo, int mhi, int l) {
   const int Y = (X + 1) % 3, Z = (X + 2) % 3;
@@ -443,23 +474,32 @@ __device__ __forceinline__ void ghost_tang_b_at(vpic_field_t *f,
       const int comp = c == 0 ? Y : Z;
       // cb_Y on (Y in 1..nY+1, Z in 1..nZ), cb_Z on (Y in 1..nY, Z in 1..nZ+1)
       if (c == 0 ? (zz > G.n[Z]) : (yy > G.n[Y])) continue;
-      const float a1 = fcomp(f, i1, 1, comp), aN = fcomp(f, iN, 1, comp);
+      const float a1 = b(i1, comp), aN = b(iN, comp);
       // low ghost (plane 0)
       if (mlo == VPIC_BC_PERIODIC)
-        fcomp(f, g0, 1, comp) = rw * aN + lw * a1;
+        low(g0, comp, rw * aN + lw * a1);
       else if (mlo == VPIC_BC_ANTI_SYMMETRIC_FIELDS)
-        fcomp(f, g0, 1, comp) = a1;
+        low(g0, comp, a1);
       else
-        fcomp(f, g0, 1, comp) = -a1;
+        low(g0, comp, -a1);
       // high ghost (plane nX+1)
       if (mhi == VPIC_BC_PERIODIC)
-        fcomp(f, g1, 1, comp) = rw * a1 + lw * aN;
+        b(g1, comp) = rw * a1 + lw * aN;
       else if (mhi == VPIC_BC_ANTI_SYMMETRIC_FIELDS)
-        fcomp(f, g1, 1, comp) = aN;
+        b(g1, comp) = aN;
       else
-        fcomp(f, g1, 1, comp) = -aN;
+        b(g1, comp) = -aN;
     }
   }
+}
+
+__device__ __forceinline__ void ghost_tang_b_at(vpic_field_t *f,
+                                                const FaceGeom &G, int X,
+                                                int mlo, int mhi, int l) {
+  ghost_tang_b_of(
+      [&](int v, int axis) -> float & { return fcomp(f, v, 1, axis); },
+      [&](int v, int axis, float x) { fcomp(f, v, 1, axis) = x; }, G, X, mlo,
+      mhi, l);
 }
 
 // Boundary codes of the six faces, by value.
@@ -481,17 +521,18 @@ __global__ void k_ghost_tang_b(vpic_field_t *f, FaceGeom G, FaceModes M) {
 }
 
 
-__device__ __forceinline__ void advance_e_at(vpic_field_t *__restrict__ f,
+// b(v): B of voxel v.
+template <class B>
+__device__ __forceinline__ void advance_e_of(B b, vpic_field_t *__restrict__ f,
                                              int x, int y, int z, int nx,
                                              int ny, int nz, const ECoef &c) {
   const int v = vox(x, y, z, nx, ny);
   const int sy = nx + 2, sz = (ny + 2) * sy;
   float4 e0 = F4(f, v)[0];
-  const float4 b0 = F4(f, v)[1];
+  const float4 b0 = b(v);
   float4 t0 = F4(f, v)[2];
   const float4 j0 = F4(f, v)[3];
-  const float4 bx = F4(f, v - 1)[1], by = F4(f, v - sy)[1],
-               bz = F4(f, v - sz)[1];
+  const float4 bx = b(v - 1), by = b(v - sy), bz = b(v - sz);
   if (x <= nx) {
     t0.x = (c.py_muz * (b0.z - by.z) - c.pz_muy * (b0.y - bz.y)) -
            c.damp * t0.x;
@@ -511,12 +552,112 @@ __device__ __forceinline__ void advance_e_at(vpic_field_t *__restrict__ f,
   F4(f, v)[2] = t0;
 }
 
+__device__ __forceinline__ void advance_e_at(vpic_field_t *__restrict__ f,
+                                             int x, int y, int z, int nx,
+                                             int ny, int nz, const ECoef &c) {
+  advance_e_of([&](int v) { return F4(f, v)[1]; }, f, x, y, z, nx, ny, nz, c);
+}
+
 __global__ __launch_bounds__(256) void k_advance_e(vpic_field_t *__restrict__ f,
                                                    Box b, int nx, int ny,
                                                    int nz, ECoef c) {
   int x, y, z;
   if (!box_coords(b, xcd_index(), x, y, z)) return;
   advance_e_at(f, x, y, z, nx, ny, nz, c);
+}
+
+// ---------------------------------------------------------------------------
+// The field part of a step of a periodic box in four launches: unload_
+// accumulator with clear_jf, synchronize_jf, advance_b(1/2), vacuum_advance_e,
+// advance_b(1/2), load_interpolator_array.
+//
+// Bound by memory: one call after the other passes over the 80-B records five
+// times and over B three times.  Here the half-step B goes to an array of its
+// own (`hb`, 16 B a voxel, ghosts included), which takes the place of B in
+// the records between the first and the last kernel: no kernel then reads a
+// neighbour's value that it also advances, so the unload joins the first
+// advance_b and the interpolators join the second (whose values on the cell's
+// upper faces are formed again, from E that the interpolators read anyway).
+// Every value is formed by the same expression as in the separate calls.
+// 257 x 150 x 128 cells: 326 + 20 + 181 + 410 us, 937 in all, against 1131 for
+// the seven launches; 32^3, where a launch is 5 us: 20 us against 34.
+// ---------------------------------------------------------------------------
+__global__ __launch_bounds__(256) void k_unload_half_b(
+    vpic_field_t *__restrict__ f, const vpic_accumulator_t *__restrict__ a,
+    float4 *__restrict__ hb, Box b, int nx, int ny, int nz, float cx, float cy,
+    float cz, float px, float py, float pz) {
+  int x, y, z;
+  if (!box_coords(b, xcd_index(), x, y, z)) return;
+  const int v = vox(x, y, z, nx, ny);
+  const int sy = nx + 2, sz = (ny + 2) * sy;
+  float4 jf = F4(f, v)[3], b0 = F4(f, v)[1];
+  jf.x = 0.0f;
+  jf.y = 0.0f;
+  jf.z = 0.0f;
+  if (x >= 1 && x <= nx + 1 && y >= 1 && y <= ny + 1 && z >= 1 &&
+      z <= nz + 1) {
+    jf = unload_add(jf, a, v, sy, sz, cx, cy, cz);
+    float4 ex1, ey1, ez1;
+    advance_b_val(f, v, x, y, z, nx, ny, nz, px, py, pz, F4(f, v)[0], ex1, ey1,
+                  ez1, b0);
+  }
+  F4(f, v)[3] = jf;
+  hb[v] = b0;
+}
+
+// The jf fold (blockIdx.y 0..2) and the tangential-B ghosts (3..5), the low
+// ones also in the records (the last kernel does not reach them).
+__global__ __launch_bounds__(256) void k_fold_jf_ghost_b(
+    vpic_field_t *f, float4 *hb, FaceGeom G) {
+  if (blockIdx.y < 3) {
+    fold_jf(f, G, 7, blockIdx.y);
+    return;
+  }
+  const int X = blockIdx.y - 3, Y = (X + 1) % 3, Z = (X + 2) % 3;
+  const int wy = G.n[Y] + 1, wz = G.n[Z] + 1;
+  for (int l = blockIdx.x * blockDim.x + threadIdx.x; l < wy * wz;
+       l += gridDim.x * blockDim.x)
+    ghost_tang_b_of(
+        [&](int v, int axis) -> float & {
+          return reinterpret_cast<float *>(hb + v)[axis];
+        },
+        [&](int v, int axis, float x) {
+          reinterpret_cast<float *>(hb + v)[axis] = x;
+          fcomp(f, v, 1, axis) = x;
+        },
+        G, X, VPIC_BC_PERIODIC, VPIC_BC_PERIODIC, l);
+}
+
+__global__ __launch_bounds__(256) void k_advance_e_hb(
+    vpic_field_t *__restrict__ f, const float4 *__restrict__ hb, Box b, int nx,
+    int ny, int nz, ECoef c) {
+  int x, y, z;
+  if (!box_coords(b, xcd_index(), x, y, z)) return;
+  advance_e_of([&](int v) { return hb[v]; }, f, x, y, z, nx, ny, nz, c);
+}
+
+__global__ __launch_bounds__(256) void k_half_b_interpolator(
+    vpic_field_t *__restrict__ f, const float4 *__restrict__ hb,
+    vpic_interpolator_t *__restrict__ fi, Box b, int nx, int ny, int nz,
+    float px, float py, float pz) {
+  int x, y, z;
+  if (!box_coords(b, xcd_index(), x, y, z)) return;
+  const int v = vox(x, y, z, nx, ny);
+  const int sy = nx + 2, sz = (ny + 2) * sy;
+  const float4 e0 = F4(f, v)[0];
+  float4 b0 = hb[v], ex1, ey1, ez1;
+  advance_b_val(f, v, x, y, z, nx, ny, nz, px, py, pz, e0, ex1, ey1, ez1, b0);
+  F4(f, v)[1] = b0;
+  if (x > nx || y > ny || z > nz) return;
+  const float e_yz = F4(f, v + sy + sz)[0].x, e_zx = F4(f, v + sz + 1)[0].y,
+              e_xy = F4(f, v + 1 + sy)[0].z;
+  // cbx at x + 1, cby at y + 1, cbz at z + 1, as advance_b forms them there
+  float bx1 = hb[v + 1].x, by1 = hb[v + sy].y, bz1 = hb[v + sz].z;
+  bx1 -= (py * (e_xy - ex1.z) - pz * (e_zx - ex1.y));
+  by1 -= (pz * (e_yz - ey1.x) - px * (e_xy - ey1.z));
+  bz1 -= (px * (e_zx - ez1.y) - py * (e_yz - ez1.x));
+  store_interpolator(fi, v, e0, ex1, ey1, ez1, e_yz, e_zx, e_xy, b0, bx1, by1,
+                     bz1);
 }
 
 // local_adjust_tang_e (local.cc:224-264): PEC faces zero e and tca tangential.
@@ -1215,6 +1356,50 @@ int launch_vacuum_advance_e(vpic_field_t *f, const vpic_grid_t *g,
                        m1);
     VPIC_LAUNCHED("k_adjust_tang_e");
   }
+  return VPIC_OK;
+}
+
+int launch_field_step(vpic_field_t *f, const vpic_accumulator_t *a,
+                      vpic_interpolator_t *fi, void *work,
+                      const vpic_grid_t *g, const vpic_field_params_t *m,
+                      hipStream_t s) {
+  bool periodic = true;
+  for (int k = 0; k < 6; k++) periodic &= g->fbc[k] == VPIC_BC_PERIODIC;
+  if (!periodic || !work) {
+    // (walls change B and jf between the calls)
+    if (int rc = launch_clear_unload_accumulator(f, a, g, s)) return rc;
+    if (int rc = launch_synchronize_jf(f, g, s)) return rc;
+    if (int rc = launch_advance_b(f, g, 0.5f, s)) return rc;
+    if (int rc = launch_vacuum_advance_e(f, g, m, s)) return rc;
+    if (int rc = launch_advance_b(f, g, 0.5f, s)) return rc;
+    return launch_load_interpolator(fi, f, g, s);
+  }
+  float4 *hb = (float4 *)work;
+  const int nx = g->nx, ny = g->ny, nz = g->nz;
+  // the coefficients of launch_clear_unload_accumulator and launch_advance_b
+  const float cx = 0.25 * g->rdy * g->rdz / g->dt;
+  const float cy = 0.25 * g->rdz * g->rdx / g->dt;
+  const float cz = 0.25 * g->rdx * g->rdy / g->dt;
+  const float frac = 0.5f;
+  const float px = (nx > 1) ? frac * g->cvac * g->dt * g->rdx : 0;
+  const float py = (ny > 1) ? frac * g->cvac * g->dt * g->rdy : 0;
+  const float pz = (nz > 1) ? frac * g->cvac * g->dt * g->rdz : 0;
+  const Box all = {0, 0, 0, nx + 2, ny + 2, nz + 2};
+  const Box b = {1, 1, 1, nx + 1, ny + 1, nz + 1};
+  const int64_t n = (int64_t)(nx + 1) * (ny + 1) * (nz + 1);
+  const dim3 grid(xcd_grid(n, 256)), bs(256);
+  hipLaunchKernelGGL(k_unload_half_b, dim3(xcd_grid(g->nv, 256)), bs, 0, s, f,
+                     a, hb, all, nx, ny, nz, cx, cy, cz, px, py, pz);
+  VPIC_LAUNCHED("k_unload_half_b");
+  hipLaunchKernelGGL(k_fold_jf_ghost_b, dim3(face_blocks(g), 6), bs, 0, s, f,
+                     hb, face_geom(g));
+  VPIC_LAUNCHED("k_fold_jf_ghost_b");
+  hipLaunchKernelGGL(k_advance_e_hb, grid, bs, 0, s, f, (const float4 *)hb, b,
+                     nx, ny, nz, make_ecoef(g, m));
+  VPIC_LAUNCHED("k_advance_e_hb");
+  hipLaunchKernelGGL(k_half_b_interpolator, grid, bs, 0, s, f,
+                     (const float4 *)hb, fi, b, nx, ny, nz, px, py, pz);
+  VPIC_LAUNCHED("k_half_b_interpolator");
   return VPIC_OK;
 }
 

@@ -65,6 +65,7 @@ class Simulation:
         self.interp.zero()
         self.acc = device.accumulators(grid)
         self.acc.zero()
+        self.field_work = None  # field_step's half-step B, on a periodic box
         self.species = []
         self.step = 0
         self.stream = None  # the default stream
@@ -199,6 +200,17 @@ class Simulation:
     def advance_e(self, frac=1.0):
         _lib.call("vpic_hip_vacuum_advance_e", self.fields.ptr, self._G(),
                   ctypes.byref(self.mp), frac, self.stream)
+
+    def field_step(self):
+        """Everything of a step after the push (advance.cc:107-141) in one
+        call: jf, both half advances of B, E and the interpolators."""
+        if self.field_work is None and all(
+                self.g.fbc[k] == T.BC_PERIODIC for k in range(6)):
+            self.field_work = device.DeviceArray((self.g.nv, 4), np.float32)
+        w = self.field_work
+        _lib.call("vpic_hip_field_step", self.fields.ptr, self.acc.ptr,
+                  self.interp.ptr, w.ptr if w is not None else None,
+                  self._G(), ctypes.byref(self.mp), self.stream)
 
     def energy_f(self):
         en = (ctypes.c_double * 6)()
@@ -452,12 +464,7 @@ class Simulation:
                 self.boundary_p()
             self.reduce_accumulator_array()
         with t("field"):
-            self.unload_accumulator_array()
-            self.advance_b(0.5)
-            self.advance_e(1.0)
-            self.advance_b(0.5)
-        with t("interp"):
-            self.load_interpolator_array()
+            self.field_step()
         self.step += 1
 
 
