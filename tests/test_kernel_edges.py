@@ -386,3 +386,44 @@ def test_field_step(dev, n, wall, work):
                   w.ptr if work else None, G, M, None)
         assert H.same_bits(b.download(), a.download())
         assert H.same_bits(ib.download(), ia.download())
+
+
+# the jf fold of all axes and the B ghosts in one launch, and their transposes,
+# where an axis has one or two cells (the copies of an element are neighbours)
+@pytest.mark.parametrize("n", [(3, 2, 4), (1, 5, 3), (2, 1, 6), (7, 1, 1)],
+                         ids=lambda v: "x".join(map(str, v)))
+def test_adjoint_faces(dev, orc, n):
+    """FP64: the run's energy is the FP64 oracle's, and its gradient in the
+    fields gives the central difference along a random direction (step 1e-6
+    of fields of 0.02: truncation and rounding both below 1e-8 of it, where no
+    particle crosses a face in between; 1e-5 leaves room for their sum over
+    the steps)."""
+    import torch
+    from oracle.trace import OracleRun
+    from vpic_amd import adjoint as A
+    g = _box(*n, cell=0.1)
+    P, F = _adjoint_inputs(g, 40, 8, True)
+    f = H.random_fields(g, 9, 0.02, 0.02)  # the inputs' fields
+    P32, _ = _adjoint_inputs(g, 40, 8, False)
+    p = P32.cpu().numpy().reshape(-1).view(T.PARTICLE)
+    steps = 6
+    say("adjoint faces", n)
+    w, _, _, fb = A.run(P, F, g, -1.0, 1.0, steps, 4, True, True, True)
+    r = OracleRun(g, [("electron", -1.0, 1.0, p)], fp64=True, fields=f)
+    r.load_interpolator()
+    for _ in range(steps):
+        r.advance()
+    wo = r.energies()[0][3:6].sum()
+    r.close()
+    assert abs(w - wo) <= 1e-12 * abs(wo)
+    d = torch.from_numpy(np.random.default_rng(3).standard_normal(
+        (g.nv, 6))).cuda()
+    dF = torch.zeros_like(F)
+    dF[:, 0:3], dF[:, 4:7] = d[:, 0:3], d[:, 3:6]
+    eps = 2e-8
+    hi, lo = (A.run(P, (F + s * eps * dF).contiguous(), g, -1.0, 1.0, steps,
+                    grads=False)[0] for s in (1, -1))
+    want = (hi - lo) / (2 * eps)
+    got = float((fb * d).sum())
+    say("adjoint", got, "difference", want)
+    assert abs(got - want) <= 1e-5 * abs(want)

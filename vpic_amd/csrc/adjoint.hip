@@ -1037,9 +1037,8 @@ __global__ void k_load_T(Fld<R> *Fb, const R *fib, Box B) {
 // clear_jf + unload_accumulator over voxels 1..n+1
 // (unload_accumulator_pipeline.cc:65-67)
 template <class R>
-__global__ void k_unload(Fld<R> *F, const R *acc, Coef<R> C, Box B) {
-  const int v = blockIdx.x * blockDim.x + threadIdx.x;
-  if (v >= B.nv) return;
+__device__ void unload_at(Fld<R> *F, const R *acc, const Coef<R> &C,
+                          const Box &B, int v) {
   int x, y, z;
   coords(B, v, x, y, z);
   Fld<R> &f = F[v];
@@ -1057,7 +1056,7 @@ __global__ void k_unload(Fld<R> *F, const R *acc, Coef<R> C, Box B) {
   f.jfz += C.uc[2] * (a0[8] + ax[9] + ay[10] + axy[11]);
 }
 
-// Transpose of k_unload: accumulator adjoint of voxel u from jf-bar.
+// Transpose of unload_at: accumulator adjoint of voxel u from jf-bar.
 template <class R>
 __global__ void k_unload_T(R *accb, const Fld<R> *Fb, Coef<R> C, Box B) {
   const int u = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1086,43 +1085,62 @@ __global__ void k_unload_T(R *accb, const Fld<R> *Fb, Coef<R> C, Box B) {
   o[11] = C.uc[2] * jb(u + sx + sy, 2);
 }
 
-// synchronize_jf on a periodic box, one axis X (remote.cc:474-502): the
-// tangential jf of the two face planes X = 1 and X = n+1 both become their
-// sum.  The map is symmetric, so it is its own transpose.
+// synchronize_jf on a periodic box (remote.cc:474-502): along each axis the
+// tangential jf of the two face planes 1 and n+1 both become their sum, axis
+// after axis.  The map of one axis is symmetric, so the transpose is the axes
+// in the other order (`back`).  All axes at once: component c = l / (places)
+// is folded along the two others, P < Q; a thread has all copies of an
+// element (two on a face, four on an edge).  A launch an axis was 4 us each.
+__host__ __device__ inline int fold_places(const Box &B, int C) {
+  return C == 0   ? B.nx * (B.nz + B.ny - 1)
+         : C == 1 ? B.ny * (B.nz + B.nx - 1)
+                  : B.nz * (B.ny + B.nx - 1);
+}
+__host__ __device__ inline int64_t fold_places(const Box &B) {
+  return (int64_t)fold_places(B, 0) + fold_places(B, 1) + fold_places(B, 2);
+}
 template <class R>
-__global__ void k_fold_jf(Fld<R> *F, Box B, int X) {
+__device__ void fold_jf_at(Fld<R> *F, const Box &B, int64_t l, bool back) {
+  int C = 0;
+  while (C < 2 && l >= fold_places(B, C)) l -= fold_places(B, C++);
   const int n[3] = {B.nx, B.ny, B.nz};
-  const int Y = (X + 1) % 3, Z = (X + 2) % 3;
-  const int nY = n[Y] + 1, nZ = n[Z] + 1;
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= nY * nZ) return;
-  const int yy = 1 + k % nY, zz = 1 + k / nY;
-  int c[3];
-  c[X] = 1;
-  c[Y] = yy;
-  c[Z] = zz;
-  const int lo = vox(c[0], c[1], c[2], B.nx, B.ny);
-  c[X] = n[X] + 1;
-  const int hi = vox(c[0], c[1], c[2], B.nx, B.ny);
-  R *flo = &F[lo].jfx, *fhi = &F[hi].jfx;
-  // jf_Y on (Y in 1..nY, Z in 1..nZ+1), jf_Z on (Y in 1..nY+1, Z in 1..nZ)
-  if (yy <= n[Y]) {
-    const R s = flo[Y] + fhi[Y];
-    flo[Y] = s;
-    fhi[Y] = s;
+  const int st[3] = {1, B.sy, B.sz};
+  const int P = C == 0 ? 1 : 0, Q = C == 2 ? 1 : 2;
+  const int nC = n[C], m = (int)l / nC, c = 1 + (int)l % nC;
+  // the P faces (places q = 1..nQ of both planes), then the Q faces off them
+  const bool on_p = m < n[Q];
+  const int hp = n[P] * st[P], hq = n[Q] * st[Q];
+  R *j = &F[c * st[C] + (on_p ? 1 : 2 + m - n[Q]) * st[P] +
+            (on_p ? 1 + m : 1) * st[Q]]
+              .jfx +
+         C;
+  auto at = [&](int h) -> R & {
+    return *reinterpret_cast<R *>(reinterpret_cast<char *>(j) +
+                                  (int64_t)h * sizeof(Fld<R>));
+  };
+  if (on_p && m == 0) {
+    const R a = at(0), b = at(hp), d = at(hq), e = at(hp + hq);
+    const R t = back ? (a + d) + (b + e) : (a + b) + (d + e);
+    at(0) = t;
+    at(hp) = t;
+    at(hq) = t;
+    at(hp + hq) = t;
+  } else {
+    const int h = on_p ? hp : hq;
+    const R t = at(0) + at(h);
+    at(0) = t;
+    at(h) = t;
   }
-  if (zz <= n[Z]) {
-    const R s = flo[Z] + fhi[Z];
-    flo[Z] = s;
-    fhi[Z] = s;
-  }
+}
+template <class R>
+__global__ void k_fold_jf_T(Fld<R> *Fb, Box B) {
+  const int64_t l = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (l < fold_places(B)) fold_jf_at(Fb, B, l, true);
 }
 
 // advance_b (advance_b_pipeline.h:57-59 over voxels 1..n+1)
 template <class R>
-__global__ void k_advance_b(Fld<R> *F, Coef<R> C, Box B) {
-  const int v = blockIdx.x * blockDim.x + threadIdx.x;
-  if (v >= B.nv) return;
+__device__ void advance_b_at(Fld<R> *F, const Coef<R> &C, const Box &B, int v) {
   int x, y, z;
   coords(B, v, x, y, z);
   if (!in_box(B, x, y, z, 1, B.nx + 1, 1, B.ny + 1, 1, B.nz + 1)) return;
@@ -1141,6 +1159,19 @@ __global__ void k_advance_b(Fld<R> *F, Coef<R> C, Box B) {
     const Fld<R> *fx = F + v + 1, *fy = F + v + B.sy;
     f->cbz -= (px * (fx->ey - f->ey) - py * (fy->ex - f->ex));
   }
+}
+template <class R>
+__global__ void k_advance_b(Fld<R> *F, Coef<R> C, Box B) {
+  const int v = blockIdx.x * blockDim.x + threadIdx.x;
+  if (v < B.nv) advance_b_at(F, C, B, v);
+}
+// (jf and B of a voxel, from the accumulator and E: one pass for both)
+template <class R>
+__global__ void k_unload_advance_b(Fld<R> *F, const R *acc, Coef<R> C, Box B) {
+  const int v = blockIdx.x * blockDim.x + threadIdx.x;
+  if (v >= B.nv) return;
+  unload_at(F, acc, C, B, v);
+  advance_b_at(F, C, B, v);
 }
 
 __device__ inline bool in_bx(const Box &B, int v) {
@@ -1205,9 +1236,7 @@ __global__ void k_advance_b_T(Fld<R> *Fb, Coef<R> C, Box B) {
 // self-loop port): the ghost plane X = n+1 takes face plane 1, X = 0 takes
 // face plane n, for the two tangential components.
 template <class R>
-__global__ void k_ghost_b(Fld<R> *F, Box B) {
-  const int v = blockIdx.x * blockDim.x + threadIdx.x;
-  if (v >= B.nv) return;
+__device__ void ghost_b_at(Fld<R> *F, const Box &B, int v) {
   int c[3];
   coords(B, v, c[0], c[1], c[2]);
   const int n[3] = {B.nx, B.ny, B.nz};
@@ -1228,54 +1257,57 @@ __global__ void k_ghost_b(Fld<R> *F, Box B) {
   }
 }
 
-// Transpose of k_ghost_b, first half: each face-plane element adds the
-// adjoints of the ghosts copied from it.
+// The jf fold and the B ghosts, which share no component.
 template <class R>
-__global__ void k_ghost_b_T_add(Fld<R> *Fb, Box B) {
+__global__ void k_fold_jf_ghost_b(Fld<R> *F, Box B, int fold_blocks) {
+  const int b = blockIdx.x;
+  if (b < fold_blocks) {
+    const int64_t l = b * (int64_t)blockDim.x + threadIdx.x;
+    if (l < fold_places(B)) fold_jf_at(F, B, l, false);
+    return;
+  }
+  const int v = (b - fold_blocks) * blockDim.x + threadIdx.x;
+  if (v < B.nv) ghost_b_at(F, B, v);
+}
+
+// Transpose of ghost_b_at: each face-plane element adds the ghosts it fed and
+// clears them (a ghost is fed by one element, and is no face-plane element of
+// another axis, so no other thread touches either).
+template <class R>
+__global__ void k_ghost_b_T(Fld<R> *Fb, Box B) {
   const int v = blockIdx.x * blockDim.x + threadIdx.x;
   if (v >= B.nv) return;
   int c[3];
   coords(B, v, c[0], c[1], c[2]);
   const int n[3] = {B.nx, B.ny, B.nz};
   R add[3] = {0, 0, 0};
+  bool any[3] = {false, false, false};
   for (int X = 0; X < 3; X++) {
     const int Y = (X + 1) % 3, Z = (X + 2) % 3;
+    const bool inY = c[Y] >= 1 && c[Y] <= n[Y] + 1 && c[Z] >= 1 && c[Z] <= n[Z];
+    const bool inZ = c[Y] >= 1 && c[Y] <= n[Y] && c[Z] >= 1 && c[Z] <= n[Z] + 1;
     for (int side = 0; side < 2; side++) {
       // face plane 1 feeds ghost n+1; face plane n feeds ghost 0
       const int face = side == 0 ? 1 : n[X];
       if (c[X] != face) continue;
       int g[3] = {c[0], c[1], c[2]};
       g[X] = side == 0 ? n[X] + 1 : 0;
-      const R *gb = &Fb[vox(g[0], g[1], g[2], B.nx, B.ny)].cbx;
-      if (c[Y] >= 1 && c[Y] <= n[Y] + 1 && c[Z] >= 1 && c[Z] <= n[Z])
+      R *gb = &Fb[vox(g[0], g[1], g[2], B.nx, B.ny)].cbx;
+      if (inY) {
         add[Y] += gb[Y];
-      if (c[Y] >= 1 && c[Y] <= n[Y] && c[Z] >= 1 && c[Z] <= n[Z] + 1)
+        gb[Y] = 0;
+        any[Y] = true;
+      }
+      if (inZ) {
         add[Z] += gb[Z];
+        gb[Z] = 0;
+        any[Z] = true;
+      }
     }
   }
-  Fb[v].cbx += add[0];
-  Fb[v].cby += add[1];
-  Fb[v].cbz += add[2];
-}
-
-// Second half: the ghosts' adjoints are consumed (the forward overwrote
-// the ghosts).
-template <class R>
-__global__ void k_ghost_b_T_zero(Fld<R> *Fb, Box B) {
-  const int v = blockIdx.x * blockDim.x + threadIdx.x;
-  if (v >= B.nv) return;
-  int c[3];
-  coords(B, v, c[0], c[1], c[2]);
-  const int n[3] = {B.nx, B.ny, B.nz};
-  R *dst = &Fb[v].cbx;
-  for (int X = 0; X < 3; X++) {
-    if (c[X] != 0 && c[X] != n[X] + 1) continue;
-    const int Y = (X + 1) % 3, Z = (X + 2) % 3;
-    if (c[Y] >= 1 && c[Y] <= n[Y] + 1 && c[Z] >= 1 && c[Z] <= n[Z])
-      dst[Y] = 0;
-    if (c[Y] >= 1 && c[Y] <= n[Y] && c[Z] >= 1 && c[Z] <= n[Z] + 1)
-      dst[Z] = 0;
-  }
+  R *b = &Fb[v].cbx;
+  for (int k = 0; k < 3; k++)
+    if (any[k]) b[k] += add[k];
 }
 
 // vacuum_advance_e with no damping (vacuum_advance_e_pipeline.h:56-69;
@@ -1585,15 +1617,10 @@ struct Run {
                    (const R *)wbuf, B, T);
       }
     }
-    ADJ_LAUNCH(k_unload<R>, cover(B.nv), F, (const R *)acc, C, B);
-    for (int X = 0; X < 3; X++) {
-      const int n[3] = {B.nx, B.ny, B.nz};
-      ADJ_LAUNCH(k_fold_jf<R>,
-                 cover((int64_t)(n[(X + 1) % 3] + 1) * (n[(X + 2) % 3] + 1)), F,
-                 B, X);
-    }
-    ADJ_LAUNCH(k_advance_b<R>, cover(B.nv), F, C, B);
-    ADJ_LAUNCH(k_ghost_b<R>, cover(B.nv), F, B);
+    ADJ_LAUNCH(k_unload_advance_b<R>, cover(B.nv), F, (const R *)acc, C, B);
+    const int fold_blocks = cover(fold_places(B)).x;
+    ADJ_LAUNCH(k_fold_jf_ghost_b<R>, dim3(fold_blocks + cover(B.nv).x), F, B,
+               fold_blocks);
     ADJ_LAUNCH(k_advance_e<R>, cover(B.nv), F, C, B);
     ADJ_LAUNCH(k_advance_b<R>, cover(B.nv), F, C, B);
     return load();
@@ -1630,15 +1657,9 @@ struct Run {
              Fld<R> *Fb, R *fib, R *accb) {
     ADJ_LAUNCH(k_advance_b_T<R>, cover(B.nv), Fb, C, B);
     ADJ_LAUNCH(k_advance_e_T<R>, cover(B.nv), Fb, C, B);
-    ADJ_LAUNCH(k_ghost_b_T_add<R>, cover(B.nv), Fb, B);
-    ADJ_LAUNCH(k_ghost_b_T_zero<R>, cover(B.nv), Fb, B);
+    ADJ_LAUNCH(k_ghost_b_T<R>, cover(B.nv), Fb, B);
     ADJ_LAUNCH(k_advance_b_T<R>, cover(B.nv), Fb, C, B);
-    for (int X = 2; X >= 0; X--) {
-      const int n[3] = {B.nx, B.ny, B.nz};
-      ADJ_LAUNCH(k_fold_jf<R>,
-                 cover((int64_t)(n[(X + 1) % 3] + 1) * (n[(X + 2) % 3] + 1)),
-                 Fb, B, X);
-    }
+    ADJ_LAUNCH(k_fold_jf_T<R>, cover(fold_places(B)), Fb, B);
     ADJ_LAUNCH(k_unload_T<R>, cover(B.nv), accb, (const Fld<R> *)Fb, C, B);
     ADJ_LAUNCH(k_load<R>, cover(B.nv), fi, Fn, B);
     ADJ_LAUNCH(k_fill<R>, cover((int64_t)NI * B.nv), fib, (size_t)NI * B.nv,
