@@ -594,13 +594,15 @@ int vpic_hip_clear_hydro_array(vpic_hydro_t *h, const vpic_grid_t *g,
                                void *stream);
 
 /* accumulate_hydro_p (hydro_p.cc:12-19 -> hydro_p_pipeline.cc:17-242):
- * adds the 14 moments of p[0..np) to the nodes, trilinear weights.  With
- * `partition` (from the last vpic_hip_sort_p of these particles) the
- * tiles of the partition are summed in LDS, the particles past it one by
- * one; without it every particle one by one.  The per-particle arithmetic
- * is the reference's; the node sums differ only in order.  Synchronous;
- * particles whose voxel is not interior are skipped and reported as an
- * error.  reduce_hydro_array has nothing to do (one device copy). */
+ * adds the 14 moments of p[0..np) to the nodes, trilinear weights.  The
+ * particles' indices are sorted by voxel (in scratch of 16 bytes a particle
+ * and 448 bytes a voxel of a slab; any order of the particles will do, and
+ * `partition` is not needed), each voxel's moments are summed in registers
+ * and the nodes gather them; grids with an axis of more than 2046 cells take
+ * the particles one by one.  The per-particle arithmetic is the reference's;
+ * the sums differ only in order.  Synchronous; particles whose voxel is not
+ * interior are skipped and reported as an error.  reduce_hydro_array has
+ * nothing to do (one device copy). */
 int vpic_hip_accumulate_hydro_p(vpic_hydro_t *h, const vpic_particle_t *p,
                                 int32_t np, float q, float m,
                                 const vpic_interpolator_t *f,
