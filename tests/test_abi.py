@@ -177,3 +177,29 @@ def test_neighbor_table_matches_oracle(orc):
     _lib.call("vpic_hip_grid_neighbor_table", ctypes.byref(g),
               nb.ctypes.data_as(ctypes.c_void_p))
     assert np.array_equal(nb, neighbor_table(g))
+
+
+def test_field_step_rejects_what_the_separate_calls_do():
+    """NULL or misaligned arrays, inconsistent strides, absorbing faces."""
+    lib = _lib.load()
+    g = T.grid_periodic(0, 0, 0, 4, 4, 4, 4, 4, 4, 0.5)
+    mp = T.vacuum_params()
+
+    def step(f, a, fi, work, grid=g):
+        vp = ctypes.c_void_p
+        return lib.vpic_hip_field_step(vp(f), vp(a), vp(fi), vp(work),
+                                       ctypes.byref(grid), ctypes.byref(mp),
+                                       None)
+
+    for bad in [(None, 16, 16, 16), (16, None, 16, 16), (16, 16, None, 16),
+                (20, 16, 16, 16), (16, 16, 20, 16), (16, 16, 16, 20)]:
+        assert step(*bad) < 0
+        assert b"argument" in lib.vpic_hip_last_error(), bad
+    g2 = g.copy()
+    g2.sy += 1
+    assert step(16, 16, 16, 16, g2) < 0
+    assert b"strides" in lib.vpic_hip_last_error()
+    g3 = g.copy()
+    g3.fbc[0] = g3.fbc[3] = T.BC_ABSORB_FIELDS
+    assert step(16, 16, 16, 16, g3) < 0
+    assert b"absorbing" in lib.vpic_hip_last_error()

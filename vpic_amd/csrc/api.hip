@@ -607,7 +607,8 @@ extern "C" int vpic_hip_field_step(vpic_field_t *f,
                                    void *stream) {
   int rc = check_grid(g);
   if (rc || (rc = check_fields_supported(g))) return rc;
-  CHECK(f && a && fi && mp && aligned16(f) && aligned16(work),
+  CHECK(f && a && fi && mp && aligned16(f) && aligned16(fi) &&
+            aligned16(work),
         "bad argument");
   return launch_field_step(f, a, fi, work, g, mp, S(stream));
 }
