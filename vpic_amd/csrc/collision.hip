@@ -18,15 +18,16 @@
 // collision takes exactly four words of the voxel's stream, and every
 // particle meets its partners in one chain (round the smaller set), so the
 // chains of a voxel are independent.  A workgroup takes a batch of voxels:
-// their momenta go to LDS, all lanes draw the shuffle's words, one lane per
-// voxel swaps indices, then a lane runs each chain with its own words of the
-// stream, and the particles are stored in their shuffled places.  The same
-// draws and the same arithmetic as voxel by voxel on one lane, bit for bit.
+// the momenta (of both species) go to LDS, all lanes draw the shuffle's
+// words, one lane per voxel swaps indices, then a lane runs each chain with
+// its own words of the stream, and the particles are stored in their shuffled
+// places.  The same draws and the same arithmetic as voxel by voxel on one
+// lane, bit for bit.
 // 48^3 cells, 64 electrons and ions in each: 269 us a call within a species
-// (88e6 wavefront instructions, half of the time on the vector units), 537 us
-// between two (the other species' particles are read and written in memory),
-// against 1118 us for either with one lane per voxel, a chain of dependent
-// memory accesses on 7 wavefronts a CU.
+// (88e6 wavefront instructions, half of the time on the vector units), 462 us
+// between two (537 with the other species' particles left in memory), against
+// 1118 us for either with one lane per voxel, a chain of dependent memory
+// accesses on 7 wavefronts a CU.
 #include "common.h"
 
 #include <cfloat>
@@ -185,13 +186,24 @@ struct TaVoxel {
   bool triple;  // and before them the odd three
 };
 
+// Species j's particles of voxel v; false (and none) where its partition does
+// not index them.
+__device__ __forceinline__ bool ta_other(const TaArgs &a, int v, int &l0,
+                                         int &nl) {
+  l0 = a.part_j[v];
+  nl = a.part_j[v + 1] - l0;
+  if (!nl || (l0 >= 0 && nl > 0 && l0 + nl <= a.np_j)) return true;
+  nl = 0;
+  return false;
+}
+
 // The reference's steps between the shuffle and the collisions: pairs of one
-// species (the odd three first), or the sets of two; false when nothing
-// collides.  `density` is species i's, `wj(k)` the weight of species j's k-th.
+// species (the odd three first), or the sets of two (V.l0, V.nl given); false
+// when nothing collides.  `density` is species i's, `wj(k)` the weight of species j's k-th.
 template <class Weight>
 __device__ __forceinline__ bool ta_pairing(const TaArgs &a, int v,
                                            float density, TaVoxel &V,
-                                           int *nbad, Weight wj) {
+                                           Weight wj) {
   V.triple = false;
   V.std3 = 0.0f;
   if (a.same) {
@@ -209,13 +221,7 @@ __device__ __forceinline__ bool ta_pairing(const TaArgs &a, int v,
     V.std = sqrtf((float)(a.cvar * density * a.dtinterval_dV));
     return true;
   }
-  V.l0 = a.part_j[v];
-  V.nl = a.part_j[v + 1] - V.l0;
   if (!V.nl) return false;
-  if (V.l0 < 0 || V.nl < 0 || V.l0 + V.nl > a.np_j) {
-    atomicAdd(nbad, 1);
-    return false;
-  }
   float density_l = 0;
 #pragma unroll 8
   for (int i = 0; i < V.nl; ++i) density_l += wj(V.l0 + i);
@@ -261,7 +267,7 @@ __device__ __forceinline__ float4 *ta_mom(vpic_particle_t *p, int k) {
   return reinterpret_cast<float4 *>(p + k) + 1;
 }
 
-// Particles of species i in a batch: with 28 KiB of momenta four workgroups
+// Particles of a batch, both species': with 28 KiB of momenta four workgroups
 // share a CU's LDS.  Voxels in a batch: one lane each shuffles them.
 constexpr int TA_BS = 256, TA_CAP = 1792, TA_VOX = 64;
 
@@ -273,7 +279,11 @@ __global__ __launch_bounds__(256) void k_ta_crowded(TaArgs a, int *nbad) {
   TaVoxel V;
   V.k0 = a.part_i[v];
   V.nk = a.part_i[v + 1] - V.k0;
-  if (V.k0 < 0 || V.nk <= TA_CAP || V.k0 + V.nk > a.np_i) return;
+  if (V.k0 < 0 || V.nk <= 0 || V.k0 + V.nk > a.np_i) return;
+  V.l0 = V.nl = 0;
+  const bool other = a.same || ta_other(a, v, V.l0, V.nl);
+  if ((int64_t)V.nk + V.nl <= TA_CAP) return;
+  if (!other) atomicAdd(nbad, 1);
   TaRng rng;
   ta_stream(a, v, rng);
   float density = 0;
@@ -290,9 +300,7 @@ __global__ __launch_bounds__(256) void k_ta_crowded(TaArgs a, int *nbad) {
   }
   density += a.pi[i].w;
   V.n = rng.n;
-  if (!ta_pairing(a, v, density, V, nbad,
-                  [&](int k) { return a.pj[k].w; }))
-    return;
+  if (!ta_pairing(a, v, density, V, [&](int k) { return a.pj[k].w; })) return;
   uint32_t w[4];
   auto meet = [&](int k, int l, float std) {
     float4 x = *ta_mom(a.pi, k), y = *ta_mom(a.pj, l);
@@ -327,6 +335,7 @@ __global__ __launch_bounds__(TA_BS, 4) void k_takizuka_abe(TaArgs a, int nvox,
   __shared__ TaVoxel VX[TA_VOX];
   __shared__ int off[TA_VOX + 1];    // first place of each voxel
   __shared__ int first[TA_VOX];      // its first particle
+  __shared__ int off_j[TA_VOX + 1], first_j[TA_VOX];  // of species j
   __shared__ int chain0[2 * TA_VOX + 1];
   __shared__ unsigned char odd[TA_VOX];  // voxels with an odd three
   __shared__ int s_m, s_odd;
@@ -343,20 +352,27 @@ __global__ __launch_bounds__(TA_BS, 4) void k_takizuka_abe(TaArgs a, int nvox,
         // voxel and count it (reported as an error by the host)
         if (nk && (k0 < 0 || nk < 0 || k0 + nk > a.np_i)) nk = -1;
       }
-      const bool bad = nk < 0;
+      bool bad = nk < 0;
       if (bad) nk = 0;
-      const long long incl = wave_incl((long long)nk);
-      const uint64_t fits = __ballot(v + t < vend && incl <= TA_CAP);
+      int l0 = 0, nl = 0;
+      if (nk > 0 && !a.same) bad = !ta_other(a, v + t, l0, nl);
+      const long long incl = wave_incl((long long)nk),
+                      incl_j = wave_incl((long long)nl);
+      const uint64_t fits =
+          __ballot(v + t < vend && incl + incl_j <= TA_CAP);
       const int m = __popcll(fits);  // (incl grows, so the first m lanes)
       if (t < m) {
         if (bad) atomicAdd(nbad, 1);
         off[t + 1] = (int)incl;
         first[t] = k0;
+        off_j[t + 1] = (int)incl_j;
+        first_j[t] = l0;
         VX[t].nk = nk;
         again[t] = 0;
       }
       if (t == 0) {
         off[0] = 0;
+        off_j[0] = 0;
         s_m = m;
       }
     }
@@ -368,7 +384,7 @@ __global__ __launch_bounds__(TA_BS, 4) void k_takizuka_abe(TaArgs a, int nvox,
       __syncthreads();
       continue;
     }
-    const int total = off[m];
+    const int total = off[m], total_j = off_j[m];
     // the last voxel that starts at s or before
     auto find_by = [&](auto at, int s, int hi) {
       int lo = 0;
@@ -385,6 +401,10 @@ __global__ __launch_bounds__(TA_BS, 4) void k_takizuka_abe(TaArgs a, int nvox,
       const int q = find(off, s);
       U[s] = *ta_mom(a.pi, first[q] + (s - off[q]));
       perm[s] = (unsigned short)s;
+    }
+    for (int s = t; s < total_j; s += TA_BS) {
+      const int q = find(off_j, s);
+      U[total + s] = *ta_mom(a.pj, first_j[q] + (s - off_j[q]));
     }
     // The shuffle's draws, four places a lane: place i takes word i unless a
     // draw is rejected (one in 2^32 / places), which shifts those behind it.
@@ -441,8 +461,9 @@ __global__ __launch_bounds__(TA_BS, 4) void k_takizuka_abe(TaArgs a, int nvox,
         float density = 0;
 #pragma unroll 8
         for (int i = V.k0; i < k1; ++i) density += U[perm[i]].w;
-        if (ta_pairing(a, v + t, density, V, nbad,
-                       [&](int k) { return a.pj[k].w; })) {
+        V.l0 = total + off_j[t];
+        V.nl = off_j[t + 1] - off_j[t];
+        if (ta_pairing(a, v + t, density, V, [&](int k) { return U[k].w; })) {
           n_long = V.rn;
           n_short = (V.nk < V.nl ? V.nk : V.nl) - V.rn;
           triple = V.triple;
@@ -495,9 +516,7 @@ __global__ __launch_bounds__(TA_BS, 4) void k_takizuka_abe(TaArgs a, int nvox,
       ta_chain(V, c, many, len);
       const uint32_t n0 = V.n + (V.triple ? 12u : 0u);
       const bool round_l = V.nk > V.nl;  // the one particle is species j's
-      auto at_l = [&](int l) {
-        return a.same ? &U[perm[l]] : ta_mom(a.pj, l);
-      };
+      auto at_l = [&](int l) { return a.same ? &U[perm[l]] : &U[l]; };
       float4 *one = round_l ? at_l(V.l0 + c) : &U[perm[V.k0 + c]];
       float4 ov = *one;
       for (int j = 0; j < len; j++) {
@@ -544,6 +563,10 @@ __global__ __launch_bounds__(TA_BS, 4) void k_takizuka_abe(TaArgs a, int nvox,
         o[1] = U[perm[s]];
       }
     }
+    for (int s = t; s < total_j; s += TA_BS) {
+      const int q = find(off_j, s);
+      *ta_mom(a.pj, first_j[q] + (s - off_j[q])) = U[total + s];
+    }
     __syncthreads();
     v += m;
   }
@@ -583,7 +606,8 @@ int launch_takizuka_abe(vpic_particle_t *pi, const int *part_i, int np_i,
   // voxels of a workgroup: three quarters of a batch at the mean number of
   // particles, since a batch that does not hold them all leaves a short second
   // one (64-particle voxels with their spread of 8: 21 of at most 28)
-  const double mean = (double)np_i / ((double)g->nx * g->ny * g->nz);
+  const double mean = ((double)np_i + (a.same ? 0.0 : (double)np_j)) /
+                      ((double)g->nx * g->ny * g->nz);
   int nvox = mean > 0 ? (int)(0.75 * TA_CAP / mean) : TA_VOX;
   nvox = nvox < 1 ? 1 : nvox > TA_VOX ? TA_VOX : nvox;
   hipLaunchKernelGGL(k_takizuka_abe, dim3((a.v1 + nvox - 1) / nvox),
