@@ -163,6 +163,12 @@ const char *vpic_hip_last_error(void);
 /* Library version string. */
 const char *vpic_hip_version(void);
 
+/* Every thread keeps scratch memory per GPU, grown on demand, that its calls
+ * share.  Calls that return with work queued are ordered by their stream: the
+ * sorts (and the calls that sort: accumulate_hydro_p, the adjoint run) also
+ * wait for the thread's sort before them on another stream; pushes of one
+ * thread belong on one stream, or in order across streams. */
+
 /* ------------------------------------------------------------------------ */
 /* Species advance (src/species_advance/species_advance.h:64-157)          */
 /* ------------------------------------------------------------------------ */

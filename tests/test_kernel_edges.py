@@ -427,3 +427,67 @@ def test_adjoint_faces(dev, orc, n):
     got = float((fb * d).sum())
     say("adjoint", got, "difference", want)
     assert abs(got - want) <= 1e-5 * abs(want)
+
+
+def test_sort_scratch_across_streams(dev):
+    """A sort left queued on one stream and the next use of its thread's
+    scratch on another (the hydro moments, the adjoint run, another sort): the
+    results of one call after the other, bit for bit (the gradient's sums have
+    no fixed order: within 1e-10 of its largest, as above)."""
+    import torch
+    from vpic_amd import adjoint as A
+    g = _box(48, 40, 36)
+    n_a, n_b = 3000000, 2900000
+    rng = np.random.default_rng(8)
+
+    def cloud(n):
+        p = np.zeros(n, dtype=T.PARTICLE)
+        p["i"] = g.voxel(*(rng.integers(1, k + 1, n)
+                           for k in (g.nx, g.ny, g.nz)))
+        p["w"] = np.arange(n, dtype=np.float32)
+        p["ux"] = rng.standard_normal(n).astype(np.float32)
+        return p
+    a, b = cloud(n_a), cloud(n_b)
+    da, db = dev.DeviceArray.from_host(a), dev.DeviceArray.from_host(b)
+    dfi = dev.DeviceArray.from_host(H.interp_array(g))
+    hydro = dev.DeviceArray((g.nv,), T.HYDRO)
+    P, F = _adjoint_inputs(_box(9, 5, 5, 0.1), 257, 5, True)
+
+    def moments(stream):
+        _lib.call("vpic_hip_accumulate_hydro_p", hydro.ptr, db.ptr, n_b, -1.0,
+                  1.0, dfi.ptr, ctypes.byref(g), None, stream)
+        return hydro.download()
+
+    def gradient(stream):  # (always on the default stream)
+        return A.run(P, F, _box(9, 5, 5, 0.1), -1.0, 1.0, 9,
+                     4)[1].cpu().numpy()
+
+    aux_b = dev.particles(n_b)
+    part_b = dev.DeviceArray((g.nv + 1,), np.int32)
+
+    def other_sort(stream):
+        _lib.call("vpic_hip_sort_p", db.ptr, aux_b.ptr, n_b, part_b.ptr,
+                  ctypes.byref(g), 0, stream)
+        return aux_b.download()
+
+    order = np.argsort(a["i"], kind="stable")
+    s1, s2 = torch.cuda.Stream(), torch.cuda.Stream()
+    for name, second in (("hydro", moments), ("adjoint", gradient),
+                         ("sort_p", other_sort)):
+        hydro.zero()
+        torch.cuda.synchronize()
+        want = second(None)
+        aux = dev.particles(n_a)
+        part = dev.DeviceArray((g.nv + 1,), np.int32)
+        hydro.zero()
+        torch.cuda.synchronize()
+        say("sort_p, then", name, "on another stream")
+        _lib.call("vpic_hip_sort_p", da.ptr, aux.ptr, n_a, part.ptr,
+                  ctypes.byref(g), 0, s1.cuda_stream)
+        got = second(s2.cuda_stream)
+        torch.cuda.synchronize()
+        assert H.same_bits(aux.download(), a[order])
+        if name == "adjoint":
+            assert np.max(np.abs(got - want)) <= 1e-10 * np.max(np.abs(want))
+        else:
+            assert H.same_bits(got, want)

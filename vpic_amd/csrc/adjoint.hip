@@ -1574,8 +1574,10 @@ struct Run {
   int sort(const vpic_grid_t *g, int *perm, int *rows, bool check) {
     ADJ_LAUNCH(k_keys<R>, dim3(nkeyblk()), (const Part<R> *)p, np, keys);
     int rc, *order, *sorted, bad = 0;
-    if ((rc = device_sort_keys(keys, np, g, &order, &sorted,
-                               check ? &bad : nullptr, s)))
+    SortScratchUse use;
+    if ((rc = use.begin(s)) ||
+        (rc = device_sort_keys(keys, np, g, &order, &sorted,
+                               check ? &bad : nullptr, use, s)))
       return rc;
     if (bad)
       return vpic_set_error(VPIC_EINVAL,

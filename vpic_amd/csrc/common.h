@@ -351,14 +351,28 @@ int launch_sort_p_keys(vpic_particle_t *p, vpic_particle_t *aux, int np,
                        int *partition, const int *keys, const vpic_grid_t *g,
                        int in_place, hipStream_t s);
 long long sort_keys_stale_count();
+// One use of this thread's sort scratch, from begin() until everything that
+// reads it is queued on the stream (the object's end) or has run
+// (synchronised()): a use on another stream waits for the one before it.
+struct SortScratchUse {
+  hipStream_t s = nullptr;
+  bool open = false;
+  SortScratchUse() = default;
+  SortScratchUse(const SortScratchUse &) = delete;
+  SortScratchUse &operator=(const SortScratchUse &) = delete;
+  ~SortScratchUse();
+  int begin(hipStream_t stream);
+  void synchronised();
+};
 // The stable sort by voxel of the keys themselves (grids sort_keys_fit
 // accepts): *order[j] = the element at place j, *sorted[j] its key (in this
-// thread's sort scratch: valid until its next sort).  A key outside [0, nv)
-// sorts as 0; *bad (may be null) receives their number after a
-// synchronisation of the stream.
+// thread's sort scratch: valid while `use`, begun on this stream, lasts).  A
+// key outside [0, nv) sorts as 0; *bad (may be null) receives their number
+// after a synchronisation of the stream.
 bool sort_keys_fit(const vpic_grid_t *g);
 int device_sort_keys(const int *keys, int np, const vpic_grid_t *g,
-                     int **order, int **sorted, int *bad, hipStream_t s);
+                     int **order, int **sorted, int *bad,
+                     const SortScratchUse &use, hipStream_t s);
 int launch_energy_p(const vpic_particle_t *p, int np, float q, float m,
                     const vpic_interpolator_t *f, const vpic_grid_t *g,
                     double *host_en, hipStream_t s);

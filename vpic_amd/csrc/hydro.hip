@@ -350,6 +350,7 @@ int launch_accumulate_hydro_p(vpic_hydro_t *h, const vpic_particle_t *p,
   // (the voxels are the particles' own: the partition of their last sort is
   // not needed)
   (void)partition;
+  SortScratchUse use;
   // voxels whose eight nodes lie on the grid
   const int vmax = g->nv - g->sz - g->sy - 1;
   if (np > 0 && !sort_keys_fit(g)) {
@@ -377,7 +378,8 @@ int launch_accumulate_hydro_p(vpic_hydro_t *h, const vpic_particle_t *p,
                        g->nv, keys, nbad);
     VPIC_LAUNCHED("k_hydro_keys");
     int *order, *sorted;
-    if ((rc = device_sort_keys(keys, np, g, &order, &sorted, nullptr, s)))
+    if ((rc = use.begin(s)) ||
+        (rc = device_sort_keys(keys, np, g, &order, &sorted, nullptr, use, s)))
       return rc;
     hipLaunchKernelGGL(k_hydro_starts, dim3(blocks_for((int64_t)g->nv + 1, 256)),
                        dim3(256), 0, s, (const int *)sorted, np, g->nv, start);
@@ -402,6 +404,7 @@ int launch_accumulate_hydro_p(vpic_hydro_t *h, const vpic_particle_t *p,
   int h_bad = 0;
   VPIC_HIP(hipMemcpyAsync(&h_bad, nbad, sizeof(int), hipMemcpyDeviceToHost, s));
   VPIC_HIP(hipStreamSynchronize(s));
+  use.synchronised();
   if (h_bad)
     return vpic_set_error(VPIC_EINVAL,
                           "accumulate_hydro_p: %d particles with a voxel "

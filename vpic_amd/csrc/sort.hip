@@ -494,6 +494,8 @@ __global__ __launch_bounds__(256) void k_gather_part(
 
 struct SortScratch {
   DeviceScratch keys, perm, count, sums, big, nbig, tmp, keys2, idx2, hist;
+  hipEvent_t used = nullptr;  // the end of the last use that was left queued
+  bool queued = false;
 };
 SortScratch &sort_scratch() {
   static thread_local SortScratch s[16];
@@ -505,6 +507,40 @@ SortScratch &sort_scratch() {
 inline int blocks_for(int64_t n, int bs) { return (int)((n + bs - 1) / bs); }
 
 }  // namespace
+
+// A thread's uses of its sort scratch come one after the other whatever their
+// streams: sort_p and the index sorts of the hydro moments and the adjoint run
+// share it, and sort_p returns with its gather still queued.  (Not while the
+// stream is captured: a graph cannot hold an event of another stream, and the
+// only sort that does not synchronise, of no particles, reads no particle.)
+int SortScratchUse::begin(hipStream_t stream) {
+  s = stream;
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  VPIC_HIP(hipStreamIsCapturing(s, &st));
+  if (st != hipStreamCaptureStatusNone) return VPIC_OK;
+  SortScratch &S = sort_scratch();
+  if (!S.used)
+    VPIC_HIP(hipEventCreateWithFlags(&S.used, hipEventDisableTiming));
+  if (S.queued) VPIC_HIP(hipStreamWaitEvent(s, S.used, 0));
+  open = true;
+  return VPIC_OK;
+}
+
+void SortScratchUse::synchronised() {
+  if (open) sort_scratch().queued = false;
+  open = false;
+}
+
+SortScratchUse::~SortScratchUse() {
+  if (!open) return;
+  SortScratch &S = sort_scratch();
+  // (nothing left to order by: wait for the stream itself)
+  S.queued = hipEventRecord(S.used, s) == hipSuccess;
+  if (!S.queued) {
+    (void)hipGetLastError();
+    (void)hipStreamSynchronize(s);
+  }
+}
 
 // Exclusive scan of n ints (in may equal out).  sums: ceil(n/2048) ints.
 int device_exclusive_scan(const int *in, int *out, int64_t n, int *sums,
@@ -673,7 +709,7 @@ int sort_pairs(const vpic_particle_t *p, int np, const vpic_grid_t *g,
 // or a key outside [0, nv), returns SORT_KEYS_STALE before p is touched.
 int sort_p_axes(vpic_particle_t *p, vpic_particle_t *aux, int np,
                 int *partition, const vpic_grid_t *g, int in_place,
-                const int *hint, hipStream_t s) {
+                const int *hint, SortScratchUse &use, hipStream_t s) {
   int rc, *ia, *ka, *nbad;
   if ((rc = sort_pairs(p, np, g, hint, &ia, &ka, &nbad, s))) return rc;
   hipLaunchKernelGGL(k_gather_part<GATHER_GU>,
@@ -686,6 +722,7 @@ int sort_p_axes(vpic_particle_t *p, vpic_particle_t *aux, int np,
     VPIC_HIP(hipMemcpyAsync(h, nbad, sizeof(h), hipMemcpyDeviceToHost, s));
     VPIC_HIP(hipStreamSynchronize(s));
     if (h[0] > 0 || h[1] > 0) return SORT_KEYS_STALE;
+    use.synchronised();
   }
   if (in_place)
     VPIC_HIP(hipMemcpyAsync(p, aux, sizeof(vpic_particle_t) * (size_t)np,
@@ -917,8 +954,10 @@ int launch_sort_p(vpic_particle_t *p, vpic_particle_t *aux, int np,
                   hipStream_t s) {
   push_invalidate_bins(p);
   push_invalidate_bins(aux);
+  SortScratchUse use;
+  if (int rc = use.begin(s)) return rc;
   if (np > 0 && sort_keys_fit(g))
-    return sort_p_axes(p, aux, np, partition, g, in_place, nullptr, s);
+    return sort_p_axes(p, aux, np, partition, g, in_place, nullptr, use, s);
   return sort_p_counting(p, aux, np, partition, g, in_place, s);
 }
 
@@ -933,10 +972,13 @@ int launch_sort_p_keys(vpic_particle_t *p, vpic_particle_t *aux, int np,
     return launch_sort_p(p, aux, np, partition, g, in_place, s);
   push_invalidate_bins(p);
   push_invalidate_bins(aux);
-  const int rc = sort_p_axes(p, aux, np, partition, g, in_place, keys, s);
+  SortScratchUse use;
+  int rc = use.begin(s);
+  if (rc) return rc;
+  rc = sort_p_axes(p, aux, np, partition, g, in_place, keys, use, s);
   if (rc != SORT_KEYS_STALE) return rc;
   note_sort_keys_stale();
-  return sort_p_axes(p, aux, np, partition, g, in_place, nullptr, s);
+  return sort_p_axes(p, aux, np, partition, g, in_place, nullptr, use, s);
 }
 
 bool sort_keys_fit(const vpic_grid_t *g) {
@@ -944,7 +986,8 @@ bool sort_keys_fit(const vpic_grid_t *g) {
 }
 
 int device_sort_keys(const int *keys, int np, const vpic_grid_t *g,
-                     int **order, int **sorted, int *bad, hipStream_t s) {
+                     int **order, int **sorted, int *bad,
+                     const SortScratchUse &, hipStream_t s) {
   int rc, *nbad;
   if ((rc = sort_pairs(nullptr, np, g, keys, order, sorted, &nbad, s)))
     return rc;
