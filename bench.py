@@ -465,8 +465,9 @@ def main():
     assert bad == 0
 
     value = npart * args.steps / el
-    tile = (ctypes.c_int32 * 4)()
-    _lib.call("vpic_hip_push_get_tile", tile)
+    tile, ntile = (ctypes.c_int32 * 4)(), ctypes.c_int32()
+    _lib.call("vpic_hip_push_tile_choices", ctypes.byref(s.g), npart, tile,
+              ctypes.byref(ntile))
     stale = ctypes.c_int64()
     _lib.call("vpic_hip_sort_keys_stale", ctypes.byref(stale))
     avg_launch_s = push_ms.value / 1e3 / max(launches.value, 1)

@@ -274,9 +274,9 @@ int vpic_hip_advance_p_noalloc(vpic_particle_t *p, int32_t np, float q,
                                const vpic_grid_t *g, void *stream);
 
 /* Tile shape (cells) of the partition-driven push; its LDS window holds
- * (tx+2)(ty+2)(tz+2) accumulators (a halo of one cell).  Until this or
- * vpic_hip_push_tile_window is called, 7x8x7 on large grids and a shape
- * chosen from the grid's size and particles on others.
+ * (tx+2)(ty+2)(tz+2) accumulators (a halo of one cell).  0, 0, 0, as
+ * at the start: the push takes 7x8x7 on large grids and a shape chosen from
+ * the grid's size and particles on others.
  * No reference counterpart (the reference's pipelines split particles,
  * not cells). */
 int vpic_hip_push_tile(int32_t tx, int32_t ty, int32_t tz);
@@ -292,9 +292,16 @@ int vpic_hip_push_tile(int32_t tx, int32_t ty, int32_t tz);
 int vpic_hip_push_tile_window(int32_t tx, int32_t ty, int32_t tz,
                               int32_t halo);
 
-/* The tile shape and halo set, or 7, 8, 7, 1: out[0..3] = tx, ty, tz, halo.  No
+/* The tile shape and halo set: out[0..3] = tx, ty, tz, halo, or 0, 0, 0, 1
+ * while the push chooses, so that setting them again restores either.  No
  * reference counterpart. */
 int vpic_hip_push_get_tile(int32_t *out);
+
+/* The tile (cut to the grid) that a push of np particles, all species of the
+ * call together, has on grid g: out[0..3] = tx, ty, tz, halo and *n = 1.
+ * Needs no GPU.  No reference counterpart. */
+int vpic_hip_push_tile_choices(const vpic_grid_t *g, int64_t np, int32_t *out,
+                               int32_t *n);
 
 /* Wavefronts whose 64 particles fall in at least `runs` runs of equal
  * voxels deposit lane by lane instead of summing runs first (default 65,

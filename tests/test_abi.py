@@ -203,3 +203,37 @@ def test_field_step_rejects_what_the_separate_calls_do():
     g3.fbc[0] = g3.fbc[3] = T.BC_ABSORB_FIELDS
     assert step(16, 16, 16, 16, g3) < 0
     assert b"absorbing" in lib.vpic_hip_last_error()
+
+
+def _push_tile(n, np_, walls=False):
+    g = T.grid_periodic(0, 0, 0, *n, *n, 0.5)
+    if walls:
+        g.fbc[0] = g.fbc[3] = T.BC_PEC_FIELDS
+        g.pbc[0] = g.pbc[3] = T.BC_REFLECT_PARTICLES
+    out, k = (ctypes.c_int32 * 12)(), ctypes.c_int32()
+    _lib.call("vpic_hip_push_tile_choices", ctypes.byref(g), int(np_), out,
+              ctypes.byref(k))
+    return [tuple(out[4 * j:4 * j + 4]) for j in range(k.value)]
+
+
+def test_push_tile_saved_and_restored():
+    """What the getter gives restores the push's own choice as well as a tile
+    that was set; a tile that is refused changes nothing."""
+    was, now = (ctypes.c_int32 * 4)(), (ctypes.c_int32 * 4)()
+    _lib.call("vpic_hip_push_tile", 0, 0, 0)
+    small, large = _push_tile((12, 10, 9), 20000), \
+        _push_tile((256, 128, 128), 8 * 10 ** 8)
+    assert small != [(7, 8, 7, 1)] and large == [(7, 8, 7, 1)]
+    _lib.call("vpic_hip_push_get_tile", was)
+    assert tuple(was) == (0, 0, 0, 1)
+    _lib.call("vpic_hip_push_tile_window", *was)
+    assert _push_tile((12, 10, 9), 20000) == small
+    _lib.call("vpic_hip_push_tile_window", 7, 8, 7, 1)
+    assert _push_tile((12, 10, 9), 20000) == [(7, 8, 7, 1)]
+    _lib.call("vpic_hip_push_get_tile", now)
+    assert tuple(now) == (7, 8, 7, 1)
+    with pytest.raises(_lib.VpicError):
+        _lib.call("vpic_hip_push_tile", 0, 8, 7)
+    assert _push_tile((5, 3, 2), 100) == [(5, 3, 2, 1)]
+    _lib.call("vpic_hip_push_tile_window", *was)
+    assert _push_tile((12, 10, 9), 20000) == small

@@ -1,7 +1,6 @@
-"""The partition-driven push with the tile it chooses itself (no test module
-before this one sets a tile): grids of fewer tiles than CUs, of several tiles
-per CU in density order, between walls, one cell thick, and particles past the
-partition."""
+"""The partition-driven push with the tile it chooses itself: grids of fewer
+tiles than CUs, of several tiles per CU in density order, between walls, one
+cell thick, and particles past the partition."""
 import ctypes
 import sys
 
@@ -29,6 +28,15 @@ def dev():
     _lib.call("vpic_hip_init", 0)
     from vpic_amd import device
     return device
+
+
+@pytest.fixture(autouse=True)
+def chosen_tile():
+    was = (ctypes.c_int32 * 4)()
+    _lib.call("vpic_hip_push_get_tile", was)
+    _lib.call("vpic_hip_push_tile", 0, 0, 0)
+    yield
+    _lib.call("vpic_hip_push_tile_window", *was)
 
 
 def _particles(g, np_, seed, dense):

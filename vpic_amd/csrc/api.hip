@@ -267,6 +267,14 @@ extern "C" int vpic_hip_push_get_tile(int32_t *out) {
   return VPIC_OK;
 }
 
+extern "C" int vpic_hip_push_tile_choices(const vpic_grid_t *g, int64_t np,
+                                          int32_t *out, int32_t *n) {
+  if (int rc = check_grid(g)) return rc;
+  CHECK(np >= 0 && out && n, "bad argument");
+  *n = push_tile_choices(g, np, out);
+  return VPIC_OK;
+}
+
 extern "C" int vpic_hip_push_tile_window(int32_t tx, int32_t ty, int32_t tz,
                                          int32_t halo) {
   CHECK(halo == 1 || halo == 2, "push window halo %d is not 1 or 2", halo);

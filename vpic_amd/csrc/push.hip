@@ -2312,8 +2312,9 @@ int pow2_at_least(int64_t n) {
 // fastest of the shapes timed on the 256x128x128 thermal plasma over whole
 // sort intervals (8x8x8, whose coefficients fit for the tile only, took 6%
 // longer per push)
-TileGeom g_tile = {7, 8, 7, 0, 0, 0, 0, 0, 0, 1, 1, 1, 1};
-bool g_tile_set = false;  // the caller chose g_tile
+constexpr TileGeom TILE_DEFAULT = {7, 8, 7, 0, 0, 0, 0, 0, 0, 1, 1, 1, 1};
+TileGeom g_tile = TILE_DEFAULT;  // the caller's tile, when there is one
+bool g_tile_set = false;
 int g_group = 16;  // lanes sharing one run of particles in the tiled push
 int g_bin_mode = 0;  // tile lists: 0 off, 1 when drift warrants, 2 always
 
@@ -2461,7 +2462,7 @@ TileGeom push_tile_for(const vpic_grid_t *g, int64_t np) {
   if (last.nx == g->nx && last.ny == g->ny && last.nz == g->nz &&
       last.np == np && memcmp(last.pbc, g->pbc, sizeof last.pbc) == 0)
     return last.T;
-  TileGeom T = g_tile;
+  TileGeom T = TILE_DEFAULT;
   const int mx = g->nx < 32 ? g->nx : 32, my = g->ny < 16 ? g->ny : 16,
             mz = g->nz < 16 ? g->nz : 16;
   double best = 0.95 * tile_cost(g, ppc, T.tx < g->nx ? T.tx : g->nx,
@@ -2498,7 +2499,12 @@ TileGeom push_tile_for(const vpic_grid_t *g, int64_t np) {
 
 // Tile shape and window halo of the tiled push (the window of a tile is
 // (tx+2h)(ty+2h)(tz+2h) cells of 96 B in LDS).
+// (0, 0, 0, 1): the push chooses, as at the start.
 int push_set_tile(int tx, int ty, int tz, int halo) {
+  if (tx == 0 && ty == 0 && tz == 0 && halo == 1) {
+    g_tile_set = false;
+    return VPIC_OK;
+  }
   if (!tile_fits(tx, ty, tz, halo)) return VPIC_EINVAL;
   g_tile_set = true;
   g_tile.tx = tx;
@@ -2509,10 +2515,19 @@ int push_set_tile(int tx, int ty, int tz, int halo) {
 }
 
 void push_get_tile(int out[4]) {
-  out[0] = g_tile.tx;
-  out[1] = g_tile.ty;
-  out[2] = g_tile.tz;
-  out[3] = g_tile.halo;
+  out[0] = g_tile_set ? g_tile.tx : 0;
+  out[1] = g_tile_set ? g_tile.ty : 0;
+  out[2] = g_tile_set ? g_tile.tz : 0;
+  out[3] = g_tile_set ? g_tile.halo : 1;
+}
+
+int push_tile_choices(const vpic_grid_t *g, int64_t np, int *out) {
+  const TileGeom T = push_tile_for(g, np);
+  out[0] = T.tx < g->nx ? T.tx : g->nx;
+  out[1] = T.ty < g->ny ? T.ty : g->ny;
+  out[2] = T.tz < g->nz ? T.tz : g->nz;
+  out[3] = T.halo;
+  return 1;
 }
 
 int push_set_group(int gs) {
