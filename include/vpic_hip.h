@@ -275,8 +275,9 @@ int vpic_hip_advance_p_noalloc(vpic_particle_t *p, int32_t np, float q,
 
 /* Tile shape (cells) of the partition-driven push; its LDS window holds
  * (tx+2)(ty+2)(tz+2) accumulators (a halo of one cell).  0, 0, 0, as
- * at the start: the push takes 7x8x7 on large grids and a shape chosen from
- * the grid's size and particles on others.
+ * at the start: the push takes 7x8x7 on large grids, a shape chosen from
+ * the grid's size and particles on others, and on 2D grids one of several by
+ * the particles' densities.
  * No reference counterpart (the reference's pipelines split particles,
  * not cells). */
 int vpic_hip_push_tile(int32_t tx, int32_t ty, int32_t tz);
@@ -297,8 +298,9 @@ int vpic_hip_push_tile_window(int32_t tx, int32_t ty, int32_t tz,
  * reference counterpart. */
 int vpic_hip_push_get_tile(int32_t *out);
 
-/* The tile (cut to the grid) that a push of np particles, all species of the
- * call together, has on grid g: out[0..3] = tx, ty, tz, halo and *n = 1.
+/* The tiles (cut to the grid) among which a push of np particles, all species
+ * of the call together, takes one by the densities it finds on grid g: *n of
+ * them (1 to 3, the largest first), each tx, ty, tz, halo in out[0..12).
  * Needs no GPU.  No reference counterpart. */
 int vpic_hip_push_tile_choices(const vpic_grid_t *g, int64_t np, int32_t *out,
                                int32_t *n);

@@ -259,3 +259,21 @@ def test_push_tile_choice_costs_little():
     # (4000 searches: 0.08 to 0.2 s; 4000 calls that find an answer: 0.006 s)
     assert time.process_time() - t0 < 0.04
     assert len(seen) <= 2
+
+
+def test_push_tiles_for_dense_regions():
+    """Where the tile for a uniform plasma is larger than 7x8x7 cut to the
+    grid, so that a dense region would fall on fewer CUs, the push has smaller
+    ones to take; walls make no difference."""
+    _lib.call("vpic_hip_push_tile", 0, 0, 0)
+    for n, ppc in (((512, 1, 257), 96), ((256, 1, 256), 128),
+                   ((300, 200, 1), 80), ((1, 300, 200), 80),
+                   ((128, 1, 128), 128)):
+        t = _push_tile(n, ppc * n[0] * n[1] * n[2])
+        cells = [a * b * c for a, b, c, _ in t]
+        assert cells[0] > 49 and cells == sorted(cells, reverse=True)
+        assert cells[-1] <= 64 and len(t) >= 2
+        assert _push_tile(n, ppc * n[0] * n[1] * n[2], True) == t
+    for n, ppc in (((12, 10, 9), 16), ((32, 32, 32), 128), ((64, 1, 64), 128),
+                   ((97, 61, 83), 40), ((256, 128, 128), 200)):
+        assert len(_push_tile(n, ppc * n[0] * n[1] * n[2])) == 1

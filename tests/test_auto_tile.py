@@ -40,8 +40,8 @@ def chosen_tile():
 
 
 def _particles(g, np_, seed, dense):
-    """Random cells, most of them in a slab of a tenth of the longest axis
-    when `dense`."""
+    """Random cells, four fifths of them in a slab of the share `dense` of the
+    longest axis (0: none)."""
     rng = np.random.default_rng(seed)
     p = np.zeros(np_, dtype=T.PARTICLE)
     n = (g.nx, g.ny, g.nz)
@@ -49,7 +49,8 @@ def _particles(g, np_, seed, dense):
     if dense:
         a = int(np.argmax(n))
         c[a] = np.where(rng.random(np_) < 0.8,
-                        1 + n[a] // 2 + c[a] % max(n[a] // 10, 1), c[a])
+                        1 + n[a] // 2 + c[a] % max(int(n[a] * dense), 1),
+                        c[a])
     p["i"] = g.voxel(*c)
     for k in ("dx", "dy", "dz"):
         p[k] = rng.uniform(-1, 1, np_).astype(np.float32)
@@ -75,13 +76,17 @@ def test_push_auto_tile(dev, orc, n, np_, dense, walls, extra):
         for k in (0, 3):
             g.fbc[k] = T.BC_PEC_FIELDS
             g.pbc[k] = T.BC_REFLECT_PARTICLES
+    _push_against_oracle(dev, orc, g, np_, 0.1 if dense else 0, extra, 2)
+
+
+def _push_against_oracle(dev, orc, g, np_, dense, extra, nsp):
     f = H.random_fields(g, 6, 0.05, 0.1)
     fi = H.interp_array(g)
     orc.load_interpolator(fi, f, g)
     hg = host_grid(g)
     ao = H.acc_array(g)
     keep, want = [], []
-    for k, (q, m) in enumerate(((-1.0, 1.0), (1.0, 25.0))):
+    for k, (q, m) in enumerate(((-1.0, 1.0), (1.0, 25.0))[:nsp]):
         p = _particles(g, np_, 7 + k, dense)
         part = orc.sort_p(p, g)
         if extra:
@@ -95,13 +100,30 @@ def test_push_auto_tile(dev, orc, n, np_, dense, walls, extra):
                      len(p), q, m])
     da, dfi = dev.DeviceArray.from_host(H.acc_array(g)), \
         dev.DeviceArray.from_host(fi)
-    arr = (T.PushSpecies * 2)(*[
+    arr = (T.PushSpecies * nsp)(*[
         T.PushSpecies(a.ptr, ln, q, m, pm.ptr, ln, nm.ptr, part.ptr, None)
         for a, pm, nm, part, ln, q, m in keep])
-    say("advance_p_species, chosen tile", n, np_)
-    _lib.call("vpic_hip_advance_p_species", 2, arr, da.ptr, dfi.ptr,
+    say("advance_p_species, chosen tile", g.nx, g.ny, g.nz, np_, dense)
+    _lib.call("vpic_hip_advance_p_species", nsp, arr, da.ptr, dfi.ptr,
               ctypes.byref(g), None)
     for (a, pm, nm, *_), (po, nmo, igo) in zip(keep, want):
         assert H.same_bits(a.download(), po)
         assert tuple(nm.download()[:3]) == (nmo, igo, 0)
     assert H.acc_rel_err(da.download(), ao) <= 1e-5
+
+
+# a plane of every orientation; the densest cells at the mean, at several times
+# it and at far more, where the push has tiles of three sizes to take; fewer
+# tiles of the largest size than CUs, and more; particles past the partition
+@pytest.mark.parametrize("dense", [0, 0.25, 0.05, 0.004])
+@pytest.mark.parametrize("n,ppc,nsp,extra", [
+    ((203, 1, 150), 14, 2, 3), ((1, 190, 161), 30, 1, 0),
+    ((260, 243, 1), 8, 2, 0)], ids=lambda v: str(v).replace(" ", ""))
+def test_push_tile_by_density(dev, orc, n, ppc, nsp, extra, dense):
+    g = T.grid_periodic(0, 0, 0, *n, *n, 0.95 * T.courant_length(*n, *n))
+    np_ = ppc * n[0] * n[1] * n[2]
+    out, k = (ctypes.c_int32 * 12)(), ctypes.c_int32()
+    _lib.call("vpic_hip_push_tile_choices", ctypes.byref(g), nsp * np_, out,
+              ctypes.byref(k))
+    assert k.value >= 2
+    _push_against_oracle(dev, orc, g, np_, dense, extra, nsp)

@@ -311,8 +311,8 @@ int launch_advance_p_noalloc(vpic_particle_t *p, int np, float q, float m,
 int push_noalloc_setup();
 int push_set_tile(int tx, int ty, int tz, int halo);
 void push_get_tile(int out[4]);
-// The tile of a push of np particles (all species) on grid g, cut to the grid:
-// tx, ty, tz, halo; returns their number.
+// The tiles among which a push of np particles (all species) takes one on grid
+// g, cut to the grid: tx, ty, tz, halo each (at most 3); returns their number.
 int push_tile_choices(const vpic_grid_t *g, int64_t np, int *out);
 int push_set_direct_runs(int runs);
 int push_set_group(int gs);

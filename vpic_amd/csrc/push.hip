@@ -35,8 +35,6 @@
 // Both end with k_order_movers: movers the grid cannot handle, sorted by
 // particle index, truncated at max_nm (excess rolled back to the voxel
 // index, advance_p_pipeline.cc:228-236).
-#include <string.h>
-
 #include <mutex>
 #include <vector>
 
@@ -991,6 +989,22 @@ struct TileGeom {
                       // lands beside it)
 };
 
+constexpr int PUSH_CUS = 256;  // compute units of the chip
+
+// One of the tiles a push may take, with what its launch needs, and its
+// estimated time, max(least, at0 + per * p) us where the densest cells hold p
+// particles each.
+struct TileChoice {
+  TileGeom T;
+  int ntiles, wstride, cap;  // cap: records of an out-of-window sub-bucket
+  float least, at0, per;
+};
+constexpr int TILE_CHOICES = 3;
+struct TileChoices {
+  TileChoice c[TILE_CHOICES];
+  int n;
+};
+
 #ifndef VPIC_TILE_BS
 #define VPIC_TILE_BS 1024
 #endif
@@ -1178,8 +1192,9 @@ __device__ __forceinline__ void drain_wave_queue(
   }
 }
 
-// Start of a tiled push: clears the species' counters and, when there are more
-// tiles than CUs, orders the tiles by their particles, the fullest first (in
+// Start of a tiled push.  Clears the species' counters.  Takes the tile for the
+// densest cells, where there is a choice (*sel), and when there are more tiles
+// than CUs, orders them by their particles, the fullest first (in
 // 16 classes of half a power of two each, in the grid's order within a class),
 // so that a dense region neither starts last nor falls on the few XCDs that
 // its columns of tiles are dealt to.  A tile's particles are estimated from
@@ -1187,15 +1202,67 @@ __device__ __forceinline__ void drain_wave_queue(
 constexpr int ORDER_CLASSES = 16;
 constexpr int ORDER_MAX = 8192;  // tiles; more keep the grid's order
 
+__host__ __device__ __forceinline__ bool tiles_ordered(int ntiles) {
+  return ntiles > PUSH_CUS && ntiles <= ORDER_MAX;
+}
+
+// Particles per cell (all species) where they are densest: the largest of
+// 1024 runs of up to eight cells along x, spread evenly over the grid, less
+// three times its statistical spread (which the largest of so many samples
+// exceeds the mean by, also where the plasma is uniform).  One workgroup of
+// 1024.  (4096 runs took 25 us.)
+__device__ __forceinline__ float densest_cells(const TileSpeciesSet &SS,
+                                               int nsp, const GridDev &G,
+                                               int *peak) {
+  const int t = threadIdx.x;
+  const int segs = (G.nx + 7) / 8;
+  const int total = segs * G.ny * G.nz;  // (below the number of voxels)
+  if (t == 0) *peak = 0;
+  __syncthreads();
+  if (t < total) {
+    const int at = total < 1024 ? t : (int)(((int64_t)total * t) >> 10);
+    const int row = at / segs, x0 = 1 + 8 * (at - row * segs);
+    const int z = row / G.ny, y = row - z * G.ny;
+    const int v = vox(x0, 1 + y, 1 + z, G.nx, G.ny);
+    const int cells = min(8, G.nx + 1 - x0);
+    int n = 0;
+    for (int s = 0; s < nsp; s++) {
+      const int *part = SS.s[s].part;
+      n += part[v + cells] - part[v];
+    }
+    const float c = (float)max(n, 0);
+    const float d = (c - 3.0f * sqrtf(c)) / (float)cells;
+    atomicMax(peak, __float_as_int(fmaxf(d, 0.0f)));  // (bits order as they do)
+  }
+  __syncthreads();
+  return __int_as_float(*peak);
+}
+
 __global__ __launch_bounds__(1024) void k_push_begin(
-    TileSpeciesSet SS, int nsp, GridDev G, TileGeom T,
-    int *__restrict__ order) {
+    TileSpeciesSet SS, int nsp, GridDev G, TileChoices TC,
+    int *__restrict__ sel, int *__restrict__ order) {
   __shared__ int est[ORDER_MAX];
   __shared__ int top, count[ORDER_CLASSES], cursor[ORDER_CLASSES];
+  __shared__ int choice;
   const int t = threadIdx.x;
   for (int k = 0; k < nsp; k++)
     if (t < 4) SS.s[k].cnt[t] = 0;
-  if (!order) return;
+  int c = 0;
+  if (TC.n > 1) {
+    const float p = densest_cells(SS, nsp, G, &choice);
+    float best = 0.0f;
+    for (int k = 0; k < TC.n; k++) {
+      const TileChoice &H = TC.c[k];
+      const float us = fmaxf(H.least, H.at0 + H.per * p);
+      if (k == 0 || us < best) {
+        best = us;
+        c = k;
+      }
+    }
+    if (t == 0) *sel = c;
+  }
+  const TileGeom &T = TC.c[c].T;
+  if (!tiles_ordered(TC.c[c].ntiles)) return;
   const int ntiles = T.ntx * T.nty * T.ntz;
   if (t == 0) top = 1;
   if (t < ORDER_CLASSES) count[t] = 0;
@@ -1226,16 +1293,16 @@ __global__ __launch_bounds__(1024) void k_push_begin(
   __syncthreads();
   const float l0 = log2f((float)top);
   auto cls = [&](int b) {
-    const int c = (int)(2.0f * (l0 - log2f((float)est[b])));
-    return min(max(c, 0), ORDER_CLASSES - 1);
+    const int k = (int)(2.0f * (l0 - log2f((float)est[b])));
+    return min(max(k, 0), ORDER_CLASSES - 1);
   };
   for (int b = t; b < ntiles; b += 1024) atomicAdd(&count[cls(b)], 1);
   __syncthreads();
   if (t == 0) {
     int at = 0;
-    for (int c = 0; c < ORDER_CLASSES; c++) {
-      cursor[c] = at;
-      at += count[c];
+    for (int k = 0; k < ORDER_CLASSES; k++) {
+      cursor[k] = at;
+      at += count[k];
     }
   }
   __syncthreads();
@@ -1767,6 +1834,27 @@ __global__ __launch_bounds__(TILE_BS, TILE_MIN_WAVES) void k_advance_p_tiled(
                             acc, wbuf, wstride, trash, G, T, Bn, OB);
 }
 
+// The same with the tile k_push_begin took; a launch has the workgroups of the
+// smallest tile, and those past the tiles taken return (a workgroup a CU that
+// takes tile after tile spills registers and was 3% slower).  A kernel of its
+// own: with one tile the geometry stays in the arguments' registers.
+template <int NSP>
+__global__ __launch_bounds__(TILE_BS, TILE_MIN_WAVES) void k_advance_p_tiled_by(
+    TileSpeciesSet SS, const vpic_interpolator_t *__restrict__ f0,
+    float *__restrict__ acc, float *__restrict__ wbuf,
+    vpic_particle_t *__restrict__ trash, GridDev G, TileChoices TC,
+    OowBuckets OB, const int *__restrict__ sel,
+    const int *__restrict__ order) {
+  const TileChoice &H = TC.c[__builtin_amdgcn_readfirstlane(*sel)];
+  if ((int)blockIdx.x >= H.ntiles) return;
+  const int tile =
+      tiles_ordered(H.ntiles) ? order[blockIdx.x] : (int)blockIdx.x;
+  const BinArgs Bn = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
+  OB.cap = H.cap;
+  tiled_push<16, 0, NSP>(__builtin_amdgcn_readfirstlane(tile), SS.s, f0, acc,
+                         wbuf, H.wstride, trash, G, H.T, Bn, OB);
+}
+
 // Add the tiles' windows into the accumulator: voxel v receives the
 // window of its own tile and, when it lies within the halo (H cells) of a
 // face of that tile, the halo of the neighbouring tiles across that face
@@ -1915,6 +2003,15 @@ __global__ __launch_bounds__(256) void k_merge_windows(
     float *__restrict__ acc, const float *__restrict__ wbuf, int wstride,
     GridDev G, TileGeom T, OowBuckets OB) {
   merge_tile(blockIdx.x, acc, wbuf, wstride, G, T, OB);
+}
+
+__global__ __launch_bounds__(256) void k_merge_windows_by(
+    float *__restrict__ acc, const float *__restrict__ wbuf, GridDev G,
+    TileChoices TC, OowBuckets OB, const int *__restrict__ sel) {
+  const TileChoice &H = TC.c[__builtin_amdgcn_readfirstlane(*sel)];
+  if ((int)blockIdx.x >= H.ntiles) return;
+  OB.cap = H.cap;
+  merge_tile(blockIdx.x, acc, wbuf, H.wstride, G, H.T, OB);
 }
 
 // --------------------------------------------------------------------------
@@ -2406,19 +2503,22 @@ bool tile_fits(int tx, int ty, int tz, int h) {
   return 96 * w + 72 * (size_t)tx * ty * tz <= (size_t)TILE_DYN_BYTES;
 }
 
-constexpr int PUSH_CUS = 256;  // compute units of the chip
-
 // Estimated microseconds of a tiled push of grid g with ppc particles per
 // cell (all species) in tiles of tx x ty x tz: a tile costs 27 us (its
 // staging, barriers and drains), 5 ns per window cell (written, then read by
 // the merge) and per particle 4.2 ns, more by 0.55 of the surface cells' share
 // (deposits outside the tile; measured 5.0 ns for 7x8x7, 5.6 for 8x8x4, 6.0
 // for 8x4x4, 6.6 for 32x2x2 at 32^3 cells, 128 per cell), one tile at a time
-// on each CU, whole tiles in whole rounds.  Between particle walls a plasma
-// is not uniform: there a tile of four times the mean density has to fit into
-// the push as well (a current sheet of 512x257 cells, 2 x 48 per cell: 709 us
-// in tiles of 32x16, 540 in tiles of 10x10).
-double tile_cost(const vpic_grid_t *g, double ppc, int tx, int ty, int tz) {
+// on each CU, whole tiles in whole rounds: `least`.  No push is faster than
+// its fullest tile, at0 + per * p us with p particles in each of its cells.
+struct TileCost {
+  double least, at0, per;
+  double at(double p) const {
+    return least > at0 + per * p ? least : at0 + per * p;
+  }
+};
+
+TileCost tile_cost(const vpic_grid_t *g, double ppc, int tx, int ty, int tz) {
   const int n[3] = {g->nx, g->ny, g->nz}, t[3] = {tx, ty, tz};
   double full = 1, all = 1, cells = 1, wcells = 1, surface = 0;
   for (int k = 0; k < 3; k++) {
@@ -2429,55 +2529,30 @@ double tile_cost(const vpic_grid_t *g, double ppc, int tx, int ty, int tz) {
     surface += n[k] > 1 ? 1.0 / t[k] : 0.0;
   }
   const double per = 4.2e-3 * (1 + 0.55 * surface);
-  const double one = 27 + 5e-3 * wcells + cells * ppc * per;
-  const double total = all * (27 + 5e-3 * wcells) +
-                       (double)g->nx * g->ny * g->nz * ppc * per;
+  TileCost c;
+  c.at0 = 27 + 5e-3 * wcells;
+  c.per = cells * per;
   double rounds = full / PUSH_CUS;
   rounds = rounds > (int)rounds ? (int)rounds + 1 : rounds;
   if (rounds < 1) rounds = 1;
-  bool walls = false;
-  for (int k = 0; k < 6; k++) walls |= g->pbc[k] != VPIC_BC_PERIODIC;
-  double bound = rounds * one;
-  const double mean = total / PUSH_CUS, dense = 27 + 4 * (one - 27);
-  if (walls && dense > bound) bound = dense;
-  return bound > mean ? bound : mean;
+  const double bound = rounds * (c.at0 + c.per * ppc);
+  const double mean =
+      (all * c.at0 + (double)g->nx * g->ny * g->nz * ppc * per) / PUSH_CUS;
+  c.least = bound > mean ? bound : mean;
+  return c;
 }
 
-// The tile of a push: the caller's, else 7x8x7 (the best of the shapes timed
-// on large grids) unless the cost above finds one 5% cheaper: on grids of
-// few tiles, where 7x8x7 leaves CUs without one (32^3 cells: 100 tiles, 277
-// us a push of 2 x 64 per cell; 8x4x4 gives every CU one, 126 us; 12x10x9
-// cells, 2 x 8 per cell: 68 to 26 us), and on 2D grids, where 7x1x7 is too
-// small to amortise a tile's fixed cost.
-// The search takes 20 to 55 us of host time, so the answers are for classes
-// of the particles per cell, an eighth of a factor of two wide, and the last
-// few are kept: a run whose particle numbers drift, or whose species go in
-// pairs of several totals, keeps its tiles and does not search at every call
-// (1.3 us a call instead of 26 at 32^3; three species on 12x10x9 cells made
-// two searches a step of 97 us, which the host could hide only while it ran
-// ahead of the GPU).
-TileGeom push_tile_for(const vpic_grid_t *g, int64_t np) {
-  if (g_tile_set) return g_tile;
-  struct Choice {
-    int nx = 0, ny = 0, nz = 0, pbc[6] = {0}, cls = 0;
-    TileGeom T;
-  };
-  constexpr int KEPT = 8;
-  static thread_local Choice kept[KEPT];
-  static thread_local int next = 0;
-  double ppc = (double)np / ((double)g->nx * g->ny * g->nz);
-  const int cls = ppc > 1.0 / 256 ? (int)lrint(8 * log2(ppc)) : -64;
-  for (const Choice &c : kept)
-    if (c.nx == g->nx && c.ny == g->ny && c.nz == g->nz && c.cls == cls &&
-        memcmp(c.pbc, g->pbc, sizeof c.pbc) == 0)
-      return c.T;
-  ppc = exp2(cls / 8.0);
+// The tile of the least cost for a plasma whose densest cells hold `dense`
+// times the mean (0: uniform): 7x8x7 (the best of the shapes timed
+// on large grids) unless another is 5% cheaper.
+TileGeom tile_search(const vpic_grid_t *g, double ppc, double dense) {
   TileGeom T = TILE_DEFAULT;
   const int mx = g->nx < 32 ? g->nx : 32, my = g->ny < 16 ? g->ny : 16,
             mz = g->nz < 16 ? g->nz : 16;
   double best = 0.95 * tile_cost(g, ppc, T.tx < g->nx ? T.tx : g->nx,
                                  T.ty < g->ny ? T.ty : g->ny,
-                                 T.tz < g->nz ? T.tz : g->nz);
+                                 T.tz < g->nz ? T.tz : g->nz)
+                           .at(dense * ppc);
   // (at least two cells along an axis that has them)
   for (int tz = mz < 2 ? mz : 2; tz <= mz; tz++)
     for (int ty = my < 2 ? my : 2; ty <= my; ty++)
@@ -2488,7 +2563,7 @@ TileGeom push_tile_for(const vpic_grid_t *g, int64_t np) {
                          (ty + (g->ny > 1 ? 2 : 0)) *
                          (tz + (g->nz > 1 ? 2 : 0));
         if ((96 + 72) * w > (size_t)TILE_DYN_BYTES) continue;
-        const double c = tile_cost(g, ppc, tx, ty, tz);
+        const double c = tile_cost(g, ppc, tx, ty, tz).at(dense * ppc);
         if (c < best) {
           best = c;
           T.tx = tx;
@@ -2496,15 +2571,85 @@ TileGeom push_tile_for(const vpic_grid_t *g, int64_t np) {
           T.tz = tz;
         }
       }
-  Choice &c = kept[next];
-  next = (next + 1) % KEPT;
-  c.nx = g->nx;
-  c.ny = g->ny;
-  c.nz = g->nz;
-  c.cls = cls;
-  memcpy(c.pbc, g->pbc, sizeof c.pbc);
-  c.T = T;
+  T.tx = T.tx < g->nx ? T.tx : g->nx;
+  T.ty = T.ty < g->ny ? T.ty : g->ny;
+  T.tz = T.tz < g->nz ? T.tz : g->nz;
   return T;
+}
+
+struct TileSet {
+  TileGeom T[TILE_CHOICES];
+  TileCost cost[TILE_CHOICES];
+  int n = 0;
+  void add(const vpic_grid_t *g, double ppc, const TileGeom &t) {
+    for (int k = 0; k < n; k++)
+      if (T[k].tx == t.tx && T[k].ty == t.ty && T[k].tz == t.tz) return;
+    T[n] = t;
+    cost[n++] = tile_cost(g, ppc, t.tx, t.ty, t.tz);
+  }
+};
+
+// The tiles of a push: the caller's, else the one of the least cost for a
+// uniform plasma.  On grids of few tiles that is smaller than 7x8x7, which
+// leaves CUs without one (32^3 cells: 100 tiles, 277
+// us a push of 2 x 64 per cell; 8x4x4 gives every CU one, 126 us; 12x10x9
+// cells, 2 x 8 per cell: 68 to 26 us); it spreads a dense region over
+// more CUs as well.  On 2D grids it is larger, since 7x1x7 is too small to
+// amortise a tile's fixed cost, and then a dense region would fall on few CUs.
+// There the push takes, by the particles it finds, that tile or the ones for
+// densities of 4 and 16 times the mean (512x257 cells, 2 x 48 per cell, 32x16,
+// 27x6 or 8x7 cells a tile; uniform: 319, 424, 569 us; 80% of the particles
+// in 0.3, 0.08, 0.02 of the cells: 530, 354, 468; 949, 593, 449; 957, 782, 516
+// us; 7x7: 595, 497, 474, 545; taken by the particles, with 8 us for looking at
+// them: 327, 365, 457, 562).
+// The search takes 20 to 55 us of host time, so the answers are for classes
+// of the particles per cell, an eighth of a factor of two wide, and the last
+// few are kept: a run whose particle numbers drift, or whose species go in
+// pairs of several totals, keeps its tiles and does not search at every call
+// (1.3 us a call instead of 26 at 32^3; three species on 12x10x9 cells made
+// two searches a step of 97 us, which the host could hide only while it ran
+// ahead of the GPU).
+TileSet push_tiles_for(const vpic_grid_t *g, int64_t np) {
+  struct Answer {
+    int nx = 0, ny = 0, nz = 0, cls = 0;
+    TileSet S;
+  };
+  constexpr int KEPT = 8;
+  static thread_local Answer kept[KEPT];
+  static thread_local int next = 0;
+  TileSet S;
+  double ppc = (double)np / ((double)g->nx * g->ny * g->nz);
+  if (g_tile_set) {
+    TileGeom T = g_tile;
+    T.tx = T.tx < g->nx ? T.tx : g->nx;
+    T.ty = T.ty < g->ny ? T.ty : g->ny;
+    T.tz = T.tz < g->nz ? T.tz : g->nz;
+    S.add(g, ppc, T);
+    return S;
+  }
+  const int cls = ppc > 1.0 / 256 ? (int)lrint(8 * log2(ppc)) : -64;
+  for (const Answer &a : kept)
+    if (a.nx == g->nx && a.ny == g->ny && a.nz == g->nz && a.cls == cls)
+      return a.S;
+  ppc = exp2(cls / 8.0);
+  const TileGeom T = tile_search(g, ppc, 0);
+  S.add(g, ppc, T);
+  const TileGeom &D = TILE_DEFAULT;
+  const int fixed = (D.tx < g->nx ? D.tx : g->nx) *
+                    (D.ty < g->ny ? D.ty : g->ny) *
+                    (D.tz < g->nz ? D.tz : g->nz);
+  if (8 * T.tx * T.ty * T.tz > 9 * fixed) {
+    S.add(g, ppc, tile_search(g, ppc, 4));
+    S.add(g, ppc, tile_search(g, ppc, 16));
+  }
+  Answer &a = kept[next];
+  next = (next + 1) % KEPT;
+  a.nx = g->nx;
+  a.ny = g->ny;
+  a.nz = g->nz;
+  a.cls = cls;
+  a.S = S;
+  return S;
 }
 
 }  // namespace
@@ -2534,12 +2679,14 @@ void push_get_tile(int out[4]) {
 }
 
 int push_tile_choices(const vpic_grid_t *g, int64_t np, int *out) {
-  const TileGeom T = push_tile_for(g, np);
-  out[0] = T.tx < g->nx ? T.tx : g->nx;
-  out[1] = T.ty < g->ny ? T.ty : g->ny;
-  out[2] = T.tz < g->nz ? T.tz : g->nz;
-  out[3] = T.halo;
-  return 1;
+  const TileSet S = push_tiles_for(g, np);
+  for (int k = 0; k < S.n; k++) {
+    out[4 * k] = S.T[k].tx;
+    out[4 * k + 1] = S.T[k].ty;
+    out[4 * k + 2] = S.T[k].tz;
+    out[4 * k + 3] = S.T[k].halo;
+  }
+  return S.n;
 }
 
 int push_set_group(int gs) {
@@ -2706,6 +2853,56 @@ int launch_advance_p(vpic_particle_t *p, int np, float q, float m,
   return launch_advance_p_set(1, &one, a, f, g, s);
 }
 
+namespace {
+
+// What a launch with tile H.T (cut to the grid) needs: the rest of the
+// geometry, the tiles, the window's floats, the records of a sub-bucket and
+// the dynamic LDS.
+int tile_launch(const vpic_grid_t *g, int64_t np, TileChoice &H, size_t &lds) {
+  // (a 2D grid's tiles are one cell thick; the window then has no halo
+  // along that axis either)
+  TileGeom &T = H.T;
+  T.ntx = (g->nx + T.tx - 1) / T.tx;
+  T.nty = (g->ny + T.ty - 1) / T.ty;
+  T.ntz = (g->nz + T.tz - 1) / T.tz;
+  const unsigned sx1 = g->nx + 2, sy1 = g->ny + 2;
+  const bool magic_ok = (uint64_t)g->nv * sx1 < ((uint64_t)1 << 32);
+  T.mx = magic_ok ? div_magic(sx1) : 0;
+  T.my = magic_ok ? div_magic(sy1) : 0;
+  tile_axis_halos(T, g);
+  const size_t wcells = tile_window(T);
+  const size_t win_bytes = sizeof(unsigned long long) * 12 * wcells;
+  const size_t scells = tile_ring(T);
+  if (win_bytes + 72 * (size_t)T.tx * T.ty * T.tz > (size_t)TILE_DYN_BYTES)
+    return vpic_set_error(VPIC_EINVAL,
+                          "advance_p: push tile %dx%dx%d with halo %d "
+                          "needs %zu window cells on this grid, more "
+                          "than the LDS holds", T.tx, T.ty, T.tz, T.halo,
+                          wcells);
+  T.stage_win = win_bytes + 72 * scells <= (size_t)TILE_DYN_BYTES;
+  lds = win_bytes + 72 * (T.stage_win ? scells : (size_t)T.tx * T.ty * T.tz);
+  H.ntiles = T.ntx * T.nty * T.ntz;
+  H.wstride = (int)(12 * wcells);
+  // Sub-buckets for out-of-window deposits: 27 per tile of 1/32 of a
+  // tile's average particle count (all species) each (late in a sort
+  // interval about a tenth of the electrons' deposits leave their
+  // window, mostly across the six faces), 64 to 4096 records; a tile's
+  // whole count when that takes at most 256 MiB (small grids, whose
+  // narrow or periodic-edge tiles can send most of their deposits to
+  // one neighbour).  A deposit that finds its sub-bucket full takes a
+  // float atomic.  Every tiled push writes all 27 counts of every
+  // tile, so they need no clearing.
+  const int64_t per_tile = np / H.ntiles + 1;
+  int64_t cap = per_tile / 32;
+  cap = cap < 64 ? 64 : cap > 4096 ? 4096 : cap;
+  if (64 * 27 * per_tile * H.ntiles <= ((int64_t)256 << 20) && per_tile > cap)
+    cap = per_tile;
+  H.cap = (int)cap;
+  return VPIC_OK;
+}
+
+}  // namespace
+
 // advance_p of nsp species into one accumulator.  Species that all have a
 // sort-time partition share one tiled launch (the same windows, staged
 // coefficients and merge, the species pushed in turn by every tile);
@@ -2767,64 +2964,43 @@ int launch_advance_p_set(int nsp, const vpic_push_species_t *sp,
     vpic_particle_t *p = sp[0].p;
     const int np = sp[0].np;
     const int *partition = sp[0].partition;
-    TileGeom T = push_tile_for(g, np_total);
-    // a tile no larger than the grid (a 2D grid's tiles are one cell
-    // thick; the window then has no halo along that axis either)
-    T.tx = T.tx < g->nx ? T.tx : g->nx;
-    T.ty = T.ty < g->ny ? T.ty : g->ny;
-    T.tz = T.tz < g->nz ? T.tz : g->nz;
-    T.ntx = (g->nx + T.tx - 1) / T.tx;
-    T.nty = (g->ny + T.ty - 1) / T.ty;
-    T.ntz = (g->nz + T.tz - 1) / T.tz;
-    const unsigned sx1 = g->nx + 2, sy1 = g->ny + 2;
-    const bool magic_ok = (uint64_t)g->nv * sx1 < ((uint64_t)1 << 32);
-    T.mx = magic_ok ? div_magic(sx1) : 0;
-    T.my = magic_ok ? div_magic(sy1) : 0;
-    tile_axis_halos(T, g);
-    const size_t wcells = tile_window(T);
-    const size_t win_bytes = sizeof(unsigned long long) * 12 * wcells;
-    const size_t scells = tile_ring(T);
-    if (win_bytes + 72 * (size_t)T.tx * T.ty * T.tz > (size_t)TILE_DYN_BYTES)
-      return vpic_set_error(VPIC_EINVAL,
-                            "advance_p: push tile %dx%dx%d with halo %d "
-                            "needs %zu window cells on this grid, more "
-                            "than the LDS holds", T.tx, T.ty, T.tz, T.halo,
-                            wcells);
-    T.stage_win = win_bytes + 72 * scells <= (size_t)TILE_DYN_BYTES;
-    const size_t lds =
-        win_bytes +
-        72 * (T.stage_win ? scells : (size_t)T.tx * T.ty * T.tz);
-    const int nblk = T.ntx * T.nty * T.ntz;
-    const int wstride = (int)(12 * wcells);
-    if ((rc = scratch_reserve(S.wbuf, sizeof(float) * (size_t)wstride *
-                                          (size_t)nblk)))
-      return rc;
+    const TileSet tiles = push_tiles_for(g, np_total);
+    // (tile lists, and lane groups of another size, know one tile: the one
+    // that copes with dense regions)
+    const bool lists = g_bin_mode > 0 && nsp == 1;
+    const int first = tiles.n > 1 && (lists || g_group != 16) ? tiles.n - 1 : 0;
+    TileChoices TC = {};
+    int nblk = 0;  // of the smallest tile
+    size_t lds = 0, wbytes = 0, nrec = 0;
+    bool ordered = false;
+    for (int k = first; k < tiles.n; k++) {
+      TileChoice &H = TC.c[TC.n++];
+      size_t need;
+      H.T = tiles.T[k];
+      if ((rc = tile_launch(g, np_total, H, need))) return rc;
+      H.least = (float)tiles.cost[k].least;
+      H.at0 = (float)tiles.cost[k].at0;
+      H.per = (float)tiles.cost[k].per;
+      const size_t w = sizeof(float) * (size_t)H.wstride * H.ntiles;
+      const size_t r = (size_t)H.cap * H.ntiles;
+      nblk = nblk > H.ntiles ? nblk : H.ntiles;
+      lds = lds > need ? lds : need;
+      wbytes = wbytes > w ? wbytes : w;
+      nrec = nrec > r ? nrec : r;
+      ordered = ordered || tiles_ordered(H.ntiles);
+    }
+    const TileGeom &T = TC.c[0].T;
+    const int wstride = TC.c[0].wstride;
+    if ((rc = scratch_reserve(S.wbuf, wbytes))) return rc;
     if ((rc = scratch_reserve(S.trash, sizeof(vpic_particle_t) * TILE_BS)))
       return rc;
-    // Sub-buckets for out-of-window deposits: 27 per tile of 1/32 of a
-    // tile's average particle count (all species) each (late in a sort
-    // interval about a tenth of the electrons' deposits leave their
-    // window, mostly across the six faces), 64 to 4096 records; a tile's
-    // whole count when that takes at most 256 MiB (small grids, whose
-    // narrow or periodic-edge tiles can send most of their deposits to
-    // one neighbour).  A deposit that finds its sub-bucket full takes a
-    // float atomic.  Every tiled push writes all 27 counts of every
-    // tile, so they need no clearing.
     OowBuckets OB;
-    {
-      const int64_t per_tile = np_total / nblk + 1;
-      int64_t cap = per_tile / 32;
-      cap = cap < 64 ? 64 : cap > 4096 ? 4096 : cap;
-      if (64 * 27 * per_tile * nblk <= ((int64_t)256 << 20) && per_tile > cap)
-        cap = per_tile;
-      if ((rc = scratch_reserve(S.ocnt, sizeof(int) * 54 * (size_t)nblk)) ||
-          (rc = scratch_reserve(S.orec,
-                                64 * 27 * (size_t)cap * (size_t)nblk)))
-        return rc;
-      OB.cnt = (int *)S.ocnt.ptr;
-      OB.rec = (float4 *)S.orec.ptr;
-      OB.cap = (int)cap;
-    }
+    if ((rc = scratch_reserve(S.ocnt, sizeof(int) * 54 * (size_t)nblk)) ||
+        (rc = scratch_reserve(S.orec, 64 * 27 * nrec)))
+      return rc;
+    OB.cnt = (int *)S.ocnt.ptr;
+    OB.rec = (float4 *)S.orec.ptr;
+    OB.cap = TC.c[0].cap;
     static bool attr_set[TILE_MAXSP][7] = {};
     const int ak = tiled_kernel_id(g_group);
     if (!attr_set[nsp - 1][ak]) {
@@ -2832,12 +3008,16 @@ int launch_advance_p_set(int nsp, const vpic_push_species_t *sp,
         VPIC_HIP(hipFuncSetAttribute(
             reinterpret_cast<const void *>(tiled_kernel(g_group, mode, nsp)),
             hipFuncAttributeMaxDynamicSharedMemorySize, TILE_DYN_BYTES));
+      VPIC_HIP(hipFuncSetAttribute(
+          nsp == 1 ? reinterpret_cast<const void *>(k_advance_p_tiled_by<1>)
+                   : reinterpret_cast<const void *>(k_advance_p_tiled_by<2>),
+          hipFuncAttributeMaxDynamicSharedMemorySize, TILE_DYN_BYTES));
       attr_set[nsp - 1][ak] = true;
     }
     // Tile lists from the codes of the last tiled push of this array.
     BinArgs BA = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
     BinState *BSt = nullptr;
-    if (g_bin_mode > 0 && nsp == 1) {
+    if (lists) {
       BinState &B = bin_state(S, p);
       const int nt = nblk;
       const int nsum = (nt + 1 + 2047) / 2048 + 1;
@@ -2899,26 +3079,36 @@ int launch_advance_p_set(int nsp, const vpic_push_species_t *sp,
     for (int k = 0; k < nsp; k++)
       SS.s[k] = {sp[k].p, sp[k].partition, rlist[k], cnt[k], sp[k].keys,
                  C[k], sp[k].np, xcap[k]};
-    // fullest tiles first, where some CU gets more than one
-    int *order = nullptr;
-    if (nblk > PUSH_CUS && nblk <= ORDER_MAX) {
-      if ((rc = scratch_reserve(S.order, sizeof(int) * (size_t)nblk)))
+    // the tile taken, then the tiles, fullest first, where some CU gets more
+    // than one
+    int *sel = nullptr, *order = nullptr;
+    if (ordered || TC.n > 1) {
+      if ((rc = scratch_reserve(S.order, sizeof(int) * (ORDER_MAX + 1))))
         return rc;
+      sel = (int *)S.order.ptr + ORDER_MAX;
       order = (int *)S.order.ptr;
     }
-    hipLaunchKernelGGL(k_push_begin, dim3(1), dim3(1024), 0, s, SS, nsp, G, T,
-                       order);
+    hipLaunchKernelGGL(k_push_begin, dim3(1), dim3(1024), 0, s, SS, nsp, G, TC,
+                       sel, order);
     VPIC_LAUNCHED("k_push_begin");
     if (timed) push_timing_record(s, np_total, true);
     // without binning only the mode-0 instance; with it all three, of
     // which the one matching the device's binning state runs
-    for (int mode = 0; mode < (BSt ? 3 : 1); mode++) {
+    for (int mode = 0; mode < (BSt ? 3 : 1) && TC.n == 1; mode++) {
       hipLaunchKernelGGL(tiled_kernel(g_group, mode, nsp), dim3(nblk),
                          dim3(TILE_BS), lds, s, SS, f, (float *)a,
                          (float *)S.wbuf.ptr, wstride,
                          (vpic_particle_t *)S.trash.ptr, G, T, BA, OB,
-                         (const int *)order);
+                         (const int *)(ordered ? order : nullptr));
       VPIC_LAUNCHED("k_advance_p_tiled");
+    }
+    if (TC.n > 1) {
+      hipLaunchKernelGGL((nsp == 1 ? k_advance_p_tiled_by<1>
+                                   : k_advance_p_tiled_by<2>),
+                         dim3(nblk), dim3(TILE_BS), lds, s, SS, f, (float *)a,
+                         (float *)S.wbuf.ptr, (vpic_particle_t *)S.trash.ptr,
+                         G, TC, OB, (const int *)sel, (const int *)order);
+      VPIC_LAUNCHED("k_advance_p_tiled_by");
     }
     if (timed) push_timing_record(s, np_total, false);
     if (BSt) {
@@ -2927,9 +3117,14 @@ int launch_advance_p_set(int nsp, const vpic_push_species_t *sp,
       VPIC_LAUNCHED("k_bin_post");
       BSt->cur ^= 1;
     }
-    hipLaunchKernelGGL(k_merge_windows, dim3(nblk), dim3(256), 0, s,
-                       (float *)a, (const float *)S.wbuf.ptr, wstride, G, T,
-                       OB);
+    if (TC.n == 1)
+      hipLaunchKernelGGL(k_merge_windows, dim3(nblk), dim3(256), 0, s,
+                         (float *)a, (const float *)S.wbuf.ptr, wstride, G, T,
+                         OB);
+    else
+      hipLaunchKernelGGL(k_merge_windows_by, dim3(nblk), dim3(256), 0, s,
+                         (float *)a, (const float *)S.wbuf.ptr, G, TC, OB,
+                         (const int *)sel);
     VPIC_LAUNCHED("k_merge_windows");
     // particles past the partition (added since the sort) go flat
     int most = 0;
