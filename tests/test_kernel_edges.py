@@ -220,10 +220,12 @@ def test_accumulate_rho_chunks(dev, n, np_, order):
 
 
 # one particle; 16 lanes of one voxel and one more; few particles over a grid
-# of two slabs of voxels; axes of one cell; an axis too long to sort by
+# of two slabs of voxels; planes just below and above half a slab, and far above;
+# axes of one cell; an axis too long to sort by
 @pytest.mark.parametrize("n,np_", [
     ((4, 3, 5), 1), ((2, 1, 2), 16 * 4 + 1), ((9, 8, 7), 12000),
-    ((70, 70, 63), 30000), ((33, 1, 20), 5000), ((2100, 1, 1), 4000)],
+    ((70, 70, 63), 30000), ((385, 384, 3), 60000), ((386, 384, 3), 60000),
+    ((900, 700, 1), 50000), ((33, 1, 20), 5000), ((2100, 1, 1), 4000)],
     ids=lambda v: str(v).replace(" ", ""))
 def test_hydro_voxel_sums(dev, orc, n, np_):
     """The moments of particles in no order against the oracle's, within the
@@ -247,8 +249,13 @@ def test_hydro_voxel_sums(dev, orc, n, np_):
     orc.accumulate_hydro_p(want, p, -1.0, 1.0, fi, g)
     dp, dfi = dev.DeviceArray.from_host(p), dev.DeviceArray.from_host(fi)
     say("accumulate_hydro_p", n, np_)
+    import torch
+    free = torch.cuda.mem_get_info()[0]
     _lib.call("vpic_hip_accumulate_hydro_p", dh.ptr, dp.ptr, np_, -1.0, 1.0,
               dfi.ptr, ctypes.byref(g), None, None)
+    # (scratch: 128 MiB of sums, an eighth more, and what a particle and a
+    # voxel take)
+    assert free - torch.cuda.mem_get_info()[0] < 200 << 20
     got = dh.download()
     for k in T.HYDRO_FIELDS:
         assert np.max(np.abs(got[k] - want[k])) <= \

@@ -29,9 +29,9 @@ struct HydroCoef {
 
 constexpr int HY_LANES = 16;  // lanes per voxel (one DPP row)
 constexpr int HY_SUMS = 8 * 14;
-// Slabs of voxels whose sums (448 B each) stay in the 256-MB cache between
-// the kernel that writes them and the one that reads them.
-constexpr int64_t HY_SLAB_BYTES = (int64_t)128 << 20;
+// Voxels whose sums (448 B each, 128 MiB in all) stay in the 256-MB cache
+// between the kernel that writes them and the one that reads them.
+constexpr int64_t HY_VOXELS = ((int64_t)128 << 20) / (4 * HY_SUMS);
 
 // The per-particle part of accumulate_hydro_p_pipeline_scalar
 // (hydro_p_pipeline.cc:65-172): node weights wn[8] and the 14 moments per
@@ -237,11 +237,13 @@ __global__ __launch_bounds__(256) void k_hydro_cells(
   }
 }
 
-// Nodes [n0, n1): 16 lanes each, one per moment, gather the eight voxels
-// (from v0 on in sums) a node belongs to.
+// Nodes [n0, n1): 16 lanes each, one per moment, gather the eight voxels a node
+// belongs to: voxel v of the node's own plane is at sums[112 (v - vu)], of the
+// plane below at sums[112 (v - vl)].
 __global__ __launch_bounds__(256) void k_hydro_nodes(
     const float *__restrict__ sums, const int *__restrict__ start,
-    float *__restrict__ hy, int v0, int vmax, int n0, int n1, int sy, int sz) {
+    float *__restrict__ hy, int vl, int vu, int vmax, int n0, int n1, int sy,
+    int sz) {
   const int c = threadIdx.x & 15;
   const int n = n0 + (int)((blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >>
                            4);
@@ -253,7 +255,7 @@ __global__ __launch_bounds__(256) void k_hydro_nodes(
     const int v = n - node_off(k, sy, sz);
     if (v < 0 || v >= vmax || start[v] == start[v + 1]) continue;
     any = true;
-    s += sums[(int64_t)(v - v0) * HY_SUMS + 14 * k + c];
+    s += sums[((int64_t)v - (k < 4 ? vu : vl)) * HY_SUMS + 14 * k + c];
   }
   if (any) hy[16 * (int64_t)n + c] += s;
 }
@@ -360,15 +362,21 @@ int launch_accumulate_hydro_p(vpic_hydro_t *h, const vpic_particle_t *p,
                        (float *)h, C, g->nv, g->sy, g->sz, nbad);
     VPIC_LAUNCHED("k_hydro_flat");
   } else if (np > 0) {
-    // nodes per slab; their voxels reach back by one plane, row and cell
-    const int back = g->sz + g->sy + 1;
-    int64_t slab = HY_SLAB_BYTES / (4 * HY_SUMS) - back;
-    if (slab < back) slab = back;
+    // Nodes per slab.  Their voxels reach back by a plane, a row and a cell:
+    // one range of voxels, as long as what it reaches back by is at most half
+    // of it, or on larger planes (of more than 150,000 voxels) two, a row and a
+    // cell longer than the slab each.  A voxel of two slabs is summed for both
+    // (1500x1500x2 cells, 4 a cell: 6.5 ms, with particle-by-particle atomics
+    // 13.9).
+    const int row = g->sy + 1, back = g->sz + row;
+    const bool two = 2 * (int64_t)back > HY_VOXELS;
+    int64_t slab = two ? HY_VOXELS / 2 - row : HY_VOXELS - back;
     if (slab > g->nv) slab = g->nv;
     if ((rc = scratch_reserve(S.keys, sizeof(int) * (size_t)np)) ||
         (rc = scratch_reserve(S.start, sizeof(int) * ((size_t)g->nv + 1))) ||
         (rc = scratch_reserve(S.sums, sizeof(float) * HY_SUMS *
-                                          (size_t)(slab + back))))
+                                          (size_t)(two ? 2 * (slab + row)
+                                                       : slab + back))))
       return rc;
     int *keys = (int *)S.keys.ptr, *start = (int *)S.start.ptr;
     float *sums = (float *)S.sums.ptr;
@@ -386,18 +394,32 @@ int launch_accumulate_hydro_p(vpic_hydro_t *h, const vpic_particle_t *p,
     VPIC_LAUNCHED("k_hydro_starts");
     for (int64_t n0 = 0; n0 < g->nv; n0 += slab) {
       const int64_t n1 = n0 + slab < g->nv ? n0 + slab : g->nv;
-      const int64_t v0 = n0 > back ? n0 - back : 0;
-      const int64_t v1 = n1 < vmax ? n1 : vmax;
-      if (v1 <= v0) continue;
-      hipLaunchKernelGGL(k_hydro_cells,
-                         dim3(blocks_for((v1 - v0) * HY_LANES, 256)),
-                         dim3(256), 0, s, p, (const int *)order,
-                         (const int *)start, f, sums, C, (int)v0, (int)v1);
+      // voxels [v0, v1) to sums from voxel `at` on; none when there are none
+      auto cells = [&](int64_t v0, int64_t v1, int64_t at) {
+        if (v0 < 0) v0 = 0;
+        if (v1 > vmax) v1 = vmax;
+        if (v1 <= v0) return;
+        hipLaunchKernelGGL(k_hydro_cells,
+                           dim3(blocks_for((v1 - v0) * HY_LANES, 256)),
+                           dim3(256), 0, s, p, (const int *)order,
+                           (const int *)start, f, sums + (v0 - at) * HY_SUMS,
+                           C, (int)v0, (int)v1);
+      };
+      // the voxel at the start of sums for the plane below and the node's own
+      int64_t vl = n0 - back, vu = vl;
+      if (two) {
+        cells(n0 - back, n1 - g->sz, vl);
+        VPIC_LAUNCHED("k_hydro_cells");
+        vu = n0 - row - (slab + row);
+        cells(n0 - row, n1, vu);
+      } else {
+        cells(n0 - back, n1, vl);
+      }
       VPIC_LAUNCHED("k_hydro_cells");
       hipLaunchKernelGGL(k_hydro_nodes, dim3(blocks_for((n1 - n0) * 16, 256)),
                          dim3(256), 0, s, (const float *)sums,
-                         (const int *)start, (float *)h, (int)v0, vmax,
-                         (int)n0, (int)n1, g->sy, g->sz);
+                         (const int *)start, (float *)h, (int)vl, (int)vu,
+                         vmax, (int)n0, (int)n1, g->sy, g->sz);
       VPIC_LAUNCHED("k_hydro_nodes");
     }
   }
