@@ -167,7 +167,12 @@ const char *vpic_hip_version(void);
  * share.  Calls that return with work queued are ordered by their stream: the
  * sorts (and the calls that sort: accumulate_hydro_p, the adjoint run) also
  * wait for the thread's sort before them on another stream; pushes of one
- * thread belong on one stream, or in order across streams. */
+ * thread belong on one stream, or in order across streams.
+ * vpic_hip_scratch_limit: the most bytes a scratch array of this thread may
+ * take (0, as at the start: no limit).  A call that needs more, or for which
+ * the GPU has no more, does without where it can (accumulate_hydro_p) and
+ * fails with VPIC_ENOMEM otherwise. */
+int vpic_hip_scratch_limit(int64_t bytes);
 
 /* ------------------------------------------------------------------------ */
 /* Species advance (src/species_advance/species_advance.h:64-157)          */
@@ -610,11 +615,12 @@ int vpic_hip_clear_hydro_array(vpic_hydro_t *h, const vpic_grid_t *g,
 
 /* accumulate_hydro_p (hydro_p.cc:12-19 -> hydro_p_pipeline.cc:17-242):
  * adds the 14 moments of p[0..np) to the nodes, trilinear weights.  The
- * particles' indices are sorted by voxel (in scratch of 16 bytes a particle
- * and 448 bytes a voxel of a slab; any order of the particles will do, and
- * `partition` is not needed), each voxel's moments are summed in registers
- * and the nodes gather them; grids with an axis of more than 2046 cells take
- * the particles one by one.  The per-particle arithmetic is the reference's;
+ * particles' indices are sorted by voxel (any order of the particles will do,
+ * and `partition` is not needed), each voxel's moments are summed in registers
+ * and the nodes gather them.  That takes scratch of 20 bytes a particle, 4 a
+ * voxel, at most 128 MiB of sums and 16 MiB of counts, which the thread keeps.
+ * Where it is not there, and on grids with an axis of more than 2046 cells, the
+ * particles go one by one.  The per-particle arithmetic is the reference's;
  * the sums differ only in order.  Synchronous; particles whose voxel is not
  * interior are skipped and reported as an error.  reduce_hydro_array has
  * nothing to do (one device copy). */

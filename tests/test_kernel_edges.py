@@ -498,3 +498,45 @@ def test_sort_scratch_across_streams(dev):
             assert np.max(np.abs(got - want)) <= 1e-10 * np.max(np.abs(want))
         else:
             assert H.same_bits(got, want)
+
+
+@pytest.mark.parametrize("limit", [16000, 40000])
+def test_hydro_without_scratch(dev, orc, limit):
+    """Where the scratch of the sorted sums is not there (the particles' keys;
+    the voxels' sums) the particles go one by one, with the oracle's moments
+    and each bad voxel counted once."""
+    g = _box(3, 2, 3)
+    np_ = 7000
+    rng = np.random.default_rng(4)
+    fi = H.interp_array(g)
+    orc.load_interpolator(fi, H.random_fields(g, 4, 0.1, 0.2), g)
+    p = np.zeros(np_, dtype=T.PARTICLE)
+    p["i"] = g.voxel(*(rng.integers(1, k + 1, np_)
+                       for k in (g.nx, g.ny, g.nz)))
+    p["dx"] = rng.uniform(-1, 1, np_).astype(np.float32)
+    p["ux"] = (0.3 * rng.standard_normal(np_)).astype(np.float32)
+    p["w"] = 1.0
+    want = np.zeros(g.nv, dtype=T.HYDRO)
+    orc.accumulate_hydro_p(want, p, -1.0, 1.0, fi, g)
+    bad = p.copy()
+    bad["i"][5] = g.nv - 2
+    dfi = dev.DeviceArray.from_host(fi)
+
+    def moments(q):
+        dh = dev.DeviceArray((g.nv,), T.HYDRO)
+        dh.zero()
+        dp = dev.DeviceArray.from_host(q)
+        _lib.call("vpic_hip_accumulate_hydro_p", dh.ptr, dp.ptr, np_, -1.0,
+                  1.0, dfi.ptr, ctypes.byref(g), None, None)
+        return dh.download()
+    say("accumulate_hydro_p, scratch limit", limit)
+    try:
+        _lib.call("vpic_hip_scratch_limit", limit)
+        got = moments(p)
+        with pytest.raises(_lib.VpicError, match="1 particles"):
+            moments(bad)
+    finally:
+        _lib.call("vpic_hip_scratch_limit", 0)
+    for k in T.HYDRO_FIELDS:
+        assert np.max(np.abs(got[k] - want[k])) <= \
+            1e-5 * max(np.max(np.abs(want[k])), 1e-30), k

@@ -38,6 +38,7 @@ _SIGS = {
     "vpic_hip_device_synchronize": [],
     "vpic_hip_push_tile": [_i32, _i32, _i32],
     "vpic_hip_push_tile_window": [_i32, _i32, _i32, _i32],
+    "vpic_hip_scratch_limit": [_i64],
     "vpic_hip_push_get_tile": [_vp],
     "vpic_hip_push_tile_choices": [_pg, _i64, _vp, _pi32],
     "vpic_hip_push_direct_runs": [_i32],

@@ -29,7 +29,14 @@ int vpic_check_hip(hipError_t e, const char *what) {
   return vpic_set_error(VPIC_EHIP, "%s: %s", what, hipGetErrorString(e));
 }
 
+// The most a scratch array of this thread may take (0: no limit).
+static thread_local int64_t g_scratch_limit = 0;
+
 int scratch_reserve(DeviceScratch &s, size_t bytes) {
+  if (g_scratch_limit > 0 && bytes > (size_t)g_scratch_limit)
+    return vpic_set_error(VPIC_ENOMEM, "%zu bytes of scratch are more than "
+                          "the limit of %lld", bytes,
+                          (long long)g_scratch_limit);
   if (bytes <= s.bytes && s.ptr) return VPIC_OK;
   if (s.ptr) {
     hipError_t e = hipFree(s.ptr);
@@ -41,6 +48,7 @@ int scratch_reserve(DeviceScratch &s, size_t bytes) {
   hipError_t e = hipMalloc(&s.ptr, want);
   if (e != hipSuccess) {
     s.ptr = nullptr;
+    (void)hipGetLastError();  // (the launches that follow are not to see it)
     return vpic_set_error(VPIC_ENOMEM, "hipMalloc(%zu bytes of scratch): %s",
                           want, hipGetErrorString(e));
   }
@@ -242,6 +250,12 @@ extern "C" int vpic_hip_push_group(int32_t gs) {
 extern "C" int vpic_hip_push_bin_mode(int32_t mode) {
   CHECK(push_set_bin_mode(mode) == VPIC_OK,
         "push bin mode %d not one of 0, 1, 2", mode);
+  return VPIC_OK;
+}
+
+extern "C" int vpic_hip_scratch_limit(int64_t bytes) {
+  CHECK(bytes >= 0, "scratch limit below 0");
+  g_scratch_limit = bytes;
   return VPIC_OK;
 }
 

@@ -17,8 +17,8 @@
 // eight it takes.  No atomics.  1.5e7 particles on 72x64x50 cells that drifted
 // by half a cell since the sort: 0.77 ms, of which the sort is 0.33 (6.5
 // ms with LDS windows per tile, whose float atomics a drifted particle needs
-// one by one).  Grids with an axis too long for that sort go particle by
-// particle with global atomics.
+// one by one).  Grids with an axis too long for that sort, and calls for which
+// its memory is not there, go particle by particle with global atomics.
 #include "common.h"
 
 namespace {
@@ -319,6 +319,77 @@ HydroScratch &hydro_scratch() {
 
 inline int blocks_for(int64_t n, int bs) { return (int)((n + bs - 1) / bs); }
 
+// The sums of all particles by sorted voxels; VPIC_ENOMEM, with nothing added
+// to the moments, when its memory is not there.  (vmax: voxels whose eight
+// nodes lie on the grid.)
+int hydro_sorted(HydroScratch &S, SortScratchUse &use, vpic_hydro_t *h,
+                 const vpic_particle_t *p, int np,
+                 const vpic_interpolator_t *f, const vpic_grid_t *g,
+                 const HydroCoef &C, int vmax, int *nbad, hipStream_t s) {
+  int rc;
+  // Nodes per slab.  Their voxels reach back by a plane, a row and a cell:
+  // one range of voxels, as long as what it reaches back by is at most half
+  // of it, or on larger planes (of more than 150,000 voxels) two, a row and a
+  // cell longer than the slab each.  A voxel of two slabs is summed for both
+  // (1500x1500x2 cells, 4 a cell: 6.5 ms, with particle-by-particle atomics
+  // 13.9).
+  const int row = g->sy + 1, back = g->sz + row;
+  const bool two = 2 * (int64_t)back > HY_VOXELS;
+  int64_t slab = two ? HY_VOXELS / 2 - row : HY_VOXELS - back;
+  if (slab > g->nv) slab = g->nv;
+  if ((rc = scratch_reserve(S.keys, sizeof(int) * (size_t)np)) ||
+      (rc = scratch_reserve(S.start, sizeof(int) * ((size_t)g->nv + 1))) ||
+      (rc = scratch_reserve(S.sums, sizeof(float) * HY_SUMS *
+                                        (size_t)(two ? 2 * (slab + row)
+                                                     : slab + back))))
+    return rc;
+  int *keys = (int *)S.keys.ptr, *start = (int *)S.start.ptr;
+  float *sums = (float *)S.sums.ptr;
+  int nb = blocks_for(np, 256);
+  if (nb > 8192) nb = 8192;
+  hipLaunchKernelGGL(k_hydro_keys, dim3(nb), dim3(256), 0, s, p, np, vmax,
+                     g->nv, keys, nbad);
+  VPIC_LAUNCHED("k_hydro_keys");
+  int *order, *sorted;
+  if ((rc = use.begin(s)) ||
+      (rc = device_sort_keys(keys, np, g, &order, &sorted, nullptr, use, s)))
+    return rc;
+  hipLaunchKernelGGL(k_hydro_starts, dim3(blocks_for((int64_t)g->nv + 1, 256)),
+                     dim3(256), 0, s, (const int *)sorted, np, g->nv, start);
+  VPIC_LAUNCHED("k_hydro_starts");
+  for (int64_t n0 = 0; n0 < g->nv; n0 += slab) {
+    const int64_t n1 = n0 + slab < g->nv ? n0 + slab : g->nv;
+    // voxels [v0, v1) to sums from voxel `at` on; none when there are none
+    auto cells = [&](int64_t v0, int64_t v1, int64_t at) {
+      if (v0 < 0) v0 = 0;
+      if (v1 > vmax) v1 = vmax;
+      if (v1 <= v0) return;
+      hipLaunchKernelGGL(k_hydro_cells,
+                         dim3(blocks_for((v1 - v0) * HY_LANES, 256)),
+                         dim3(256), 0, s, p, (const int *)order,
+                         (const int *)start, f, sums + (v0 - at) * HY_SUMS,
+                         C, (int)v0, (int)v1);
+    };
+    // the voxel at the start of sums for the plane below and the node's own
+    int64_t vl = n0 - back, vu = vl;
+    if (two) {
+      cells(n0 - back, n1 - g->sz, vl);
+      VPIC_LAUNCHED("k_hydro_cells");
+      vu = n0 - row - (slab + row);
+      cells(n0 - row, n1, vu);
+    } else {
+      cells(n0 - back, n1, vl);
+    }
+    VPIC_LAUNCHED("k_hydro_cells");
+    hipLaunchKernelGGL(k_hydro_nodes, dim3(blocks_for((n1 - n0) * 16, 256)),
+                       dim3(256), 0, s, (const float *)sums,
+                       (const int *)start, (float *)h, (int)vl, (int)vu,
+                       vmax, (int)n0, (int)n1, g->sy, g->sz);
+    VPIC_LAUNCHED("k_hydro_nodes");
+  }
+  return VPIC_OK;
+}
+
 }  // namespace
 
 int launch_clear_hydro(vpic_hydro_t *h, const vpic_grid_t *g, hipStream_t s) {
@@ -355,73 +426,21 @@ int launch_accumulate_hydro_p(vpic_hydro_t *h, const vpic_particle_t *p,
   SortScratchUse use;
   // voxels whose eight nodes lie on the grid
   const int vmax = g->nv - g->sz - g->sy - 1;
-  if (np > 0 && !sort_keys_fit(g)) {
+  rc = VPIC_ENOMEM;
+  if (np > 0 && sort_keys_fit(g)) {
+    rc = hydro_sorted(S, use, h, p, np, f, g, C, vmax, nbad, s);
+    if (rc && rc != VPIC_ENOMEM) return rc;
+    if (rc) {
+      hipLaunchKernelGGL(k_hydro_clear_count, dim3(1), dim3(64), 0, s, nbad);
+      VPIC_LAUNCHED("k_hydro_clear_count");
+    }
+  }
+  if (np > 0 && rc) {
     int nb = blocks_for(np, 256);
     if (nb > 16384) nb = 16384;
     hipLaunchKernelGGL(k_hydro_flat, dim3(nb), dim3(256), 0, s, p, np, f,
                        (float *)h, C, g->nv, g->sy, g->sz, nbad);
     VPIC_LAUNCHED("k_hydro_flat");
-  } else if (np > 0) {
-    // Nodes per slab.  Their voxels reach back by a plane, a row and a cell:
-    // one range of voxels, as long as what it reaches back by is at most half
-    // of it, or on larger planes (of more than 150,000 voxels) two, a row and a
-    // cell longer than the slab each.  A voxel of two slabs is summed for both
-    // (1500x1500x2 cells, 4 a cell: 6.5 ms, with particle-by-particle atomics
-    // 13.9).
-    const int row = g->sy + 1, back = g->sz + row;
-    const bool two = 2 * (int64_t)back > HY_VOXELS;
-    int64_t slab = two ? HY_VOXELS / 2 - row : HY_VOXELS - back;
-    if (slab > g->nv) slab = g->nv;
-    if ((rc = scratch_reserve(S.keys, sizeof(int) * (size_t)np)) ||
-        (rc = scratch_reserve(S.start, sizeof(int) * ((size_t)g->nv + 1))) ||
-        (rc = scratch_reserve(S.sums, sizeof(float) * HY_SUMS *
-                                          (size_t)(two ? 2 * (slab + row)
-                                                       : slab + back))))
-      return rc;
-    int *keys = (int *)S.keys.ptr, *start = (int *)S.start.ptr;
-    float *sums = (float *)S.sums.ptr;
-    int nb = blocks_for(np, 256);
-    if (nb > 8192) nb = 8192;
-    hipLaunchKernelGGL(k_hydro_keys, dim3(nb), dim3(256), 0, s, p, np, vmax,
-                       g->nv, keys, nbad);
-    VPIC_LAUNCHED("k_hydro_keys");
-    int *order, *sorted;
-    if ((rc = use.begin(s)) ||
-        (rc = device_sort_keys(keys, np, g, &order, &sorted, nullptr, use, s)))
-      return rc;
-    hipLaunchKernelGGL(k_hydro_starts, dim3(blocks_for((int64_t)g->nv + 1, 256)),
-                       dim3(256), 0, s, (const int *)sorted, np, g->nv, start);
-    VPIC_LAUNCHED("k_hydro_starts");
-    for (int64_t n0 = 0; n0 < g->nv; n0 += slab) {
-      const int64_t n1 = n0 + slab < g->nv ? n0 + slab : g->nv;
-      // voxels [v0, v1) to sums from voxel `at` on; none when there are none
-      auto cells = [&](int64_t v0, int64_t v1, int64_t at) {
-        if (v0 < 0) v0 = 0;
-        if (v1 > vmax) v1 = vmax;
-        if (v1 <= v0) return;
-        hipLaunchKernelGGL(k_hydro_cells,
-                           dim3(blocks_for((v1 - v0) * HY_LANES, 256)),
-                           dim3(256), 0, s, p, (const int *)order,
-                           (const int *)start, f, sums + (v0 - at) * HY_SUMS,
-                           C, (int)v0, (int)v1);
-      };
-      // the voxel at the start of sums for the plane below and the node's own
-      int64_t vl = n0 - back, vu = vl;
-      if (two) {
-        cells(n0 - back, n1 - g->sz, vl);
-        VPIC_LAUNCHED("k_hydro_cells");
-        vu = n0 - row - (slab + row);
-        cells(n0 - row, n1, vu);
-      } else {
-        cells(n0 - back, n1, vl);
-      }
-      VPIC_LAUNCHED("k_hydro_cells");
-      hipLaunchKernelGGL(k_hydro_nodes, dim3(blocks_for((n1 - n0) * 16, 256)),
-                         dim3(256), 0, s, (const float *)sums,
-                         (const int *)start, (float *)h, (int)vl, (int)vu,
-                         vmax, (int)n0, (int)n1, g->sy, g->sz);
-      VPIC_LAUNCHED("k_hydro_nodes");
-    }
   }
   int h_bad = 0;
   VPIC_HIP(hipMemcpyAsync(&h_bad, nbad, sizeof(int), hipMemcpyDeviceToHost, s));
