@@ -878,7 +878,8 @@ int vpic_hip_ensemble_tune(vpic_ensemble_t *e, int32_t trial_steps,
  * Outputs (device arrays in the run's precision, may be NULL except u_bar
  * when gradients are wanted): u_bar[np][3] = dW/d(ux,uy,uz), d_bar[np][3] =
  * dW/d(dx,dy,dz), f_bar[nv][6] = dW/d(ex,ey,ez,cbx,cby,cbz) of the initial
- * state.  *host_energy receives W.  All grid faces must be periodic.
+ * state.  *host_energy receives W.  All grid faces must be periodic
+ * and every particle in a cell (not a ghost voxel).
  * Synchronous; allocates its checkpoints (about (n_step/ckpt_interval +
  * ckpt_interval) particle and field arrays, and a permutation of the
  * particles per eight steps) and releases them before it returns. */

@@ -540,3 +540,27 @@ def test_hydro_without_scratch(dev, orc, limit):
     for k in T.HYDRO_FIELDS:
         assert np.max(np.abs(got[k] - want[k])) <= \
             1e-5 * max(np.max(np.abs(want[k])), 1e-30), k
+
+
+@pytest.mark.parametrize("n", [(9, 5, 5), (2100, 1, 1)],
+                         ids=lambda v: str(v).replace(" ", ""))
+@pytest.mark.parametrize("fp64", [False, True])
+def test_adjoint_refuses_particles_in_no_cell(dev, n, fp64):
+    """A particle in a ghost voxel belongs to no tile: refused, not left out
+    with a gradient of zero; the same where the voxel is off the grid."""
+    import torch
+    from vpic_amd import adjoint as A
+    g = _box(*n, cell=0.1)
+    P, F = _adjoint_inputs(g, 300, 8, fp64)
+    cells = P.view(-1).view(torch.int32)
+    at = (7 * 16 + 6) if fp64 else (7 * 8 + 3)  # particle 7's voxel
+    good = int(cells[at])
+    A.run(P, F, g, -1.0, 1.0, 3, 2)
+    for v in (g.voxel(0, 1, 1), g.voxel(1, 1, n[2] + 1), g.nv, -1):
+        cells[at] = v
+        say("adjoint, particle in voxel", v, n, fp64)
+        for grads in (True, False):
+            with pytest.raises(_lib.VpicError, match="1 particles"):
+                A.run(P, F, g, -1.0, 1.0, 3, 2, grads)
+    cells[at] = good
+    A.run(P, F, g, -1.0, 1.0, 3, 2)

@@ -297,6 +297,24 @@ __global__ void k_keys(const Part<R> *__restrict__ P, int np,
     keys[n] = P[n].i;
 }
 
+// Counts the particles in no cell of the box (outside the array, or in a ghost
+// voxel, whose interpolators nobody writes).
+template <class R>
+__global__ void k_check_cells(const Part<R> *__restrict__ P, int np, Box B,
+                              int *__restrict__ bad) {
+  for (int n = blockIdx.x * blockDim.x + threadIdx.x; n < np;
+       n += gridDim.x * blockDim.x) {
+    const int v = P[n].i;
+    bool ok = (unsigned)v < (unsigned)B.nv;
+    if (ok) {
+      int x, y, z;
+      coords(B, v, x, y, z);
+      ok = x >= 1 && x <= B.nx && y >= 1 && y <= B.ny && z >= 1 && z <= B.nz;
+    }
+    if (!ok) atomicAdd(bad, 1);
+  }
+}
+
 // part[v] = the first slot whose key is not below v: a search per voxel (a
 // thread per slot that fills the voxels up to its key takes 130 us on a 64^3
 // box, for the ghost plane below the first key).
@@ -1571,18 +1589,13 @@ struct Run {
 
   // Sort the particles of step n by cell (p and p2 swap roles), with the
   // permutation and the partition kept in perm and rows.
-  int sort(const vpic_grid_t *g, int *perm, int *rows, bool check) {
+  int sort(const vpic_grid_t *g, int *perm, int *rows) {
     ADJ_LAUNCH(k_keys<R>, dim3(nkeyblk()), (const Part<R> *)p, np, keys);
-    int rc, *order, *sorted, bad = 0;
+    int rc, *order, *sorted;
     SortScratchUse use;
     if ((rc = use.begin(s)) ||
-        (rc = device_sort_keys(keys, np, g, &order, &sorted,
-                               check ? &bad : nullptr, use, s)))
+        (rc = device_sort_keys(keys, np, g, &order, &sorted, use, s)))
       return rc;
-    if (bad)
-      return vpic_set_error(VPIC_EINVAL,
-                            "adjoint run: %d particles have a voxel index "
-                            "outside [0,nv)", bad);
     VPIC_HIP(hipMemcpyAsync(perm, order, sizeof(int) * (size_t)np,
                             hipMemcpyDeviceToDevice, s));
     ADJ_LAUNCH(k_partition, cover((int64_t)B.nv + 1), (const int *)sorted, np,
@@ -1637,6 +1650,22 @@ struct Run {
     double e = 0;
     for (double v : h) e += v;
     *out = e * escale;
+    return VPIC_OK;
+  }
+
+  // A particle in no cell belongs to no tile: refused before the first step.
+  int check_cells() {
+    if (np == 0) return VPIC_OK;
+    int h = 0;
+    ADJ_LAUNCH(k_check_cells<R>, dim3(nkeyblk()), (const Part<R> *)p, np, B,
+               err + 1);
+    VPIC_HIP(hipMemcpyAsync(&h, err + 1, sizeof(int), hipMemcpyDeviceToHost,
+                            s));
+    VPIC_HIP(hipStreamSynchronize(s));
+    if (h)
+      return vpic_set_error(VPIC_EINVAL,
+                            "adjoint run: %d particles are in no cell of the "
+                            "grid (a voxel outside it or a ghost voxel)", h);
     return VPIC_OK;
   }
 
@@ -1774,6 +1803,7 @@ int adjoint_run(const void *p0, int np, float q, float m, const void *f0,
                      (const R *)f0, rstride, nv);
   VPIC_LAUNCHED("k_fields_in");
   if ((rc = run.load())) return rc;
+  if (n_step > 0 && (rc = run.check_cells())) return rc;
   // the sort in force at step n (none: null)
   auto rows_at = [&](int n) -> const int * {
     return nsort ? rows[grads ? n / SORT_EVERY : 0] : nullptr;
@@ -1789,7 +1819,7 @@ int adjoint_run(const void *p0, int np, float q, float m, const void *f0,
     }
     if (sorts && n % SORT_EVERY == 0) {
       const int k = grads ? n / SORT_EVERY : 0;
-      if ((rc = run.sort(g, perm[k], rows[k], n == 0))) return rc;
+      if ((rc = run.sort(g, perm[k], rows[k]))) return rc;
     }
     if ((rc = run.step(run.p, run.p, rows_at(n)))) return rc;
   }

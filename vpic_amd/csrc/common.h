@@ -370,12 +370,11 @@ struct SortScratchUse {
 // The stable sort by voxel of the keys themselves (grids sort_keys_fit
 // accepts): *order[j] = the element at place j, *sorted[j] its key (in this
 // thread's sort scratch: valid while `use`, begun on this stream, lasts).  A
-// key outside [0, nv) sorts as 0; *bad (may be null) receives their number
-// after a synchronisation of the stream.
+// key outside [0, nv) sorts as 0.
 bool sort_keys_fit(const vpic_grid_t *g);
 int device_sort_keys(const int *keys, int np, const vpic_grid_t *g,
-                     int **order, int **sorted, int *bad,
-                     const SortScratchUse &use, hipStream_t s);
+                     int **order, int **sorted, const SortScratchUse &use,
+                     hipStream_t s);
 int launch_energy_p(const vpic_particle_t *p, int np, float q, float m,
                     const vpic_interpolator_t *f, const vpic_grid_t *g,
                     double *host_en, hipStream_t s);

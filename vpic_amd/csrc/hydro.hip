@@ -352,7 +352,7 @@ int hydro_sorted(HydroScratch &S, SortScratchUse &use, vpic_hydro_t *h,
   VPIC_LAUNCHED("k_hydro_keys");
   int *order, *sorted;
   if ((rc = use.begin(s)) ||
-      (rc = device_sort_keys(keys, np, g, &order, &sorted, nullptr, use, s)))
+      (rc = device_sort_keys(keys, np, g, &order, &sorted, use, s)))
     return rc;
   hipLaunchKernelGGL(k_hydro_starts, dim3(blocks_for((int64_t)g->nv + 1, 256)),
                      dim3(256), 0, s, (const int *)sorted, np, g->nv, start);

@@ -986,16 +986,10 @@ bool sort_keys_fit(const vpic_grid_t *g) {
 }
 
 int device_sort_keys(const int *keys, int np, const vpic_grid_t *g,
-                     int **order, int **sorted, int *bad,
-                     const SortScratchUse &, hipStream_t s) {
-  int rc, *nbad;
-  if ((rc = sort_pairs(nullptr, np, g, keys, order, sorted, &nbad, s)))
-    return rc;
-  if (bad) {
-    VPIC_HIP(hipMemcpyAsync(bad, nbad, sizeof(int), hipMemcpyDeviceToHost, s));
-    VPIC_HIP(hipStreamSynchronize(s));
-  }
-  return VPIC_OK;
+                     int **order, int **sorted, const SortScratchUse &,
+                     hipStream_t s) {
+  int *nbad;
+  return sort_pairs(nullptr, np, g, keys, order, sorted, &nbad, s);
 }
 
 long long sort_keys_stale_count() { return g_sort_keys_stale.load(); }
