@@ -277,3 +277,18 @@ def test_push_tiles_for_dense_regions():
     for n, ppc in (((12, 10, 9), 16), ((32, 32, 32), 128), ((64, 1, 64), 128),
                    ((97, 61, 83), 40), ((256, 128, 128), 200)):
         assert len(_push_tile(n, ppc * n[0] * n[1] * n[2])) == 1
+
+
+def test_adjoint_workspace_of_any_checkpoint_interval():
+    """An interval past the run's end, up to the largest int, is the run's
+    length: as much memory as one segment takes."""
+    g = T.grid_periodic(0, 0, 0, 4, 4, 4, 4, 4, 4, 0.5)
+    need = ctypes.c_int64()
+
+    def bytes_for(steps, ckpt):
+        _lib.call("vpic_hip_adjoint_workspace", 100, ctypes.byref(g), steps,
+                  ckpt, 4, 1, ctypes.byref(need))
+        return need.value
+    for ckpt in (11, 20, 2 ** 31 - 9, 2 ** 31 - 1, 0, -1):
+        assert bytes_for(10, ckpt) == bytes_for(10, 10)
+    assert bytes_for(10, 4) < bytes_for(10, 10)

@@ -1736,7 +1736,7 @@ int adjoint_run(const void *p0, int np, float q, float m, const void *f0,
   if (np < 0 || n_step < 0 ||
       (!want && ((np > 0 && !p0) || !f0 || !host_L)))
     return vpic_set_error(VPIC_EINVAL, "adjoint run: bad arguments");
-  if (ckpt < 1) ckpt = n_step > 0 ? n_step : 1;
+  if (ckpt < 1 || ckpt > n_step) ckpt = n_step > 0 ? n_step : 1;
   Run<R> run;
   run.setup(g, np, q, m, s);
   const int nv = g->nv;
@@ -1746,11 +1746,11 @@ int adjoint_run(const void *p0, int np, float q, float m, const void *f0,
   const size_t rbytes = sizeof(int) * ((size_t)nv + 1);
   const bool sorts = run.tiled() && np > 0;
   // checkpoints, and the states of one segment (all of it when shorter)
-  const int nseg = grads ? (n_step + ckpt - 1) / ckpt : 0;
-  const int nst = grads ? (ckpt < n_step ? ckpt : n_step) : 0;
+  const int nseg = grads ? n_step / ckpt + (n_step % ckpt ? 1 : 0) : 0;
+  const int nst = grads && n_step > 0 ? ckpt : 0;
   // sorts kept: all for the reverse, the last one otherwise
   const int nsort = !sorts || n_step < 1 ? 0
-                    : grads ? (n_step + SORT_EVERY - 1) / SORT_EVERY : 1;
+                    : grads ? 1 + (n_step - 1) / SORT_EVERY : 1;
   std::vector<Part<R> *> cp(nseg), sp(nst);
   std::vector<Fld<R> *> cF(nseg), sF(nst);
   std::vector<int *> perm(nsort), rows(nsort);
@@ -1835,7 +1835,7 @@ int adjoint_run(const void *p0, int np, float q, float m, const void *f0,
                      (const Fld<R> *)run.F, run.B, (R)run.escale);
   VPIC_LAUNCHED("k_benergy_grad");
   for (int k = nseg - 1; k >= 0; k--) {
-    const int n0 = k * ckpt, n1 = n0 + ckpt < n_step ? n0 + ckpt : n_step;
+    const int n0 = k * ckpt, n1 = n_step - n0 > ckpt ? n0 + ckpt : n_step;
     VPIC_HIP(hipMemcpyAsync(run.F, cF[k], fbytes, hipMemcpyDeviceToDevice, s));
     if ((rc = run.load())) return rc;
     // the segment's states: st[j] before step n0 + j, in the order of the
