@@ -5,6 +5,7 @@ import ctypes
 import os
 import re
 import subprocess
+import sys
 
 import pytest
 
@@ -292,3 +293,26 @@ def test_adjoint_workspace_of_any_checkpoint_interval():
     for ckpt in (11, 20, 2 ** 31 - 9, 2 ** 31 - 1, 0, -1):
         assert bytes_for(10, ckpt) == bytes_for(10, 10)
     assert bytes_for(10, 4) < bytes_for(10, 10)
+
+
+def test_adjoint_lists_beyond_the_hosts_memory():
+    """A run whose lists of checkpoints do not fit the host's memory is an
+    error, not an exception through the C entry (which ends the process)."""
+    code = """
+import ctypes, resource, sys
+sys.path.insert(0, %r)
+from vpic_amd import _lib, types as T
+g = T.grid_periodic(0, 0, 0, 4, 4, 4, 4, 4, 4, 0.5)
+n = ctypes.c_int64()
+_lib.load()
+size = int(open("/proc/self/statm").read().split()[0]) * 4096
+resource.setrlimit(resource.RLIMIT_AS, (size + (1 << 30),) * 2)
+try:
+    _lib.call("vpic_hip_adjoint_workspace", 100, ctypes.byref(g), 2 ** 31 - 1,
+              1, 4, 1, ctypes.byref(n))
+except _lib.VpicError as e:
+    print("refused:", e)
+""" % ROOT
+    out = subprocess.run([sys.executable, "-c", code], capture_output=True,
+                         text=True, timeout=120)
+    assert out.returncode == 0 and "refused" in out.stdout, out.stderr

@@ -49,6 +49,7 @@
 // passes it.
 #include "common.h"
 
+#include <exception>
 #include <utility>
 #include <vector>
 
@@ -1886,6 +1887,16 @@ int adjoint_run(const void *p0, int np, float q, float m, const void *f0,
   return VPIC_OK;
 }
 
+// (the lists of a run of very many steps may not fit the host's memory)
+template <class F>
+int no_throw(F run) {
+  try {
+    return run();
+  } catch (const std::exception &e) {
+    return vpic_set_error(VPIC_ENOMEM, "adjoint run: %s", e.what());
+  }
+}
+
 }  // namespace
 
 extern "C" int vpic_hip_adjoint_workspace(int32_t np, const vpic_grid_t *g,
@@ -1896,10 +1907,12 @@ extern "C" int vpic_hip_adjoint_workspace(int32_t np, const vpic_grid_t *g,
   if (!bytes)
     return vpic_set_error(VPIC_EINVAL, "adjoint workspace: bytes is NULL");
   auto ask = [&](auto zero) {
-    return adjoint_run<decltype(zero)>(nullptr, np, 1.0f, 1.0f, nullptr, g,
-                                       n_step, ckpt_interval, grads != 0,
-                                       nullptr, nullptr, nullptr, nullptr,
-                                       nullptr, 0, bytes, nullptr);
+    return no_throw([&] {
+      return adjoint_run<decltype(zero)>(nullptr, np, 1.0f, 1.0f, nullptr, g,
+                                         n_step, ckpt_interval, grads != 0,
+                                         nullptr, nullptr, nullptr, nullptr,
+                                         nullptr, 0, bytes, nullptr);
+    });
   };
   if (precision == 4) return ask(0.0f);
   if (precision == 8) return ask(0.0);
@@ -1915,13 +1928,17 @@ extern "C" int vpic_hip_adjoint_bfield_energy_ws(
   const hipStream_t s = (hipStream_t)stream;
   const bool grads = u_bar != nullptr;
   if (precision == 4)
-    return adjoint_run<float>(p0, np, q, m, f0, g, n_step, ckpt_interval,
-                              grads, host_energy, u_bar, d_bar, f_bar,
-                              workspace, workspace_bytes, nullptr, s);
+    return no_throw([&] {
+      return adjoint_run<float>(p0, np, q, m, f0, g, n_step, ckpt_interval,
+                                grads, host_energy, u_bar, d_bar, f_bar,
+                                workspace, workspace_bytes, nullptr, s);
+    });
   if (precision == 8)
-    return adjoint_run<double>(p0, np, q, m, f0, g, n_step, ckpt_interval,
-                               grads, host_energy, u_bar, d_bar, f_bar,
-                               workspace, workspace_bytes, nullptr, s);
+    return no_throw([&] {
+      return adjoint_run<double>(p0, np, q, m, f0, g, n_step, ckpt_interval,
+                                 grads, host_energy, u_bar, d_bar, f_bar,
+                                 workspace, workspace_bytes, nullptr, s);
+    });
   return vpic_set_error(VPIC_EINVAL, "adjoint run: precision %d (4 or 8)",
                         precision);
 }
