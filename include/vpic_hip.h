@@ -618,7 +618,8 @@ int vpic_hip_clear_hydro_array(vpic_hydro_t *h, const vpic_grid_t *g,
  * particles' indices are sorted by voxel (any order of the particles will do,
  * and `partition` is not needed), each voxel's moments are summed in registers
  * and the nodes gather them.  That takes scratch of 20 bytes a particle, 4 a
- * voxel, at most 128 MiB of sums and 16 MiB of counts, which the thread keeps.
+ * voxel, at most 128 MiB of sums and the sort's counts (16 MiB, or up to half a
+ * byte a particle where that is more), which the thread keeps.
  * Where it is not there, and on grids with an axis of more than 2046 cells, the
  * particles go one by one.  The per-particle arithmetic is the reference's;
  * the sums differ only in order.  Synchronous; particles whose voxel is not
@@ -882,7 +883,9 @@ int vpic_hip_ensemble_tune(vpic_ensemble_t *e, int32_t trial_steps,
  * and every particle in a cell (not a ghost voxel).
  * Synchronous; allocates its checkpoints (about (n_step/ckpt_interval +
  * ckpt_interval) particle and field arrays, and a permutation of the
- * particles per eight steps) and releases them before it returns. */
+ * particles per eight steps) and releases them before it returns; its sorts
+ * use the thread's scratch (16 bytes a particle and the counts), which
+ * stays. */
 int vpic_hip_adjoint_bfield_energy(const void *p0, int32_t np, float q,
                                    float m, const void *f0,
                                    const vpic_grid_t *g, int32_t n_step,
@@ -894,7 +897,8 @@ int vpic_hip_adjoint_bfield_energy(const void *p0, int32_t np, float q,
  * from call to call: `workspace` of at least the bytes that
  * vpic_hip_adjoint_workspace gives for the same np, grid, steps, checkpoint
  * interval, precision and grads (u_bar given or not).  The call owns it until
- * it returns.  NULL: allocated and released by the call. */
+ * it returns.  NULL: allocated and released by the call.  The sorts' scratch
+ * (above) lies outside it. */
 int vpic_hip_adjoint_workspace(int32_t np, const vpic_grid_t *g,
                                int32_t n_step, int32_t ckpt_interval,
                                int32_t precision, int32_t grads,

@@ -564,3 +564,30 @@ def test_adjoint_refuses_particles_in_no_cell(dev, n, fp64):
                 A.run(P, F, g, -1.0, 1.0, 3, 2, grads)
     cells[at] = good
     A.run(P, F, g, -1.0, 1.0, 3, 2)
+
+
+def test_adjoint_large_workspace_is_given_back(dev, monkeypatch):
+    """A call that needs more than its share of the GPU's memory leaves nothing
+    in torch's cache, where the library could not use it."""
+    import torch
+    from vpic_amd import adjoint as A
+    g = _box(33, 25, 25, cell=0.1)
+    P, F = _adjoint_inputs(g, 257, 5, True)
+    w, u = A.run(P, F, g, -1.0, 1.0, 9, 4)[:2]
+    need = ctypes.c_int64()
+    _lib.call("vpic_hip_adjoint_workspace", 257, ctypes.byref(g), 9, 4, 8, 1,
+              ctypes.byref(need))
+    total = torch.cuda.get_device_properties(0).total_memory
+    torch.cuda.empty_cache()
+    before = torch.cuda.memory_reserved()
+    say("adjoint, workspace beyond its share")
+    monkeypatch.setattr(A, "KEEP_SHARE", (need.value - 1) / total)
+    w2, u2 = A.run(P, F, g, -1.0, 1.0, 9, 4)[:2]
+    # (u2 itself is a small block of torch's, from its 2-MiB pools)
+    assert need.value > 20 << 20
+    assert torch.cuda.memory_reserved() - before <= 4 << 20
+    assert abs(w - w2) <= 1e-12 * abs(w)
+    assert float((u - u2).abs().max()) <= 1e-10 * float(u.abs().max())
+    monkeypatch.setattr(A, "KEEP_SHARE", need.value / total)
+    A.run(P, F, g, -1.0, 1.0, 9, 4)
+    assert torch.cuda.memory_reserved() - before >= need.value

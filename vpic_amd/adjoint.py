@@ -35,15 +35,25 @@ def set_momenta(part, u):
     return out
 
 
+# The largest share of the GPU's memory that a call's workspace leaves in torch's
+# cache.  The library's own allocations (the scratch of a push, a sort, an
+# ensemble) cannot use what lies there.
+KEEP_SHARE = 1 / 8
+
+
 def _workspace(np_, grid, n_step, ckpt, precision, grads, device):
     """Device memory for one call from torch's caching allocator (a call's own
     allocation of gigabytes costs up to three times its kernels): a tensor of
-    the default stream, which the library's work is ordered with, or None when
-    it does not fit (the library then allocates what it needs itself)."""
+    the default stream, which the library's work is ordered with.  None where
+    it does not fit or is more than KEEP_SHARE of the GPU's memory (the library
+    then allocates what it needs itself and releases it)."""
     need = ctypes.c_int64()
     _lib.call("vpic_hip_adjoint_workspace", np_, ctypes.byref(grid),
               int(n_step), int(ckpt), precision, int(grads),
               ctypes.byref(need))
+    total = torch.cuda.get_device_properties(device).total_memory
+    if need.value > KEEP_SHARE * total:
+        return None
     try:
         with torch.cuda.stream(torch.cuda.default_stream(device)):
             # (the allocator aligns its blocks to 512 bytes)
