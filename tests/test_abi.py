@@ -275,6 +275,14 @@ def test_push_tiles_for_dense_regions():
         assert cells[0] > 49 and cells == sorted(cells, reverse=True)
         assert cells[-1] <= 64 and len(t) >= 2
         assert _push_tile(n, ppc * n[0] * n[1] * n[2], True) == t
+    # 7x8x7 where few or no tiles are saved: cut tiles in a second round of
+    # CUs, whole tiles in one more round
+    for n, ppc in (((63, 25, 53), 64), ((256, 32, 32), 64),
+                   ((13, 183, 35), 224), ((29, 117, 153), 46)):
+        assert _push_tile(n, ppc * n[0] * n[1] * n[2]) == [(7, 8, 7, 1)]
+    n = (100, 3, 100)
+    t = _push_tile(n, 134 * n[0] * n[1] * n[2])[0]
+    assert -(-100 // t[0]) * -(-100 // t[2]) <= 256
     for n, ppc in (((12, 10, 9), 16), ((32, 32, 32), 128), ((64, 1, 64), 128),
                    ((97, 61, 83), 40), ((256, 128, 128), 200)):
         assert len(_push_tile(n, ppc * n[0] * n[1] * n[2])) == 1

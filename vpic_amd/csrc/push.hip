@@ -2509,8 +2509,15 @@ bool tile_fits(int tx, int ty, int tz, int h) {
 // the merge) and per particle 4.2 ns, more by 0.55 of the surface cells' share
 // (deposits outside the tile; measured 5.0 ns for 7x8x7, 5.6 for 8x8x4, 6.0
 // for 8x4x4, 6.6 for 32x2x2 at 32^3 cells, 128 per cell), one tile at a time
-// on each CU, whole tiles in whole rounds: `least`.  No push is faster than
+// on each CU, the fullest first: `least`.  Up to two rounds of tiles it is the
+// fullest one or pair (100x3x100 cells, 134 per cell, as 260 tiles of 8x3x5, of
+// which 20 are halves, takes 188 us, as 225 of 7x3x7 149), of more the whole
+// tiles in whole rounds (1024x512 cells, 32 per cell: 617 us in 1024 tiles of
+// 32x16, 723 in 1056 of 31x16 and 32 slivers) or, where some are cut, the mean
+// of the CUs and half a smallest tile.  No push is faster than
 // its fullest tile, at0 + per * p us with p particles in each of its cells.
+// Against 60 grids of 500 to 1e6 cells the ratio of two tiles' times is within
+// 12% (one standard deviation).
 struct TileCost {
   double least, at0, per;
   double at(double p) const {
@@ -2518,11 +2525,49 @@ struct TileCost {
   }
 };
 
+// Cells in the two tiles (the fullest first, the tiles after the 256th with the
+// least full before it) that one CU gets of between 256 and 512 tiles.
+double paired_cells(const int (&n)[3], const int (&t)[3]) {
+  // the tiles by size: whole or cut along each axis
+  double cells[8];
+  int count[8], kinds = 0, all = 0;
+  for (int k = 0; k < 8; k++) {
+    int many = 1;
+    double size = 1;
+    for (int a = 0; a < 3; a++) {
+      const int rest = n[a] % t[a];
+      many *= k >> a & 1 ? rest > 0 : n[a] / t[a];
+      size *= k >> a & 1 ? rest : t[a];
+    }
+    if (!many) continue;
+    int at = kinds++;
+    for (; at > 0 && cells[at - 1] < size; at--) {
+      cells[at] = cells[at - 1];
+      count[at] = count[at - 1];
+    }
+    cells[at] = size;
+    count[at] = many;
+    all += many;
+  }
+  auto tile = [&](int i) {
+    int k = 0;
+    while (i >= count[k]) i -= count[k++];
+    return cells[k];
+  };
+  double most = 0;
+  for (int j = 0; PUSH_CUS + j < all; j++) {
+    const double c = tile(PUSH_CUS - 1 - j) + tile(PUSH_CUS + j);
+    most = most > c ? most : c;
+  }
+  return most;
+}
+
 TileCost tile_cost(const vpic_grid_t *g, double ppc, int tx, int ty, int tz) {
   const int n[3] = {g->nx, g->ny, g->nz}, t[3] = {tx, ty, tz};
-  double full = 1, all = 1, cells = 1, wcells = 1, surface = 0;
+  double full = 1, all = 1, cells = 1, wcells = 1, surface = 0, smallest = 1;
   for (int k = 0; k < 3; k++) {
     full *= n[k] / t[k];
+    smallest *= n[k] % t[k] ? n[k] % t[k] : t[k];
     all *= (n[k] + t[k] - 1) / t[k];
     cells *= t[k];
     wcells *= t[k] + (n[k] > 1 ? 2 : 0);
@@ -2532,27 +2577,34 @@ TileCost tile_cost(const vpic_grid_t *g, double ppc, int tx, int ty, int tz) {
   TileCost c;
   c.at0 = 27 + 5e-3 * wcells;
   c.per = cells * per;
-  double rounds = full / PUSH_CUS;
-  rounds = rounds > (int)rounds ? (int)rounds + 1 : rounds;
-  if (rounds < 1) rounds = 1;
-  const double bound = rounds * (c.at0 + c.per * ppc);
-  const double mean =
+  const double one = c.at0 + c.per * ppc;
+  double mean =
       (all * c.at0 + (double)g->nx * g->ny * g->nz * ppc * per) / PUSH_CUS;
-  c.least = bound > mean ? bound : mean;
+  double rounds = 1;
+  if (all > 2 * PUSH_CUS) {
+    if (all > full) mean += 0.5 * (c.at0 + smallest * per * ppc);
+    rounds = ceil(full / PUSH_CUS);
+  }
+  c.least = rounds * one > mean ? rounds * one : mean;
+  if (all > PUSH_CUS && all <= 2 * PUSH_CUS) {
+    const double two = 2 * c.at0 + paired_cells(n, t) * per * ppc;
+    c.least = c.least > two ? c.least : two;
+  }
   return c;
 }
 
 // The tile of the least cost for a plasma whose densest cells hold `dense`
 // times the mean (0: uniform): 7x8x7 (the best of the shapes timed
-// on large grids) unless another is 5% cheaper.
+// on large grids) unless another is a tenth cheaper (of the grids above, those
+// where the other then took longer were estimated at 0.92 or more).
 TileGeom tile_search(const vpic_grid_t *g, double ppc, double dense) {
   TileGeom T = TILE_DEFAULT;
   const int mx = g->nx < 32 ? g->nx : 32, my = g->ny < 16 ? g->ny : 16,
             mz = g->nz < 16 ? g->nz : 16;
-  double best = 0.95 * tile_cost(g, ppc, T.tx < g->nx ? T.tx : g->nx,
-                                 T.ty < g->ny ? T.ty : g->ny,
-                                 T.tz < g->nz ? T.tz : g->nz)
-                           .at(dense * ppc);
+  double best = 0.9 * tile_cost(g, ppc, T.tx < g->nx ? T.tx : g->nx,
+                                T.ty < g->ny ? T.ty : g->ny,
+                                T.tz < g->nz ? T.tz : g->nz)
+                          .at(dense * ppc);
   // (at least two cells along an axis that has them)
   for (int tz = mz < 2 ? mz : 2; tz <= mz; tz++)
     for (int ty = my < 2 ? my : 2; ty <= my; ty++)
@@ -2597,11 +2649,11 @@ struct TileSet {
 // more CUs as well.  On 2D grids it is larger, since 7x1x7 is too small to
 // amortise a tile's fixed cost, and then a dense region would fall on few CUs.
 // There the push takes, by the particles it finds, that tile or the ones for
-// densities of 4 and 16 times the mean (512x257 cells, 2 x 48 per cell, 32x16,
-// 27x6 or 8x7 cells a tile; uniform: 319, 424, 569 us; 80% of the particles
-// in 0.3, 0.08, 0.02 of the cells: 530, 354, 468; 949, 593, 449; 957, 782, 516
-// us; 7x7: 595, 497, 474, 545; taken by the particles, with 8 us for looking at
-// them: 327, 365, 457, 562).
+// densities of 4 and 16 times the mean (512x257 cells, 2 x 48 per cell, in tiles
+// of 32x16, 27x6, 8x7, 7x7 cells; uniform: 319, 424, 569, 595 us; 80% of the
+// particles in 0.3 of the cells: 530, 354, 468, 497; in 0.08: 949, 593, 449,
+// 474; in 0.02: 957, 782, 516, 545; taken by the particles, with 8 us for
+// looking at them: 330, 364, 434, 806).
 // The search takes 20 to 55 us of host time, so the answers are for classes
 // of the particles per cell, an eighth of a factor of two wide, and the last
 // few are kept: a run whose particle numbers drift, or whose species go in
