@@ -301,12 +301,12 @@ def test_faces_in_one_launch(dev, orc, n, wall):
 # batches of voxels in the collision operator: 64 voxels at most (sparse, most
 # voxels with 0 or 1 particle), batches that end inside a neighbourhood, and
 # voxels that just fill a batch of 1792 particles or exceed it; partners many,
-# few and none
+# few and none; few particles in so many voxels that each has a lane
 @pytest.mark.parametrize("n,lo,hi,crowd", [
     ((70, 2, 2), 0, 2, ()), ((13, 5, 4), 20, 90, ()),
     ((4, 3, 3), 0, 9, (1791, 1792, 1793, 4100)), ((2, 1, 1), 1792, 1792, ()),
-    ((3, 2, 1), 700, 1500, ())],
-    ids=["sparse", "ordinary", "crowded", "full", "large"])
+    ((3, 2, 1), 700, 1500, ()), ((64, 64, 33), 0, 2, (3000, 1))],
+    ids=["sparse", "ordinary", "crowded", "full", "large", "many"])
 def test_collision_batches(dev, orc, n, lo, hi, crowd):
     """Bit for bit the oracle's voxel after voxel, within a species and
     between two in both orders of their sizes."""
@@ -334,7 +334,8 @@ def test_collision_batches(dev, orc, n, lo, hi, crowd):
         return p, part
 
     pe, parte = species(lo, hi, crowd, [1.0])
-    pi, parti = species(0, 7, crowd[:2], [1.0, 2.5])
+    pi, parti = species(0, 7 if len(inner) < 1 << 17 else 2, crowd[:2],
+                        [1.0, 2.5])
     de, dpe = dev.DeviceArray.from_host(pe), dev.DeviceArray.from_host(parte)
     di, dpi = dev.DeviceArray.from_host(pi), dev.DeviceArray.from_host(parti)
     E = (pe, parte, de, dpe, -1.0, 1.0)

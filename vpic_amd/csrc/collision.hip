@@ -270,19 +270,33 @@ __device__ __forceinline__ float4 *ta_mom(vpic_particle_t *p, int k) {
 // Particles of a batch, both species': with 28 KiB of momenta four workgroups
 // share a CU's LDS.  Voxels in a batch: one lane each shuffles them.
 constexpr int TA_BS = 256, TA_CAP = 1792, TA_VOX = 64;
+// Where many voxels hold few particles a batch is 64 of them with a handful of
+// chains, and a lane per voxel is faster: below TA_SPARSE particles of one
+// species, TA_SPARSE2 of two together, in at least TA_SPARSE_CELLS cells (128^3
+// cells, 1, 2, 4, 6 of each species: 441, 477, 552, 648 us a call within one in
+// batches, 195, 252, 422, 857 with a lane per voxel, between two 555, 757, 1032,
+// 1298 and 327, 607, 1169, 1789; 64^3: 87, 93, 103, 112 and 69, 81, 103, 130,
+// between two 104, 134, 172, 207 and 104, 153, 242, 320; 24^3: batches always).
+constexpr double TA_SPARSE = 4, TA_SPARSE2 = 3;
+constexpr int64_t TA_SPARSE_CELLS = 1 << 17;
 
 // One lane, one voxel, in memory: the voxels of more particles than a batch
-// holds.
-__global__ __launch_bounds__(256) void k_ta_crowded(TaArgs a, int *nbad) {
+// holds, or (ALL) every voxel of a sparse plasma.
+template <bool ALL>
+__global__ __launch_bounds__(256) void k_ta_lane(TaArgs a, int *nbad) {
   const int v = blockIdx.x * 256 + threadIdx.x;
   if (v >= a.v1) return;
   TaVoxel V;
   V.k0 = a.part_i[v];
   V.nk = a.part_i[v + 1] - V.k0;
-  if (V.k0 < 0 || V.nk <= 0 || V.k0 + V.nk > a.np_i) return;
+  if (!V.nk) return;
+  if (V.k0 < 0 || V.nk < 0 || V.k0 + V.nk > a.np_i) {
+    if (ALL) atomicAdd(nbad, 1);
+    return;
+  }
   V.l0 = V.nl = 0;
   const bool other = a.same || ta_other(a, v, V.l0, V.nl);
-  if ((int64_t)V.nk + V.nl <= TA_CAP) return;
+  if (!ALL && (int64_t)V.nk + V.nl <= TA_CAP) return;
   if (!other) atomicAdd(nbad, 1);
   TaRng rng;
   ta_stream(a, v, rng);
@@ -299,13 +313,12 @@ __global__ __launch_bounds__(256) void k_ta_crowded(TaArgs a, int *nbad) {
     density += a.pi[i].w;
   }
   density += a.pi[i].w;
-  V.n = rng.n;
   if (!ta_pairing(a, v, density, V, [&](int k) { return a.pj[k].w; })) return;
   uint32_t w[4];
   auto meet = [&](int k, int l, float std) {
     float4 x = *ta_mom(a.pi, k), y = *ta_mom(a.pj, l);
-    ta_words(rng, V.n, w);
-    V.n += 4;
+#pragma unroll
+    for (int c = 0; c < 4; c++) w[c] = rng.u32();
     ta_collide(x, y, a.mu_i, a.mu_j, std, w);
     *ta_mom(a.pi, k) = x;
     *ta_mom(a.pj, l) = y;
@@ -379,7 +392,7 @@ __global__ __launch_bounds__(TA_BS, 4) void k_takizuka_abe(TaArgs a, int nvox,
     __syncthreads();
     const int m = s_m;
     if (m == 0) {
-      if (t == 0) atomicAdd(nbad + 1, 1);  // left for k_ta_crowded
+      if (t == 0) atomicAdd(nbad + 1, 1);  // left for k_ta_lane
       v++;
       __syncthreads();
       continue;
@@ -606,21 +619,29 @@ int launch_takizuka_abe(vpic_particle_t *pi, const int *part_i, int np_i,
   // voxels of a workgroup: three quarters of a batch at the mean number of
   // particles, since a batch that does not hold them all leaves a short second
   // one (64-particle voxels with their spread of 8: 21 of at most 28)
-  const double mean = ((double)np_i + (a.same ? 0.0 : (double)np_j)) /
-                      ((double)g->nx * g->ny * g->nz);
+  const int64_t cells = (int64_t)g->nx * g->ny * g->nz;
+  const double mean =
+      ((double)np_i + (a.same ? 0.0 : (double)np_j)) / (double)cells;
   int nvox = mean > 0 ? (int)(0.75 * TA_CAP / mean) : TA_VOX;
   nvox = nvox < 1 ? 1 : nvox > TA_VOX ? TA_VOX : nvox;
-  hipLaunchKernelGGL(k_takizuka_abe, dim3((a.v1 + nvox - 1) / nvox),
-                     dim3(TA_BS), 0, s, a, nvox, nbad);
-  VPIC_LAUNCHED("k_takizuka_abe");
+  if (cells >= TA_SPARSE_CELLS &&
+      mean < (a.same ? TA_SPARSE : TA_SPARSE2)) {
+    hipLaunchKernelGGL(k_ta_lane<true>, dim3((a.v1 + 255) / 256), dim3(256), 0,
+                       s, a, nbad);
+    VPIC_LAUNCHED("k_ta_lane");
+  } else {
+    hipLaunchKernelGGL(k_takizuka_abe, dim3((a.v1 + nvox - 1) / nvox),
+                       dim3(TA_BS), 0, s, a, nvox, nbad);
+    VPIC_LAUNCHED("k_takizuka_abe");
+  }
   int h[2] = {0, 0};
   VPIC_HIP(
       hipMemcpyAsync(h, nbad, sizeof(h), hipMemcpyDeviceToHost, s));
   VPIC_HIP(hipStreamSynchronize(s));
   if (h[1]) {
-    hipLaunchKernelGGL(k_ta_crowded, dim3((a.v1 + 255) / 256), dim3(256), 0,
-                       s, a, nbad);
-    VPIC_LAUNCHED("k_ta_crowded");
+    hipLaunchKernelGGL(k_ta_lane<false>, dim3((a.v1 + 255) / 256), dim3(256),
+                       0, s, a, nbad);
+    VPIC_LAUNCHED("k_ta_lane");
     VPIC_HIP(
         hipMemcpyAsync(h, nbad, sizeof(int), hipMemcpyDeviceToHost, s));
     VPIC_HIP(hipStreamSynchronize(s));
