@@ -94,13 +94,16 @@ def _adjoint_inputs(g, np_, seed, fp64):
 
 # tiles of 8x4x4 cells: one tile with a window that wraps onto itself, two
 # tiles an axis, a last tile of one cell, axes of one cell, an axis too long
-# to sort (chunks of particles, no windows); particle counts around a
+# to sort or few particles (chunks of particles, no windows), the chunks at their
+# shortest and longer; particle counts around a
 # wavefront and a workgroup; steps past a sort, checkpoints that do and
 # do not fall on one
 @pytest.mark.parametrize("n,np_,steps,ckpt", [
     ((3, 2, 4), 1, 3, 2), ((8, 4, 4), 65, 10, 4), ((9, 5, 5), 257, 17, 3),
     ((17, 8, 9), 3000, 9, 20), ((16, 1, 13), 1500, 12, 5),
-    ((1, 9, 1), 300, 9, 8), ((2100, 1, 1), 9000, 10, 4)],
+    ((1, 9, 1), 300, 9, 8), ((2100, 1, 1), 9000, 10, 4),
+    ((2100, 1, 1), 530000, 3, 2), ((20, 15, 14), 1399, 9, 4),
+    ((20, 15, 14), 1400, 9, 4)],
     ids=lambda v: str(v).replace(" ", ""))
 def test_adjoint_tiles(dev, n, np_, steps, ckpt):
     """The gradients do not depend on how particles share tiles: the same

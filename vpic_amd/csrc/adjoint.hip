@@ -115,16 +115,24 @@ constexpr int AT_X = 8, AT_Y = 4, AT_Z = 4;
 constexpr int AT_BS = 256, AT_WAVES = AT_BS / 64;
 constexpr int AT_CELLS = (AT_X + 2) * (AT_Y + 2) * (AT_Z + 2);
 constexpr int AT_ROWS = AT_Y * AT_Z;
-// Particles per workgroup where there is no partition (unsorted runs).
-constexpr int AT_CHUNK = 4096;
+// Most particles per workgroup without tiles; fewer, whole rounds of its lanes,
+// as long as that leaves AT_CHUNKS workgroups or fewer (2100x1x1 cells, 60000
+// particles, 16 steps with gradient: 8.3 ms with 4096 in each, 4.3 with 256).
+constexpr int AT_CHUNK = 4096, AT_CHUNKS = 2048;
+// No tiles for fewer particles than a third of the cells: the windows, their
+// merge and the sorts cost by the cell (64^3 cells, 16 steps with gradient, 0.05,
+// 0.2, 0.5 particles per cell: 7.8, 8.1, 8.3 ms with tiles, 5.6, 6.9, 9.6
+// without; 128x128x64: 27.3, 28.8, 29.4 and 19.1, 24.7, 35.3).
+constexpr int AT_SPARSE = 3;
 // A thermal particle drifts by one cell in about ten steps; sorting more
 // often costs more than the deposits that leave the windows until then.
 constexpr int SORT_EVERY = 8;
 
-// Tiles per axis; 0: no tiles (an axis too long for the sort's digits), the
-// workgroups take AT_CHUNK particles each and have no window.
+// Tiles per axis; 0: no tiles (an axis too long for the sort's digits, or few
+// particles), the workgroups take `chunk` particles each and have no window.
 struct Tiles {
   int nt[3];
+  int chunk;
 };
 
 struct TileAxis {
@@ -176,14 +184,15 @@ struct TileWin {
 struct TileRows {
   int start[AT_ROWS], pref[AT_ROWS + 1], nrow;
   __device__ __forceinline__ void load(const TileWin &W, const Box &B,
-                                       const int *part, int np, int tile) {
+                                       const Tiles &T, const int *part, int np,
+                                       int tile) {
     const int t = threadIdx.x;
     if (!W.on) {
       if (t == 0) {
         nrow = 1;
-        start[0] = tile * AT_CHUNK;
+        start[0] = tile * T.chunk;
         pref[0] = 0;
-        pref[1] = min(AT_CHUNK, np - tile * AT_CHUNK);
+        pref[1] = min(T.chunk, np - tile * T.chunk);
       }
     } else {
       if (t < W.y.n * W.z.n) {
@@ -471,7 +480,7 @@ __global__ void __launch_bounds__(AT_BS)
   W.at(T, B, tile);
   const int ncell = W.cells();
   for (int k = threadIdx.x; k < 12 * ncell; k += AT_BS) win[k] = 0;
-  rows.load(W, B, part, np, tile);
+  rows.load(W, B, T, part, np, tile);
   const int total = rows.pref[rows.nrow];
   FwdCross<R> *q = queue[wv];
   int qn = 0;
@@ -890,7 +899,7 @@ __global__ void __launch_bounds__(AT_BS)
   W.at(T, B, tile);
   const int ncell = W.cells();
   for (int k = threadIdx.x; k < NI * ncell; k += AT_BS) win[k] = 0;
-  rows.load(W, B, part, np, tile);
+  rows.load(W, B, T, part, np, tile);
   const int total = rows.pref[rows.nrow];
   int *q = queue[wv];
   int qn = 0;
@@ -1545,12 +1554,17 @@ struct Run {
     np = np_;
     s = st;
     // tiles where the particles can be sorted by cell
-    const bool tiled = sort_keys_fit(g);
+    const bool tiled = sort_keys_fit(g) &&
+                       (int64_t)np * AT_SPARSE >=
+                           (int64_t)B.nx * B.ny * B.nz;
     T.nt[0] = tiled ? (B.nx + AT_X - 1) / AT_X : 0;
     T.nt[1] = tiled ? (B.ny + AT_Y - 1) / AT_Y : 0;
     T.nt[2] = tiled ? (B.nz + AT_Z - 1) / AT_Z : 0;
+    const int share = (int)(((int64_t)np / AT_CHUNKS + AT_BS - 1) / AT_BS) *
+                      AT_BS;
+    T.chunk = share < AT_BS ? AT_BS : share > AT_CHUNK ? AT_CHUNK : share;
     nblk = tiled ? T.nt[0] * T.nt[1] * T.nt[2]
-                 : (int)(((int64_t)np + AT_CHUNK - 1) / AT_CHUNK);
+                 : (int)(((int64_t)np + T.chunk - 1) / T.chunk);
     // advance_p_pipeline.cc:279-283 (in float for the FP32 run)
     const R rq = q, rm = m, dt = g->dt, c = g->cvac;
     C.qdt_2mc = (rq * dt) / (2 * rm * c);
