@@ -224,11 +224,13 @@ def test_accumulate_rho_chunks(dev, n, np_, order):
 
 # one particle; 16 lanes of one voxel and one more; few particles over a grid
 # of two slabs of voxels; planes just below and above half a slab, and far above;
-# axes of one cell; an axis too long to sort by
+# axes of one cell; an axis too long to sort by; just below and above a particle
+# in twelve cells
 @pytest.mark.parametrize("n,np_", [
     ((4, 3, 5), 1), ((2, 1, 2), 16 * 4 + 1), ((9, 8, 7), 12000),
     ((70, 70, 63), 30000), ((385, 384, 3), 60000), ((386, 384, 3), 60000),
-    ((900, 700, 1), 50000), ((33, 1, 20), 5000), ((2100, 1, 1), 4000)],
+    ((900, 700, 1), 60000), ((33, 1, 20), 5000), ((2100, 1, 1), 4000),
+    ((20, 20, 20), 666), ((20, 20, 20), 667)],
     ids=lambda v: str(v).replace(" ", ""))
 def test_hydro_voxel_sums(dev, orc, n, np_):
     """The moments of particles in no order against the oracle's, within the

@@ -17,8 +17,9 @@
 // eight it takes.  No atomics.  1.5e7 particles on 72x64x50 cells that drifted
 // by half a cell since the sort: 0.77 ms, of which the sort is 0.33 (6.5
 // ms with LDS windows per tile, whose float atomics a drifted particle needs
-// one by one).  Grids with an axis too long for that sort, and calls for which
-// its memory is not there, go particle by particle with global atomics.
+// one by one).  Grids with an axis too long for that sort, sparse species and calls
+// for which its memory is not there go particle by particle with global
+// atomics.
 #include "common.h"
 
 namespace {
@@ -29,6 +30,11 @@ struct HydroCoef {
 
 constexpr int HY_LANES = 16;  // lanes per voxel (one DPP row)
 constexpr int HY_SUMS = 8 * 14;
+// Fewer particles than one in HY_SPARSE cells go one by one: the starts, sums and
+// nodes cost by the voxel, 0.4 to 0.6 ns, the atomics 6 ns a particle (256^3
+// cells, 0.05, 0.1, 0.2 particles per cell: 8.2, 9.4, 10.5 ms sorted, 4.8, 9.6,
+// 19.3 one by one; 64^3: 196, 217, 233 us and 119, 190, 337).
+constexpr int HY_SPARSE = 12;
 // Voxels whose sums (448 B each, 128 MiB in all) stay in the 256-MB cache
 // between the kernel that writes them and the one that reads them.
 constexpr int64_t HY_VOXELS = ((int64_t)128 << 20) / (4 * HY_SUMS);
@@ -427,7 +433,8 @@ int launch_accumulate_hydro_p(vpic_hydro_t *h, const vpic_particle_t *p,
   // voxels whose eight nodes lie on the grid
   const int vmax = g->nv - g->sz - g->sy - 1;
   rc = VPIC_ENOMEM;
-  if (np > 0 && sort_keys_fit(g)) {
+  const int64_t cells = (int64_t)g->nx * g->ny * g->nz;
+  if (np > 0 && sort_keys_fit(g) && (int64_t)np * HY_SPARSE >= cells) {
     rc = hydro_sorted(S, use, h, p, np, f, g, C, vmax, nbad, s);
     if (rc && rc != VPIC_ENOMEM) return rc;
     if (rc) {
