@@ -171,7 +171,7 @@ const char *vpic_hip_version(void);
  * vpic_hip_scratch_limit: the most bytes a scratch array of this thread may
  * take (0, as at the start: no limit).  A call that needs more, or for which
  * the GPU has no more, does without where it can (accumulate_hydro_p) and
- * fails with VPIC_ENOMEM otherwise. */
+ * fails otherwise. */
 int vpic_hip_scratch_limit(int64_t bytes);
 
 /* ------------------------------------------------------------------------ */

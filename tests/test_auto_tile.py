@@ -61,11 +61,13 @@ def _particles(g, np_, seed, dense):
 
 
 # a single cell; fewer tiles than CUs; more, with a dense slab; a thin
-# grid; particle walls; particles appended after the sort
+# grid; particle walls; particles appended after the sort, also more than it
+# sorted
 @pytest.mark.parametrize("n,np_,dense,walls,extra", [
     ((1, 1, 1), 40, False, False, 0), ((12, 10, 9), 3000, False, False, 70),
     ((64, 48, 40), 60000, True, False, 0), ((200, 1, 90), 30000, True, True, 5),
-    ((3, 90, 80), 20000, True, False, 1)],
+    ((3, 90, 80), 20000, True, False, 1),
+    ((20, 18, 16), 4000, False, False, 9001)],
     ids=lambda v: str(v).replace(" ", ""))
 def test_push_auto_tile(dev, orc, n, np_, dense, walls, extra):
     """Two species in one call against the oracle: particles bit for bit, the

@@ -36,7 +36,8 @@
 // steps: a workgroup takes the particles of a tile of cells, sums the lanes of
 // one cell in registers (a segmented wavefront scan) and adds the sums to a
 // window of the tile and its neighbouring cells in LDS; k_merge adds the
-// windows.  Deposits outside the window are global atomics.
+// windows.  Deposits outside the window are global atomics, and so are all of
+// them where there are no tiles (few particles, axes too long to sort by).
 //
 // Checkpointing: the forward stores the state (particles and fields) every
 // `ckpt` steps; the reverse takes the segments last first, recomputes the
@@ -267,7 +268,7 @@ struct Cover {
 };
 
 // out[v] += the windows' sums at v (out holds the deposits outside the
-// windows); one thread per voxel and N / 6 of its components.
+// windows); one thread per voxel.
 template <class R, int N>
 __global__ void __launch_bounds__(256)
     k_merge(R *__restrict__ out, const R *__restrict__ wbuf, Box B, Tiles T) {

@@ -520,7 +520,8 @@ int SortScratchUse::begin(hipStream_t stream) {
   if (st != hipStreamCaptureStatusNone) return VPIC_OK;
   SortScratch &S = sort_scratch();
   if (!S.used)
-    VPIC_HIP(hipEventCreateWithFlags(&S.used, hipEventDisableTiming));
+    VPIC_HIP(hipEventCreateWithFlags(&S.used, hipEventDisableTiming |
+                                                  hipEventDisableSystemFence));
   if (S.queued) VPIC_HIP(hipStreamWaitEvent(s, S.used, 0));
   open = true;
   return VPIC_OK;

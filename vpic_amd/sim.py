@@ -448,6 +448,8 @@ class Simulation:
 
     # -- one time step (advance.cc:15-207) ----------------------------------
     def advance(self, timer=None):
+        """One step; `timer(name)` brackets its phases: "sort", "push" and
+        "field" (which forms the interpolators as well)."""
         t = timer or (lambda name: _NullCtx())
         with t("sort"):
             for sp in self.species:
