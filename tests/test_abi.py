@@ -280,6 +280,8 @@ def test_push_tiles_for_dense_regions():
     for n, ppc in (((63, 25, 53), 64), ((256, 32, 32), 64),
                    ((13, 183, 35), 224), ((29, 117, 153), 46)):
         assert _push_tile(n, ppc * n[0] * n[1] * n[2]) == [(7, 8, 7, 1)]
+    # a cut tile that would wait for a whole one on its die
+    assert _push_tile((178, 20, 20), 184 * 178 * 400) != [(7, 10, 4, 1)]
     n = (100, 3, 100)
     t = _push_tile(n, 134 * n[0] * n[1] * n[2])[0]
     assert -(-100 // t[0]) * -(-100 // t[2]) <= 256

@@ -2519,8 +2519,8 @@ bool tile_fits(int tx, int ty, int tz, int h) {
 // 32x16, 723 in 1056 of 31x16 and 32 slivers) or, where some are cut, the mean
 // of the CUs and half a smallest tile.  No push is faster than
 // its fullest tile, at0 + per * p us with p particles in each of its cells.
-// Against 60 grids of 500 to 1e6 cells the ratio of two tiles' times is within
-// 12% (one standard deviation).
+// Over grids of 500 to 1e6 cells the ratio of two tiles' times is estimated
+// within 12% (one standard deviation).
 struct TileCost {
   double least, at0, per;
   double at(double p) const {
@@ -2528,8 +2528,10 @@ struct TileCost {
   }
 };
 
-// Cells in the two tiles (the fullest first, the tiles after the 256th with the
-// least full before it) that one CU gets of between 256 and 512 tiles.
+// Cells in the two tiles that one CU gets of between 256 and 512 tiles, dealt
+// to the eight dies in turn, the fullest first (178x20x20 cells in 260 tiles of
+// 7x10x4, ten of them cut: on two dies a cut one waits for a whole one, 468 us
+// against 414 in 7x8x7).
 double paired_cells(const int (&n)[3], const int (&t)[3]) {
   // the tiles by size: whole or cut along each axis
   double cells[8];
@@ -2558,8 +2560,9 @@ double paired_cells(const int (&n)[3], const int (&t)[3]) {
     return cells[k];
   };
   double most = 0;
-  for (int j = 0; PUSH_CUS + j < all; j++) {
-    const double c = tile(PUSH_CUS - 1 - j) + tile(PUSH_CUS + j);
+  // (tile i goes to die i % 8, whose 32 CUs take its tiles in turn)
+  for (int i = PUSH_CUS; i < all; i++) {
+    const double c = tile(i % 8 + 8 * (63 - i / 8)) + tile(i);
     most = most > c ? most : c;
   }
   return most;
@@ -2598,8 +2601,9 @@ TileCost tile_cost(const vpic_grid_t *g, double ppc, int tx, int ty, int tz) {
 
 // The tile of the least cost for a plasma whose densest cells hold `dense`
 // times the mean (0: uniform): 7x8x7 (the best of the shapes timed
-// on large grids) unless another is a tenth cheaper (of the grids above, those
-// where the other then took longer were estimated at 0.92 or more).
+// on large grids) unless another is a tenth cheaper (on 150 grids of 500 to 1e6
+// cells the tile taken needs 0.70 of 7x8x7's time, 0.16 to 1.04; unless it is
+// 5% cheaper, 0.70, up to 1.16).
 TileGeom tile_search(const vpic_grid_t *g, double ppc, double dense) {
   TileGeom T = TILE_DEFAULT;
   const int mx = g->nx < 32 ? g->nx : 32, my = g->ny < 16 ? g->ny : 16,
