@@ -2602,7 +2602,7 @@ TileCost tile_cost(const vpic_grid_t *g, double ppc, int tx, int ty, int tz) {
 // The tile of the least cost for a plasma whose densest cells hold `dense`
 // times the mean (0: uniform): 7x8x7 (the best of the shapes timed
 // on large grids) unless another is a tenth cheaper (on 150 grids of 500 to 1e6
-// cells the tile taken needs 0.70 of 7x8x7's time, 0.16 to 1.04; unless it is
+// cells the tile taken needs 0.70 of 7x8x7's time, 0.17 to 1.04; unless it is
 // 5% cheaper, 0.70, up to 1.16).
 TileGeom tile_search(const vpic_grid_t *g, double ppc, double dense) {
   TileGeom T = TILE_DEFAULT;
